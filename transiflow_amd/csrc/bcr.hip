@@ -16,7 +16,7 @@
 //   r_k <- r_k - P1 r_e1 - P2 r_e2
 //
 // Every level is a batch of independent dense operations: the inversions of
-// its eliminated lines (blocked Gauss-Jordan, 64-wide panels) and six GEMMs
+// its eliminated lines (blocked Gauss-Jordan, 128-wide panels) and six GEMMs
 // per kept line -- so the sequential depth is (levels x panels), about 100 for
 // 256 lines, instead of (lines x panels) for the Thomas recursion.  At level
 // 0 the couplings are the sparse CSR entries (a few per row), so the level-0
@@ -44,11 +44,6 @@
 
 namespace {
 
-using tf::gj::PB;
-using tf::gj::k_panel;
-using tf::gj::k_panel_copy;
-using tf::gj::k_panel_store;
-using tf::gj::readlane_t;
 constexpr int KC = 8;   // couplings per row/column to a neighbouring line
 
 struct Cpl {
@@ -1120,10 +1115,7 @@ struct tf_bcr {
   void* Um;   // N m^2
   void* P1;   // slots m^2 (one per kept line per level)
   void* P2;   // slots m^2
-  void* Pinv; // batch x 64 x 64
-  void* Kr;   // batch x 64 x m
-  void* Kc;   // batch x m x 64
-  void* Tb;   // batch x 64 x m
+  void *Pinv, *Kc, *Tb;  // scratch of the inversions (gj.h), largest level
   Cpl *Lr, *Ur, *Ut, *Lt;
   int *nLr, *nUr, *nUt, *nLt;
   int* flags;  // [err, nperturb]
@@ -1193,38 +1185,6 @@ void level_gemm(tf_bcr* h, int M, int N, int K, void** A, int lda, void** B, int
   gemm<T>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
 }
 
-template <typename T>
-void invert_batch(tf_bcr* h, void** Xp, int batch, hipStream_t st) {
-  const int m = h->m;
-  T* Pinv = (T*)h->Pinv;
-  T* Kr = (T*)h->Kr;
-  T* Kc = (T*)h->Kc;
-  T* Tb = (T*)h->Tb;
-  // per-batch pointers to the snapshot buffers are laid out contiguously: the
-  // GEMMs need pointer lists, which live right after Xp in the pool
-  void** pinvp = Xp + batch;
-  void** krp = pinvp + batch;
-  void** kcp = krp + batch;
-  void** tbp = kcp + batch;
-  const long sz = (long)PB * m;
-  const int gcopy = (int)((sz + 255) / 256) < 1024 ? (int)((sz + 255) / 256) : 1024;
-  for (int k0 = 0; k0 < m; k0 += PB) {
-    const int pb = m - k0 < PB ? m - k0 : PB;
-    TF_PROF_WORK(tf::PROF_GJ_PANEL, 2.0 * 64 * 64 * 128 * batch);
-    TF_PROF_BEGIN(tf::PROF_GJ_PANEL, st);
-    hipLaunchKernelGGL(k_panel<T>, dim3(batch), dim3(512), 0, st, m, k0, pb, (T* const*)Xp, Pinv, h->flags + 1);
-    TF_PROF_END(tf::PROF_GJ_PANEL, st);
-    hipLaunchKernelGGL(k_panel_copy<T>, dim3(gcopy, batch), dim3(256), 0, st, m, k0, pb, (T* const*)Xp, Kr, Kc);
-    // T = Pinv * Kr   (pb x pb) x (pb x m)
-    gemm<T>(pb, m, pb, pinvp, pb, krp, m, tbp, m, 1.0, 0.0, batch, st);
-    // X -= Kc * T     (m x pb) x (pb x m)
-    gemm<T>(m, m, pb, kcp, pb, tbp, m, Xp, m, -1.0, 1.0, batch, st);
-    hipLaunchKernelGGL(k_panel_store<T>, dim3(gcopy, batch), dim3(256), 0, st, m, k0, pb, (T* const*)Xp,
-                       (const T*)Tb);
-  }
-  (void)Pinv; (void)Kr; (void)Kc; (void)Tb;
-}
-
 // the captured applies (every vector type and column count) are made again on next use
 void drop_graphs(tf_bcr* h) {
   for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
@@ -1246,10 +1206,11 @@ int factor_impl(tf_bcr* h, const int* rp, const int* ci, const double* v, int ga
   hipLaunchKernelGGL(k_sort_cols, dim3((n + 255) / 256), dim3(256), 0, st, n, h->Ut, h->nUt);
   hipLaunchKernelGGL(k_sort_cols, dim3((n + 255) / 256), dim3(256), 0, st, n, h->Lt, h->nLt);
   hipLaunchKernelGGL(k_diag_blocks<T>, dim3(m, N), dim3(256), 0, st, m, h->order, rp, ci, v, gauge, (T*)h->D);
+  const tf::gj::Scratch<T> w{(T*)h->Pinv, (T*)h->Kc, (T*)h->Tb};
   for (size_t l = 0; l < h->lev.size(); ++l) {
     BcrLevelDev& L = h->lev[l];
     // 1. invert the eliminated lines' diagonal blocks in place
-    invert_batch<T>(h, L.Ye, L.ne, st);
+    if (int e = tf::gj::invert<T>(m, (T* const*)L.Ye, L.ne, w, h->flags + 1, 0.0, st)) return e;
     if (L.nk == 0) continue;
     if (l == 0) {
       // sparse couplings at level 0 (e1 = k-1, e2 = k+1):
@@ -1754,10 +1715,9 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   h->slots = slots;
   TF_HIP(hipMalloc(&h->P1, h->es * mm * slots));
   TF_HIP(hipMalloc(&h->P2, h->es * mm * slots));
-  TF_HIP(hipMalloc(&h->Pinv, h->es * PB * PB * maxb));
-  TF_HIP(hipMalloc(&h->Kr, h->es * PB * (size_t)m * maxb));
-  TF_HIP(hipMalloc(&h->Kc, h->es * PB * (size_t)m * maxb));
-  TF_HIP(hipMalloc(&h->Tb, h->es * PB * (size_t)m * maxb));
+  TF_HIP(hipMalloc(&h->Pinv, h->es * tf::gj::scratch_P() * maxb));
+  TF_HIP(hipMalloc(&h->Kc, h->es * tf::gj::scratch_K(m) * maxb));
+  TF_HIP(hipMalloc(&h->Tb, h->es * tf::gj::scratch_K(m) * maxb));
   for (Cpl** c : {&h->Lr, &h->Ur, &h->Ut, &h->Lt}) TF_HIP(hipMalloc(c, sizeof(Cpl) * KC * (size_t)n));
   for (int** c : {&h->nLr, &h->nUr, &h->nUt, &h->nLt}) TF_HIP(hipMalloc(c, sizeof(int) * (size_t)n));
   TF_HIP(hipMalloc(&h->flags, sizeof(int) * 2));
@@ -1811,20 +1771,13 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
     o.e = pb.add_ints(L.e);
     o.ea = pb.add_ints(L.ea);
     o.eb = pb.add_ints(L.eb);
-    std::vector<void*> ye, le, ue, pinv, kr, kc, tbv;
+    std::vector<void*> ye, le, ue;
     for (int b = 0; b < o.ne; ++b) {
       ye.push_back(blk(D, L.e[b]));
       le.push_back(blk(Lm, L.e[b]));
       ue.push_back(blk(Um, L.e[b]));
-      pinv.push_back((char*)h->Pinv + h->es * PB * PB * b);
-      kr.push_back((char*)h->Kr + h->es * PB * (size_t)m * b);
-      kc.push_back((char*)h->Kc + h->es * PB * (size_t)m * b);
-      tbv.push_back((char*)h->Tb + h->es * PB * (size_t)m * b);
     }
-    // Ye must be followed by the snapshot pointer lists (see invert_batch)
-    std::vector<void*> ychain = ye;
-    for (auto* v : {&pinv, &kr, &kc, &tbv}) ychain.insert(ychain.end(), v->begin(), v->end());
-    o.Ye = pb.add_ptrs(ychain);
+    o.Ye = pb.add_ptrs(ye);
     o.Le = pb.add_ptrs(le);
     o.Ue = pb.add_ptrs(ue);
     o.k = pb.add_ints(L.k);
@@ -2015,7 +1968,7 @@ int tf_bcr_destroy(tf_bcr* h) {
     if (g->graph) (void)hipGraphDestroy(g->graph);
   }
   if (h->cap) (void)hipStreamDestroy(h->cap);
-  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kr, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
+  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
                   (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
                   (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
                   (void*)h->topsync, h->Z, h->zpool, h->xtab})

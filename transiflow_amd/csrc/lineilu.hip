@@ -30,7 +30,6 @@
 
 namespace {
 
-using tf::gj::PB;
 constexpr int KL = 16;  // off-line couplings kept per row and per column
 constexpr int NDIR = 6;
 __constant__ int c_dj[NDIR] = {-1, 1, 0, 0, -1, 1};
@@ -270,8 +269,8 @@ struct tf_lineilu {
   void* W;             // max colour count x m x m (Schur pass buffer)
   Cp *rc, *cc;         // n x KL row / column coupling lists
   int *nrc, *ncc;
-  void *Pinv, *Kr, *Kc, *Tb;  // Gauss-Jordan panel scratch (max colour count)
-  void** lists;        // per colour: Xp | pinv | kr | kc | tb pointer lists (device)
+  void *Pinv, *Kc, *Tb;  // scratch of the inversions (gj.h), largest colour
+  void** lists;        // pivots of every colour, colour by colour (device)
   int lists_off[4];
   int* flags;          // [0] structure errors, [1] perturbed pivots
   int* flags_host;
@@ -280,42 +279,14 @@ struct tf_lineilu {
 
 namespace {
 
+// In-place inversion of the pivots of colour c (blocked Gauss-Jordan).  A pivot that
+// is still singular (a local pressure null space the Schur updates did not remove) is
+// regularised: its zero pivot becomes 1e-3 of the panel's largest entry, the scale of
+// the smallest regular pivots.
 template <typename T>
-void gj_gemm(int M, int N, int K, void** A, int lda, void** B, int ldb, void** C, int ldc, double alpha, double beta,
-             int batch, hipStream_t st) {
-  if (batch <= 0) return;
-  TF_PROF_WORK(tf::PROF_GEMM, 2.0 * M * N * K * batch);
-  TF_PROF_BEGIN(tf::PROF_GEMM, st);
-  tf::gemm_batched<T>(M, N, K, (T* const*)A, lda, (T* const*)B, ldb, (T* const*)C, ldc, alpha, beta, batch, st);
-  TF_PROF_END(tf::PROF_GEMM, st);
-}
-
-// In-place inversion of the pivots of colour c (blocked Gauss-Jordan).
-template <typename T>
-void invert_colour(tf_lineilu* h, int c, hipStream_t st) {
-  const int m = h->m, batch = h->count[c];
-  if (batch == 0) return;
-  void** Xp = h->lists + h->lists_off[c];
-  void** pinvp = Xp + batch;
-  void** krp = pinvp + batch;
-  void** kcp = krp + batch;
-  void** tbp = kcp + batch;
-  const long sz = (long)PB * m;
-  const int gcopy = (int)((sz + 255) / 256) < 1024 ? (int)((sz + 255) / 256) : 1024;
-  for (int k0 = 0; k0 < m; k0 += PB) {
-    const int pb = m - k0 < PB ? m - k0 : PB;
-    // a pivot that is still singular (a local pressure null space the Schur
-    // updates did not remove) is regularised: its zero pivot becomes 1e-3 of the
-    // panel's largest entry, the scale of the smallest regular pivots
-    hipLaunchKernelGGL(tf::gj::k_panel<T>, dim3(batch), dim3(512), 0, st, m, k0, pb, (T* const*)Xp, (T*)h->Pinv,
-                       h->flags + 1, 1e-3);
-    hipLaunchKernelGGL(tf::gj::k_panel_copy<T>, dim3(gcopy, batch), dim3(256), 0, st, m, k0, pb, (T* const*)Xp,
-                       (T*)h->Kr, (T*)h->Kc);
-    gj_gemm<T>(pb, m, pb, pinvp, pb, krp, m, tbp, m, 1.0, 0.0, batch, st);
-    gj_gemm<T>(m, m, pb, kcp, pb, tbp, m, Xp, m, -1.0, 1.0, batch, st);
-    hipLaunchKernelGGL(tf::gj::k_panel_store<T>, dim3(gcopy, batch), dim3(256), 0, st, m, k0, pb, (T* const*)Xp,
-                       (const T*)h->Tb);
-  }
+int invert_colour(tf_lineilu* h, int c, hipStream_t st) {
+  const tf::gj::Scratch<T> w{(T*)h->Pinv, (T*)h->Kc, (T*)h->Tb};
+  return tf::gj::invert<T>(h->m, (T* const*)(h->lists + h->lists_off[c]), h->count[c], w, h->flags + 1, 1e-3, st);
 }
 
 int grid_of(long work) {
@@ -348,7 +319,7 @@ int factor_impl(tf_lineilu* h, const int* rp, const int* ci, const double* v, in
                            lines, (T*)h->P, h->rc, h->nrc, (const T*)h->W);
       }
     }
-    invert_colour<T>(h, c, st);
+    if (int e = invert_colour<T>(h, c, st)) return e;
     TF_LAUNCH_CHECK("line ILU colour");
   }
   return 0;
@@ -389,14 +360,13 @@ int create_impl(tf_lineilu* h) {
   TF_HIP(hipMalloc(&h->cc, sizeof(Cp) * KL * (size_t)h->n));
   TF_HIP(hipMalloc(&h->nrc, sizeof(int) * (size_t)h->n));
   TF_HIP(hipMalloc(&h->ncc, sizeof(int) * (size_t)h->n));
-  TF_HIP(hipMalloc(&h->Pinv, h->es * PB * PB * maxc));
-  TF_HIP(hipMalloc(&h->Kr, h->es * PB * (size_t)m * maxc));
-  TF_HIP(hipMalloc(&h->Kc, h->es * PB * (size_t)m * maxc));
-  TF_HIP(hipMalloc(&h->Tb, h->es * PB * (size_t)m * maxc));
+  TF_HIP(hipMalloc(&h->Pinv, h->es * tf::gj::scratch_P() * maxc));
+  TF_HIP(hipMalloc(&h->Kc, h->es * tf::gj::scratch_K(m) * maxc));
+  TF_HIP(hipMalloc(&h->Tb, h->es * tf::gj::scratch_K(m) * maxc));
   TF_HIP(hipMalloc(&h->flags, sizeof(int) * 2));
   TF_HIP(hipHostMalloc(&h->flags_host, sizeof(int) * 2, hipHostMallocDefault));
   TF_HIP(hipMalloc(&h->t, h->es * (size_t)h->n));
-  // lines grouped by colour, and the Gauss-Jordan pointer lists of each colour
+  // lines grouped by colour, and the pointers to their pivots
   std::vector<int> lines;
   std::vector<void*> ptrs;
   for (int c = 0; c < h->ncolour; ++c) {
@@ -406,10 +376,6 @@ int create_impl(tf_lineilu* h) {
     for (int l = 0; l < N; ++l)
       if (colour_of(l, h->ny, h->nz, h->ncolour) == c) mine.push_back(l);
     for (int l : mine) ptrs.push_back((char*)h->P + h->es * mm * l);
-    for (size_t b = 0; b < mine.size(); ++b) ptrs.push_back((char*)h->Pinv + h->es * PB * PB * b);
-    for (size_t b = 0; b < mine.size(); ++b) ptrs.push_back((char*)h->Kr + h->es * PB * (size_t)m * b);
-    for (size_t b = 0; b < mine.size(); ++b) ptrs.push_back((char*)h->Kc + h->es * PB * (size_t)m * b);
-    for (size_t b = 0; b < mine.size(); ++b) ptrs.push_back((char*)h->Tb + h->es * PB * (size_t)m * b);
     lines.insert(lines.end(), mine.begin(), mine.end());
   }
   TF_HIP(hipMalloc(&h->lines_d, sizeof(int) * lines.size()));
@@ -451,7 +417,7 @@ int tf_lineilu_create(tf_lineilu** out, int nx, int ny, int nz, int dof, int sin
 
 int tf_lineilu_destroy(tf_lineilu* h) {
   if (!h) return 0;
-  for (void* p : {h->P, h->W, (void*)h->rc, (void*)h->cc, (void*)h->nrc, (void*)h->ncc, h->Pinv, h->Kr, h->Kc, h->Tb,
+  for (void* p : {h->P, h->W, (void*)h->rc, (void*)h->cc, (void*)h->nrc, (void*)h->ncc, h->Pinv, h->Kc, h->Tb,
                   (void*)h->flags, h->t, (void*)h->lines_d, (void*)h->lists})
     (void)hipFree(p);
   (void)hipHostFree(h->flags_host);

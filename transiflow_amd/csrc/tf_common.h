@@ -29,6 +29,20 @@ inline int fail_hip(hipError_t e, const char* where) {
   return -2;
 }
 
+#if defined(__HIPCC__)
+// A pointer to global memory as a type of its own.  One that was read from a list in
+// memory is addressed as flat memory otherwise, whose loads also hold up every wait for
+// LDS.  (A cast back to a plain pointer loses it.)
+template <typename T>
+struct Global {
+  typedef __attribute__((address_space(1))) T type;
+};
+template <typename T>
+__device__ __forceinline__ typename Global<T>::type* global_ptr(T* p) {
+  return (typename Global<T>::type*)p;
+}
+#endif
+
 // ---- opt-in kernel timing -------------------------------------------------
 // When enabled (tf_prof_enable), launches wrapped in TF_PROF_BEGIN/END record
 // a pair of HIP events on the launch stream; tf_prof_read() synchronises and
