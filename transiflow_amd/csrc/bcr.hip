@@ -44,6 +44,8 @@
 
 namespace {
 
+using tf::Global;
+using tf::global_ptr;
 constexpr int KC = 8;   // couplings per row/column to a neighbouring line
 
 struct Cpl {
@@ -230,6 +232,99 @@ __global__ __launch_bounds__(256) void k_sp_cols(int m, const Cpl* __restrict__ 
       if (q < cnt) acc += (double)prow[idx[q]] * val[q];
     T* o = O + (long)r * m + c;
     *o = (T)((accumulate ? (double)*o : 0.0) + sign * acc);
+  }
+}
+
+// All of a kept line's level-0 products in one launch.  A block forms R rows of
+// P1 = L_k Y_e1 in LDS (a few rows of Y each, a wave per row), and from them the same
+// rows of D_k - P1 U_e1 and -P1 L_e1; then the same with P2.  Y, D, L and U pass through
+// memory once and the multipliers never reach it; what remains is the latency of the
+// coupling lists and of the rows they point to, so a wave keeps every coupling's loads
+// of four column chunks in flight, and a thread the R old values of D.
+// Six launches through the multipliers took 2.32 ms for 128 lines of 768 (FP64), 1.08 ms
+// for 10 of 1600 and 6.6 ms for 16 of 4096 (FP32); this takes 1.21, 0.50 and 5.3.
+constexpr size_t L0_LDS = 65536;
+
+struct Couplings {
+  const Cpl* c;
+  const int* n;
+};
+
+template <typename T, int R, int NT>
+__global__ __launch_bounds__(NT) void k_level0(int m, const int* __restrict__ k_line, const int* __restrict__ fa,
+                                                const int* __restrict__ fb, T* const* __restrict__ Y1p,
+                                                T* const* __restrict__ Y2p, T* const* __restrict__ Dp,
+                                                T* const* __restrict__ Lp, T* const* __restrict__ Up, Couplings Lr,
+                                                Couplings Ur, Couplings Ut, Couplings Lt) {
+  extern __shared__ __align__(16) char lds[];
+  T* prow = (T*)lds;  // R rows of m
+  const int b = blockIdx.y, r0 = blockIdx.x * R;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long line = (long)k_line[b] * m;
+  for (int side = 0; side < 2; ++side) {
+    const T* Yg = side ? Y2p[b] : Y1p[b];
+    if (!Yg) continue;
+    typename Global<const T>::type* Y = global_ptr(Yg);
+    const Couplings rows = side ? Ur : Lr;   // row couplings of line k into the neighbour
+    const Couplings same = side ? Lt : Ut;   // the neighbour's rows into the columns of line k
+    const Couplings far = side ? Ut : Lt;    // ... into the columns of the line beyond
+    const int beyond = side ? fb[b] : fa[b];
+    if (side) __syncthreads();  // the first side's rows are consumed
+    constexpr int NW = NT / 64, PARTS = NW > R ? NW / R : 1;  // waves per row
+    for (int i = wave / PARTS; i < R; i += NW / PARTS) {
+      if (r0 + i >= m) break;
+      const long r = line + r0 + i;
+      const int cnt = __builtin_amdgcn_readfirstlane(rows.n[r]);
+      Cpl cp{0, 0, 0.0};
+      if (lane < cnt) cp = rows.c[r * KC + lane];
+      for (int c0 = lane + 256 * (wave % PARTS); c0 < m; c0 += 256 * PARTS) {
+        double acc[4] = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int q = 0; q < KC; ++q) {
+          if (q >= cnt) break;
+          const long at = (long)__builtin_amdgcn_readlane(cp.idx, q) * m;
+          const double v = __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(cp.val), q),
+                                            __builtin_amdgcn_readlane(__double2loint(cp.val), q));
+          T y[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) y[u] = c0 + 64 * u < m ? Y[at + c0 + 64 * u] : (T)0;
+#pragma unroll
+          for (int u = 0; u < 4; ++u) acc[u] += v * (double)y[u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (c0 + 64 * u < m) prow[i * m + c0 + 64 * u] = (T)acc[u];
+      }
+    }
+    __syncthreads();
+    typename Global<T>::type* D = global_ptr(Dp[b]);
+    typename Global<T>::type* F = global_ptr(side ? Up[b] : Lp[b]);
+    for (int c = threadIdx.x; c < m; c += NT) {
+      T d[R];
+#pragma unroll
+      for (int i = 0; i < R; ++i) d[i] = r0 + i < m ? D[(long)(r0 + i) * m + c] : (T)0;
+      const long col[2] = {line + c, beyond >= 0 ? (long)beyond * m + c : 0};
+      const int cnt[2] = {same.n[col[0]], beyond >= 0 ? far.n[col[1]] : 0};
+      double acc[2][R];
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        const Couplings& cl = t ? far : same;
+#pragma unroll
+        for (int i = 0; i < R; ++i) acc[t][i] = 0.0;
+        for (int q = 0; q < cnt[t]; ++q) {
+          const Cpl cp = cl.c[col[t] * KC + q];
+#pragma unroll
+          for (int i = 0; i < R; ++i) acc[t][i] += (double)prow[i * m + cp.idx] * cp.val;
+        }
+      }
+#pragma unroll
+      for (int i = 0; i < R; ++i)
+        if (r0 + i < m) {
+          const long e = (long)(r0 + i) * m + c;
+          D[e] = (T)((double)d[i] - acc[0][i]);
+          if (beyond >= 0) F[e] = (T)(-acc[1][i]);
+        }
+    }
   }
 }
 
@@ -1069,15 +1164,19 @@ struct BcrLevelDev {
   int *k, *k1, *k2;        // kept lines and their eliminated neighbours (-1: none)
   void **P1, **P2;         // per kept line
   // operand lists of the sub-batches (kept lines with e1 / with e2 / with a line before e1 / after e2)
-  int n_p1, n_p2, n_fa, n_fb, n_nofa, n_nofb;
+  int n_p1, n_p2, n_fa, n_fb;
   int *k_hase1_line, *k_hase2_line, *k_fa_line, *k_fb_line;
-  void **g_p1_A, **g_p1_B, **g_p1_C;  // P1 = L_k Y_e1
-  void **g_d1_A, **g_d1_B;            // D_k -= P1 U_e1
-  void **g_p2_A, **g_p2_B, **g_p2_C;  // P2 = U_k Y_e2
-  void **g_d2_A, **g_d2_B;            // D_k -= P2 L_e2
-  void **g_fa_A, **g_fa_B, **g_fa_C;  // L_k = -P1 L_e1
-  void **g_fb_A, **g_fb_B, **g_fb_C;  // U_k = -P2 U_e2
-  void **z_fa, **z_fb;                // L_k (U_k) that become zero
+  // n_p1 products P1 = L_k Y_e1, then n_p2 products P2 = U_k Y_e2
+  void **g_p_A, **g_p_B, **g_p_C;
+  // per kept line D_k -= P1 U_e1 + P2 L_e2 (null: no such neighbour)
+  void **g_d_A1, **g_d_B1, **g_d_A2, **g_d_B2, **g_d_C;
+  // n_fa products L_k = -P1 L_e1, then n_fb products U_k = -P2 U_e2
+  void **g_f_A, **g_f_B, **g_f_C;
+  // level 0, per kept line: Y_e1, Y_e2, D_k, L_k, U_k and the lines before e1 and after
+  // e2 (null, -1: none)
+  void **z_Y1, **z_Y2, **z_D, **z_L, **z_U;
+  int *z_fa, *z_fb;
+  void **g_d1_A, **g_d2_A;            // D_k of the lines with e1 (e2)
   // fused factors: L_e <- Y_e L_e, U_e <- Y_e U_e (through the scratch W) at levels >= 1
   int n_yl, n_yu;
   void **g_yl_A, **g_yl_B, **g_yl_C;  // Y_e, L_e, W
@@ -1168,21 +1267,18 @@ void gemm(int M, int N, int K, void** A, int lda, void** B, int ldb, void** C, i
   TF_PROF_END(tf::PROF_GEMM, st);
 }
 
-// The level GEMMs of an FP32 factor, optionally on BF16 terms (tf_bcr_set_gemm_split).
+// m x m x m products of a level (A2, B2: a second pair per product), those of an FP32
+// factor optionally on BF16 terms (tf_bcr_set_gemm_split); n: products in all.
 template <typename T>
-void level_gemm(tf_bcr* h, int M, int N, int K, void** A, int lda, void** B, int ldb, void** C, int ldc, double alpha,
-                double beta, int batch, hipStream_t st) {
-  if constexpr (sizeof(T) == 4) {
-    if (h->split && batch > 0) {
-      TF_PROF_WORK(tf::PROF_GEMM, 2.0 * M * N * K * batch);
-      TF_PROF_BEGIN(tf::PROF_GEMM, st);
-      tf::gemm_batched_split(h->split, M, N, K, (float* const*)A, lda, (float* const*)B, ldb, (float* const*)C, ldc,
-                             alpha, beta, batch, st);
-      TF_PROF_END(tf::PROF_GEMM, st);
-      return;
-    }
-  }
-  gemm<T>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
+void level_gemm(tf_bcr* h, void** A, void** B, void** C, double alpha, double beta, int batch, int n, hipStream_t st,
+                void** A2 = nullptr, void** B2 = nullptr) {
+  const int m = h->m;
+  if (batch <= 0) return;
+  TF_PROF_WORK(tf::PROF_GEMM, 2.0 * m * m * (double)m * n);
+  TF_PROF_BEGIN(tf::PROF_GEMM, st);
+  tf::gemm_batched<T>(m, m, m, (T* const*)A, m, (T* const*)B, m, (T* const*)C, m, alpha, beta, batch, st,
+                      (T* const*)A2, (T* const*)B2, h->split);
+  TF_PROF_END(tf::PROF_GEMM, st);
 }
 
 // the captured applies (every vector type and column count) are made again on next use
@@ -1192,6 +1288,46 @@ void drop_graphs(tf_bcr* h) {
     if (g->graph) (void)hipGraphDestroy(g->graph);
     *g = BcrGraph{};
   }
+}
+
+// Level 0, kept lines: D_k -= P1 U_e1 + P2 L_e2, L_k = -P1 L_e1, U_k = -P2 U_e2 with
+// P1 = L_k Y_e1, P2 = U_k Y_e2 and the sparse couplings of both (e1 = k-1, e2 = k+1).
+template <typename T>
+void level0(tf_bcr* h, const BcrLevelDev& L, hipStream_t st) {
+  const int m = h->m;
+  const dim3 blk(256);
+  const size_t row = sizeof(T) * (size_t)m;
+  auto go = [&](auto Rc) {
+    constexpr int R = decltype(Rc)::value, NT = R == 8 ? 256 : 1024;
+    hipLaunchKernelGGL((k_level0<T, R, NT>), dim3((m + R - 1) / R, L.nk), dim3(NT), R * row, st, m, L.k, L.z_fa,
+                       L.z_fb, (T* const*)L.z_Y1, (T* const*)L.z_Y2, (T* const*)L.z_D, (T* const*)L.z_L, (T* const*)L.z_U,
+                       Couplings{h->Lr, h->nLr}, Couplings{h->Ur, h->nUr}, Couplings{h->Ut, h->nUt},
+                       Couplings{h->Lt, h->nLt});
+  };
+  if (8 * row <= L0_LDS) return go(std::integral_constant<int, 8>());
+  if (4 * row <= L0_LDS) return go(std::integral_constant<int, 4>());
+  if (2 * row <= L0_LDS) return go(std::integral_constant<int, 2>());
+  // rows that do not fit in LDS: through the multipliers in memory
+  T* const* P1 = (T* const*)L.g_p_C;
+  T* const* P2 = P1 + L.n_p1;
+  if (L.n_p1)
+    hipLaunchKernelGGL(k_sp_rows<T>, dim3(m, L.n_p1), blk, 0, st, m, h->Lr, h->nLr, L.k_hase1_line,
+                       (T* const*)L.g_p_B, P1);
+  if (L.n_p2)
+    hipLaunchKernelGGL(k_sp_rows<T>, dim3(m, L.n_p2), blk, 0, st, m, h->Ur, h->nUr, L.k_hase2_line,
+                       (T* const*)L.g_p_B + L.n_p1, P2);
+  if (L.n_p1)
+    hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_p1), blk, 0, st, m, h->Ut, h->nUt, L.k_hase1_line, P1,
+                       (T* const*)L.g_d1_A, -1.0, 1);
+  if (L.n_p2)
+    hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_p2), blk, 0, st, m, h->Lt, h->nLt, L.k_hase2_line, P2,
+                       (T* const*)L.g_d2_A, -1.0, 1);
+  if (L.n_fa)
+    hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_fa), blk, 0, st, m, h->Lt, h->nLt, L.k_fa_line,
+                       (T* const*)L.g_f_A, (T* const*)L.g_f_C, -1.0, 0);
+  if (L.n_fb)
+    hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_fb), blk, 0, st, m, h->Ut, h->nUt, L.k_fb_line,
+                       (T* const*)L.g_f_A + L.n_fa, (T* const*)L.g_f_C + L.n_fa, -1.0, 0);
 }
 
 template <typename T>
@@ -1213,60 +1349,26 @@ int factor_impl(tf_bcr* h, const int* rp, const int* ci, const double* v, int ga
     if (int e = tf::gj::invert<T>(m, (T* const*)L.Ye, L.ne, w, h->flags + 1, 0.0, st)) return e;
     if (L.nk == 0) continue;
     if (l == 0) {
-      // sparse couplings at level 0 (e1 = k-1, e2 = k+1):
-      // P1 = L_k Y_e1, P2 = U_k Y_e2 (sparse rows of line k)
-      if (L.n_p1)
-        hipLaunchKernelGGL(k_sp_rows<T>, dim3(m, L.n_p1), dim3(256), 0, st, m, h->Lr, h->nLr, L.k_hase1_line,
-                           (T* const*)L.g_p1_B, (T* const*)L.g_p1_C);
-      if (L.n_p2)
-        hipLaunchKernelGGL(k_sp_rows<T>, dim3(m, L.n_p2), dim3(256), 0, st, m, h->Ur, h->nUr, L.k_hase2_line,
-                           (T* const*)L.g_p2_B, (T* const*)L.g_p2_C);
-      // D_k -= P1 U_e1 (rows of line k-1 into the columns of line k: Ut)
-      // D_k -= P2 L_e2 (rows of line k+1 into the columns of line k: Lt)
-      if (L.n_p1)
-        hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_p1), dim3(256), 0, st, m, h->Ut, h->nUt,
-                           L.k_hase1_line,
-                           (T* const*)L.g_p1_C, (T* const*)L.g_d1_A, -1.0, 1);
-      if (L.n_p2)
-        hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_p2), dim3(256), 0, st, m, h->Lt, h->nLt,
-                           L.k_hase2_line,
-                           (T* const*)L.g_p2_C, (T* const*)L.g_d2_A, -1.0, 1);
-      // L_k = -P1 L_e1 (columns of line k-2: Lt) ; U_k = -P2 U_e2 (columns of line k+2: Ut)
-      if (L.n_fa)
-        hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_fa), dim3(256), 0, st, m, h->Lt, h->nLt,
-                           L.k_fa_line,
-                           (T* const*)L.g_fa_A, (T* const*)L.g_fa_C, -1.0, 0);
-      if (L.n_fb)
-        hipLaunchKernelGGL(k_sp_cols<T>, spc_grid(m, L.n_fb), dim3(256), 0, st, m, h->Ut, h->nUt,
-                           L.k_fb_line,
-                           (T* const*)L.g_fb_A, (T* const*)L.g_fb_C, -1.0, 0);
-    } else {
-      level_gemm<T>(h, m, m, m, L.g_p1_A, m, L.g_p1_B, m, L.g_p1_C, m, 1.0, 0.0, L.n_p1, st);
-      level_gemm<T>(h, m, m, m, L.g_p2_A, m, L.g_p2_B, m, L.g_p2_C, m, 1.0, 0.0, L.n_p2, st);
-      level_gemm<T>(h, m, m, m, L.g_p1_C, m, L.g_d1_B, m, L.g_d1_A, m, -1.0, 1.0, L.n_p1, st);
-      level_gemm<T>(h, m, m, m, L.g_p2_C, m, L.g_d2_B, m, L.g_d2_A, m, -1.0, 1.0, L.n_p2, st);
-      level_gemm<T>(h, m, m, m, L.g_fa_A, m, L.g_fa_B, m, L.g_fa_C, m, -1.0, 0.0, L.n_fa, st);
-      level_gemm<T>(h, m, m, m, L.g_fb_A, m, L.g_fb_B, m, L.g_fb_C, m, -1.0, 0.0, L.n_fb, st);
-      if (h->fused) {
-        // the eliminated lines' L_e, U_e are not used by the factorisation after
-        // this level: replace them by Y_e L_e and Y_e U_e for the one-pass backward
-        const long mm2 = (long)m * m;
-        gemm<T>(m, m, m, L.g_yl_A, m, L.g_yl_B, m, L.g_yl_C, m, 1.0, 0.0, L.n_yl, st);
-        if (L.n_yl)
-          hipLaunchKernelGGL(k_copy_blocks<T>, dim3(256, L.n_yl), dim3(256), 0, st, mm2, (T* const*)L.g_yl_C,
-                             (T* const*)L.g_yl_B);
-        gemm<T>(m, m, m, L.g_yu_A, m, L.g_yu_B, m, L.g_yu_C, m, 1.0, 0.0, L.n_yu, st);
-        if (L.n_yu)
-          hipLaunchKernelGGL(k_copy_blocks<T>, dim3(256, L.n_yu), dim3(256), 0, st, mm2, (T* const*)L.g_yu_C,
-                             (T* const*)L.g_yu_B);
-      }
+      level0<T>(h, L, st);
+      continue;
     }
-    // couplings that no longer exist
-    const long mm = (long)m * m;
-    if (L.n_nofa)
-      hipLaunchKernelGGL(k_zero_many<T>, dim3(256, L.n_nofa), dim3(256), 0, st, mm, (T* const*)L.z_fa);
-    if (L.n_nofb)
-      hipLaunchKernelGGL(k_zero_many<T>, dim3(256, L.n_nofb), dim3(256), 0, st, mm, (T* const*)L.z_fb);
+    level_gemm<T>(h, L.g_p_A, L.g_p_B, L.g_p_C, 1.0, 0.0, L.n_p1 + L.n_p2, L.n_p1 + L.n_p2, st);
+    level_gemm<T>(h, L.g_d_A1, L.g_d_B1, L.g_d_C, -1.0, 1.0, L.nk, L.n_p1 + L.n_p2, st, L.g_d_A2, L.g_d_B2);
+    // (an L_k or U_k whose neighbour no longer exists keeps its old contents: nothing reads it)
+    level_gemm<T>(h, L.g_f_A, L.g_f_B, L.g_f_C, -1.0, 0.0, L.n_fa + L.n_fb, L.n_fa + L.n_fb, st);
+    if (h->fused) {
+      // the eliminated lines' L_e, U_e are not used by the factorisation after
+      // this level: replace them by Y_e L_e and Y_e U_e for the one-pass backward
+      const long mm2 = (long)m * m;
+      gemm<T>(m, m, m, L.g_yl_A, m, L.g_yl_B, m, L.g_yl_C, m, 1.0, 0.0, L.n_yl, st);
+      if (L.n_yl)
+        hipLaunchKernelGGL(k_copy_blocks<T>, dim3(256, L.n_yl), dim3(256), 0, st, mm2, (T* const*)L.g_yl_C,
+                           (T* const*)L.g_yl_B);
+      gemm<T>(m, m, m, L.g_yu_A, m, L.g_yu_B, m, L.g_yu_C, m, 1.0, 0.0, L.n_yu, st);
+      if (L.n_yu)
+        hipLaunchKernelGGL(k_copy_blocks<T>, dim3(256, L.n_yu), dim3(256), 0, st, mm2, (T* const*)L.g_yu_C,
+                           (T* const*)L.g_yu_B);
+    }
   }
   h->factored = 1;
   if constexpr (sizeof(T) == 4) {
@@ -1747,9 +1849,8 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   auto blk = [&](char* base, int j) -> void* { return (void*)(base + bm * (size_t)j); };
   PoolBuilder pb;
   struct Off {
-    size_t e, ea, eb, Ye, Le, Ue, k, k1, k2, P1, P2, p1A, p1B, p1C, d1A, d1B, p2A, p2B, p2C, d2A, d2B, faA, faB,
-        faC, fbA, fbB, fbC, zfa, zfb, hase1, hase2, faline, fbline, ylA, ylB, ylC, yuA, yuB, yuC;
-    int ne, nk, np1, np2, nfa, nfb, nnofa, nnofb, nyl, nyu;
+    size_t e, ea, eb, Ye, Le, Ue, k, k1, k2, P1, P2, pA, pB, pC, dA1, dB1, dA2, dB2, dC, d1A, d2A, fA, fB, fC, zY1, zY2, zL, zU, zfa, zfb, hase1, hase2, faline, fbline, ylA, ylB, ylC, yuA, yuB, yuC;
+    int ne, nk, np1, np2, nfa, nfb, nyl, nyu;
   };
   std::vector<Off> offs;
   // scratch of the fused products: the largest batch of one level (levels >= 1)
@@ -1784,18 +1885,29 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
     o.k1 = pb.add_ints(L.k1);
     o.k2 = pb.add_ints(L.k2);
     std::vector<void*> p1, p2;
-    std::vector<void*> p1A, p1B, p1C, d1A, d1B, p2A, p2B, p2C, d2A, d2B, faA, faB, faC, fbA, fbB, fbC, zfa, zfb;
-    std::vector<int> hase1, hase2, faline, fbline;
+    std::vector<void*> p1A, p1B, p1C, d1A, p2A, p2B, p2C, d2A, faA, faB, faC, fbA, fbB, fbC;
+    std::vector<void*> dA1, dB1, dA2, dB2, dC, zY1, zY2, zL, zU;
+    std::vector<int> hase1, hase2, faline, fbline, zfa, zfb;
     for (int b = 0; b < o.nk; ++b) {
       const int k = L.k[b], e1 = L.k1[b], e2 = L.k2[b], s = L.kslot[b];
       p1.push_back(blk(P1, s));
       p2.push_back(blk(P2, s));
+      dA1.push_back(e1 >= 0 ? blk(P1, s) : nullptr);
+      dB1.push_back(e1 >= 0 ? blk(Um, e1) : nullptr);
+      dA2.push_back(e2 >= 0 ? blk(P2, s) : nullptr);
+      dB2.push_back(e2 >= 0 ? blk(Lm, e2) : nullptr);
+      dC.push_back(blk(D, k));
+      zY1.push_back(e1 >= 0 ? blk(D, e1) : nullptr);
+      zY2.push_back(e2 >= 0 ? blk(D, e2) : nullptr);
+      zL.push_back(blk(Lm, k));
+      zU.push_back(blk(Um, k));
+      zfa.push_back(e1 >= 0 ? L.kfa[b] : -1);
+      zfb.push_back(e2 >= 0 ? L.kfb[b] : -1);
       if (e1 >= 0) {
         p1A.push_back(blk(Lm, k));
         p1B.push_back(blk(D, e1));
         p1C.push_back(blk(P1, s));
         d1A.push_back(blk(D, k));
-        d1B.push_back(blk(Um, e1));
         hase1.push_back(k);
       }
       if (e2 >= 0) {
@@ -1803,7 +1915,6 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
         p2B.push_back(blk(D, e2));
         p2C.push_back(blk(P2, s));
         d2A.push_back(blk(D, k));
-        d2B.push_back(blk(Lm, e2));
         hase2.push_back(k);
       }
       if (e1 >= 0 && L.kfa[b] >= 0) {
@@ -1811,48 +1922,47 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
         faB.push_back(blk(Lm, e1));
         faC.push_back(blk(Lm, k));
         faline.push_back(L.kfa[b]);
-      } else {
-        zfa.push_back(blk(Lm, k));
       }
       if (e2 >= 0 && L.kfb[b] >= 0) {
         fbA.push_back(blk(P2, s));
         fbB.push_back(blk(Um, e2));
         fbC.push_back(blk(Um, k));
         fbline.push_back(L.kfb[b]);
-      } else {
-        zfb.push_back(blk(Um, k));
       }
     }
+    auto joined = [](std::vector<void*> a, const std::vector<void*>& b) {
+      a.insert(a.end(), b.begin(), b.end());
+      return a;
+    };
     o.P1 = pb.add_ptrs(p1);
     o.P2 = pb.add_ptrs(p2);
     o.np1 = (int)p1A.size();
-    o.p1A = pb.add_ptrs(p1A);
-    o.p1B = pb.add_ptrs(p1B);
-    o.p1C = pb.add_ptrs(p1C);
-    o.d1A = pb.add_ptrs(d1A);
-    o.d1B = pb.add_ptrs(d1B);
-    o.hase1 = pb.add_ints(hase1);
     o.np2 = (int)p2A.size();
-    o.p2A = pb.add_ptrs(p2A);
-    o.p2B = pb.add_ptrs(p2B);
-    o.p2C = pb.add_ptrs(p2C);
+    o.pA = pb.add_ptrs(joined(p1A, p2A));
+    o.pB = pb.add_ptrs(joined(p1B, p2B));
+    o.pC = pb.add_ptrs(joined(p1C, p2C));
+    o.dA1 = pb.add_ptrs(dA1);
+    o.dB1 = pb.add_ptrs(dB1);
+    o.dA2 = pb.add_ptrs(dA2);
+    o.dB2 = pb.add_ptrs(dB2);
+    o.dC = pb.add_ptrs(dC);
+    o.d1A = pb.add_ptrs(d1A);
     o.d2A = pb.add_ptrs(d2A);
-    o.d2B = pb.add_ptrs(d2B);
+    o.hase1 = pb.add_ints(hase1);
     o.hase2 = pb.add_ints(hase2);
     o.nfa = (int)faA.size();
-    o.faA = pb.add_ptrs(faA);
-    o.faB = pb.add_ptrs(faB);
-    o.faC = pb.add_ptrs(faC);
-    o.faline = pb.add_ints(faline);
     o.nfb = (int)fbA.size();
-    o.fbA = pb.add_ptrs(fbA);
-    o.fbB = pb.add_ptrs(fbB);
-    o.fbC = pb.add_ptrs(fbC);
+    o.fA = pb.add_ptrs(joined(faA, fbA));
+    o.fB = pb.add_ptrs(joined(faB, fbB));
+    o.fC = pb.add_ptrs(joined(faC, fbC));
+    o.faline = pb.add_ints(faline);
     o.fbline = pb.add_ints(fbline);
-    o.nnofa = (int)zfa.size();
-    o.zfa = pb.add_ptrs(zfa);
-    o.nnofb = (int)zfb.size();
-    o.zfb = pb.add_ptrs(zfb);
+    o.zY1 = pb.add_ptrs(zY1);
+    o.zY2 = pb.add_ptrs(zY2);
+    o.zL = pb.add_ptrs(zL);
+    o.zU = pb.add_ptrs(zU);
+    o.zfa = pb.add_ints(zfa);
+    o.zfb = pb.add_ints(zfb);
     // fused products Y_e L_e, Y_e U_e of the eliminated lines at levels >= 1 (W: scratch slots)
     std::vector<void*> ylA, ylB, ylC, yuA, yuB, yuC;
     if (l_index > 0) {
@@ -1921,33 +2031,33 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
     L.P1 = (void**)(P + o.P1);
     L.P2 = (void**)(P + o.P2);
     L.n_p1 = o.np1;
-    L.g_p1_A = (void**)(P + o.p1A);
-    L.g_p1_B = (void**)(P + o.p1B);
-    L.g_p1_C = (void**)(P + o.p1C);
-    L.g_d1_A = (void**)(P + o.d1A);
-    L.g_d1_B = (void**)(P + o.d1B);
-    L.k_hase1_line = (int*)(P + o.hase1);
     L.n_p2 = o.np2;
-    L.g_p2_A = (void**)(P + o.p2A);
-    L.g_p2_B = (void**)(P + o.p2B);
-    L.g_p2_C = (void**)(P + o.p2C);
-    L.g_d2_A = (void**)(P + o.d2A);
-    L.g_d2_B = (void**)(P + o.d2B);
-    L.k_hase2_line = (int*)(P + o.hase2);
     L.n_fa = o.nfa;
-    L.g_fa_A = (void**)(P + o.faA);
-    L.g_fa_B = (void**)(P + o.faB);
-    L.g_fa_C = (void**)(P + o.faC);
-    L.k_fa_line = (int*)(P + o.faline);
     L.n_fb = o.nfb;
-    L.g_fb_A = (void**)(P + o.fbA);
-    L.g_fb_B = (void**)(P + o.fbB);
-    L.g_fb_C = (void**)(P + o.fbC);
+    L.g_p_A = (void**)(P + o.pA);
+    L.g_p_B = (void**)(P + o.pB);
+    L.g_p_C = (void**)(P + o.pC);
+    L.g_d_A1 = (void**)(P + o.dA1);
+    L.g_d_B1 = (void**)(P + o.dB1);
+    L.g_d_A2 = (void**)(P + o.dA2);
+    L.g_d_B2 = (void**)(P + o.dB2);
+    L.g_d_C = (void**)(P + o.dC);
+    L.g_d1_A = (void**)(P + o.d1A);
+    L.g_d2_A = (void**)(P + o.d2A);
+    L.g_f_A = (void**)(P + o.fA);
+    L.g_f_B = (void**)(P + o.fB);
+    L.g_f_C = (void**)(P + o.fC);
+    L.z_Y1 = (void**)(P + o.zY1);
+    L.z_Y2 = (void**)(P + o.zY2);
+    L.z_D = (void**)(P + o.dC);
+    L.z_L = (void**)(P + o.zL);
+    L.z_U = (void**)(P + o.zU);
+    L.k_hase1_line = (int*)(P + o.hase1);
+    L.k_hase2_line = (int*)(P + o.hase2);
+    L.k_fa_line = (int*)(P + o.faline);
     L.k_fb_line = (int*)(P + o.fbline);
-    L.n_nofa = o.nnofa;
-    L.z_fa = (void**)(P + o.zfa);
-    L.n_nofb = o.nnofb;
-    L.z_fb = (void**)(P + o.zfb);
+    L.z_fa = (int*)(P + o.zfa);
+    L.z_fb = (int*)(P + o.zfb);
     L.n_yl = o.nyl;
     L.g_yl_A = (void**)(P + o.ylA);
     L.g_yl_B = (void**)(P + o.ylB);

@@ -69,7 +69,7 @@ __device__ __forceinline__ void tf_split4(const float v[4], tf_bf16x4& hi, tf_bf
   }
 }
 
-// One BM x BN tile of A B on 256 threads (4 waves, 2 x 2; each wave TM x TN MFMA
+// One BM x BN tile of A B (added to acc with add) on 256 threads (4 waves, 2 x 2; each wave TM x TN MFMA
 // tiles).  K is consumed in chunks of BK through two LDS buffers: while a chunk is
 // multiplied the next one is stored from registers into the other buffer and the one
 // after that is loaded, so a chunk costs one barrier and its loads have a whole
@@ -109,14 +109,18 @@ struct GemmTile {
 
   static __device__ __forceinline__ void run(int M, int N, int K, GT* __restrict__ A, int lda,
                                              GT* __restrict__ B, int ldb, int m0, int n0, Lds& sh,
-                                             acc_t (&acc)[TM][TN]) {
+                                             acc_t (&acc)[TM][TN], bool add = false) {
     const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
     const int wm0 = (wave >> 1) * (BM / 2), wn0 = (wave & 1) * (BN / 2);
     const int lr = lane & 15, lk = lane >> 4;
+    if (add) {
+      __syncthreads();  // an earlier product of the block has left the buffers
+    } else {
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+      for (int i = 0; i < TM; ++i)
 #pragma unroll
-      for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+        for (int j = 0; j < TN; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    }
     V va[FAST ? NA / W : 1], vb[FAST ? NB / W : 1];
     T ra[FAST ? 1 : NA], rb[FAST ? 1 : NB];
     GT* pa[FAST ? NA / W : 1];
@@ -246,14 +250,16 @@ inline bool gemm_fast(int N, int K, int lda, int ldb, int BK = 16) {
   return lda % W == 0 && ldb % W == 0 && N % W == 0 && K % BK == 0 && K > 0;
 }
 
-// C_b = alpha A_b B_b + beta C_b (ADD: beta is not zero).  The old values of C are
+// C_b = alpha (A_b B_b [+ A2_b B2_b]) + beta C_b (ADD: beta is not zero).  A2 may be a
+// null list; with one, null operands of either pair leave that product out.  The old values of C are
 // read before the product is formed: read after it they stand alone at the end of
 // every tile (the rank-64 update of 128 matrices of 768 took 1.7 times as long).
 template <typename T, int BM, int BN, int MINW, bool FAST, bool ADD, int SPLIT = 0, int BK = 16>
 __global__ __launch_bounds__(256, MINW) void k_gemm_mfma(int M, int N, int K, T* const* __restrict__ Ap,
                                                          int lda, T* const* __restrict__ Bp, int ldb,
                                                          T* const* __restrict__ Cp, int ldc, double alpha,
-                                                         double beta) {
+                                                         double beta, T* const* __restrict__ A2p,
+                                                         T* const* __restrict__ B2p) {
   typedef GemmTile<T, BM, BN, BK, FAST, SPLIT> Tile;
   __shared__ __align__(16) typename Tile::Lds sh;
   typename Global<T>::type* __restrict__ C = global_ptr(Cp[blockIdx.z]);
@@ -271,7 +277,9 @@ __global__ __launch_bounds__(256, MINW) void k_gemm_mfma(int M, int N, int K, T*
         }
   }
   typename Tile::acc_t acc[Tile::TM][Tile::TN];
-  Tile::run(M, N, K, global_ptr(Ap[blockIdx.z]), lda, global_ptr(Bp[blockIdx.z]), ldb, m0, n0, sh, acc);
+  const T *A = Ap[blockIdx.z], *A2 = A2p ? A2p[blockIdx.z] : nullptr;
+  if (A || !A2p) Tile::run(M, N, K, global_ptr(A), lda, global_ptr((const T*)Bp[blockIdx.z]), ldb, m0, n0, sh, acc);
+  if (A2) Tile::run(M, N, K, global_ptr(A2), lda, global_ptr((const T*)B2p[blockIdx.z]), ldb, m0, n0, sh, acc, A != nullptr);
 #pragma unroll
   for (int i = 0; i < Tile::TM; ++i)
 #pragma unroll
@@ -301,11 +309,11 @@ enum GemmTileId : int { GEMM_128x128 = 0, GEMM_64x64 = 1, GEMM_32x32 = 2, GEMM_T
 
 template <typename T, int BM, int BN, int MINW, int SPLIT, int BK = 16>
 inline void gemm_launch_tile(int M, int N, int K, T* const* A, int lda, T* const* B, int ldb, T* const* C, int ldc,
-                             double alpha, double beta, int batch, hipStream_t st) {
+                             double alpha, double beta, int batch, hipStream_t st, T* const* A2, T* const* B2) {
   const dim3 grid((N + BN - 1) / BN, (M + BM - 1) / BM, batch);
   auto go = [&](auto fast, auto add) {
     hipLaunchKernelGGL((k_gemm_mfma<T, BM, BN, MINW, decltype(fast)::value, decltype(add)::value, SPLIT, BK>), grid,
-                       dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta);
+                       dim3(256), 0, st, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, A2, B2);
   };
   const bool f = gemm_fast<T>(N, K, lda, ldb, BK), a = beta != 0.0;
   if (f && a) go(std::true_type(), std::true_type());
@@ -316,40 +324,36 @@ inline void gemm_launch_tile(int M, int N, int K, T* const* A, int lda, T* const
 
 template <typename T, int SPLIT = 0>
 inline void gemm_launch(int tile, int M, int N, int K, T* const* A, int lda, T* const* B, int ldb, T* const* C,
-                        int ldc, double alpha, double beta, int batch, hipStream_t st) {
+                        int ldc, double alpha, double beta, int batch, hipStream_t st, T* const* A2 = nullptr,
+                        T* const* B2 = nullptr) {
   switch (tile) {
     case GEMM_128x128:
-      gemm_launch_tile<T, 128, 128, 2, SPLIT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
+      gemm_launch_tile<T, 128, 128, 2, SPLIT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
       break;
     case GEMM_32x32:
-      gemm_launch_tile<T, 32, 32, 4, SPLIT, 32>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
+      gemm_launch_tile<T, 32, 32, 4, SPLIT, 32>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
       break;
     default:
-      gemm_launch_tile<T, 64, 64, 4, SPLIT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
+      gemm_launch_tile<T, 64, 64, 4, SPLIT>(M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
   }
 }
 
 int gemm_tuned_tile(int single, int M, int N, int K, int batch, hipStream_t st);
 
-// FP32 GEMM on BF16 terms of the operands (split 1: hi*hi; 3: hi*hi + hi*lo + lo*hi),
-// with the tile the tuner picked for the FP32 kernel of the same shape.
-inline void gemm_batched_split(int split, int M, int N, int K, float* const* A, int lda, float* const* B, int ldb,
-                               float* const* C, int ldc, double alpha, double beta, int batch, hipStream_t st) {
-  if (batch <= 0 || M <= 0 || N <= 0) return;
-  const int tile = gemm_tuned_tile(1, M, N, K, batch, st);
-  if (split == 1)
-    gemm_launch<float, 1>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
-  else
-    gemm_launch<float, 3>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
-}
-
-// C_b = alpha A_b B_b + beta C_b for b < batch (device pointer lists).
+// C_b = alpha (A_b B_b [+ A2_b B2_b]) + beta C_b for b < batch (device pointer lists).
+// split (float only): 1 or 3 BF16 terms per operand (hi*hi; hi*hi + hi*lo + lo*hi), with
+// the tile that the tuner picked for the FP32 kernel of the same shape.
 template <typename T>
 inline void gemm_batched(int M, int N, int K, T* const* A, int lda, T* const* B, int ldb, T* const* C, int ldc,
-                         double alpha, double beta, int batch, hipStream_t st) {
+                         double alpha, double beta, int batch, hipStream_t st, T* const* A2 = nullptr,
+                         T* const* B2 = nullptr, int split = 0) {
   if (batch <= 0 || M <= 0 || N <= 0) return;
   const int tile = gemm_tuned_tile(sizeof(T) == 4, M, N, K, batch, st);
-  gemm_launch<T>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st);
+  if constexpr (sizeof(T) == 4) {
+    if (split == 1) return gemm_launch<T, 1>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
+    if (split == 3) return gemm_launch<T, 3>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
+  }
+  gemm_launch<T>(tile, M, N, K, A, lda, B, ldb, C, ldc, alpha, beta, batch, st, A2, B2);
 }
 
 }  // namespace tf

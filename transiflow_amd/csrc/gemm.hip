@@ -49,11 +49,12 @@ int time_candidates(int M, int N, int K, int batch, hipStream_t st) {
       // the first round wakes the device's clocks (the first candidate timed on an idle
       // device looks a quarter slower); the second decides
       float best_ms = 0.f;
+      const int reps = 2.0 * M * N * K * batch < 1e9 ? 8 : 2;  // short launches: more of them between the events
       for (int i = 0; i < 2 * GEMM_TILES; ++i) {
         const int tile = i % GEMM_TILES;
         gemm_launch<T>(tile, M, N, K, lists, K, lists + batch, N, lists + 2 * batch, N, 1.0, 0.0, batch, st);
         (void)hipEventRecord(e0, st);
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < reps; ++r)
           gemm_launch<T>(tile, M, N, K, lists, K, lists + batch, N, lists + 2 * batch, N, 1.0, 0.0, batch, st);
         (void)hipEventRecord(e1, st);
         float ms = 0.f;
@@ -87,6 +88,13 @@ int gemm_tuned_tile(int single, int M, int N, int K, int batch, hipStream_t st) 
     if (it != s.table.end()) return it->second;
     if (s.mode == 0) return fixed_rule(single, M, N, K, batch);
   }
+  // many tiles fill the device either way: the largest tile, whose operands are reused
+  // most (the scratch operands would hide that: they are one matrix for the whole
+  // batch); few tiles: the smallest one (they last too briefly to be told apart by time)
+  const long t128 = (long)((M + 127) / 128) * ((N + 127) / 128) * batch;
+  const long t64 = (long)((M + 63) / 64) * ((N + 63) / 64) * batch;
+  if (t128 >= 2048) return GEMM_128x128;
+  if (t64 <= 256) return GEMM_32x32;
   int tile = single ? time_candidates<float>(M, N, K, batch, st) : time_candidates<double>(M, N, K, batch, st);
   if (tile < 0) tile = fixed_rule(single, M, N, K, batch);
   std::lock_guard<std::mutex> g(s.mu);
