@@ -18,6 +18,7 @@
 #include "tf_common.h"
 
 #include <cstdint>
+#include <type_traits>
 
 namespace {
 
@@ -36,52 +37,67 @@ struct Grid3 {
   int nx, ny, nz, dim;
 };
 
-// in-grid neighbour of cell (x, y, z) through tap, or -1
-__device__ __forceinline__ long neighbour(const Grid3& g, int x, int y, int z, int tap) {
-  const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = g.dim == 3 ? tap / 9 - 1 : 0;
-  const int X = x + dx, Y = y + dy, Z = z + dz;
-  if (X < 0 || X >= g.nx || Y < 0 || Y >= g.ny || Z < 0 || Z >= g.nz) return -1;
-  return (long)X + (long)g.nx * (Y + (long)g.ny * Z);
+// Cell c < ncell as coordinates.
+__device__ __forceinline__ void coordinates(const Grid3& g, long ncell, long c, int& x, int& y, int& z) {
+  if (ncell <= 0x7fffffffL) {
+    const unsigned row = (unsigned)c / (unsigned)g.nx;
+    x = (int)((unsigned)c - row * (unsigned)g.nx);
+    z = (int)(row / (unsigned)g.ny);
+    y = (int)(row - (unsigned)z * (unsigned)g.ny);
+  } else {
+    x = (int)(c % g.nx);
+    y = (int)((c / g.nx) % g.ny);
+    z = (int)(c / ((long)g.nx * g.ny));
+  }
 }
 
-// One wave: 16 cells x all output tiles.  Block: 4 waves = 64 cells.
-// W (MFMA layout, BF16) is staged in LDS; A fragments are gathered from the
-// neighbours' activations.
-constexpr int CONV_LDS = 28 * 1024;  // uint16 elements: K x N up to 864 x 32
+// Any number of input channels (the 2D networks' three).  One wave: 16 cells x all
+// output tiles.  Block: 4 waves = 64 cells.  W (MFMA layout, BF16) and, per row k of it,
+// the tap and the offset of its input from the cell's own are staged in LDS; a lane
+// keeps one bit per tap that stays in the grid, so an A entry costs a bit test and a load.
+constexpr int CONV_LDS = 28 * 1024;  // uint16 elements of W: K x N up to 864 x 32
+
+struct TapRow {
+  long off;
+  int tap, pad;
+};
 
 __global__ __launch_bounds__(256) void k_conv_fwd(Grid3 g, long ncell, int cin, int cout, int kpad, int npad,
                                                   const uint16_t* __restrict__ in, const uint16_t* __restrict__ W,
                                                   const float* __restrict__ bias, int relu, float* __restrict__ out32,
                                                   uint16_t* __restrict__ out16) {
-  __shared__ uint16_t Ws[CONV_LDS];
-  const int K = (g.dim == 3 ? 27 : 9) * cin;
+  extern __shared__ __align__(16) char conv_lds[];
+  TapRow* rows = (TapRow*)conv_lds;                  // kpad
+  uint16_t* Ws = (uint16_t*)(rows + kpad);           // kpad * npad
+  const int taps = g.dim == 3 ? 27 : 9, K = taps * cin;
   for (int e = threadIdx.x; e < kpad * npad; e += 256) Ws[e] = W[e];
+  for (int k = threadIdx.x; k < kpad; k += 256) {
+    const int tap = k / cin, dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = g.dim == 3 ? tap / 9 - 1 : 0;
+    rows[k] = TapRow{((long)dx + (long)g.nx * (dy + (long)g.ny * dz)) * cin + (k - tap * cin), k < K ? tap : 31, 0};
+  }
   __syncthreads();
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long cell0 = ((long)blockIdx.x * 4 + wave) * 16;
   const long cell = cell0 + (lane & 15);
   const int q = lane >> 4;
-  int x = 0, y = 0, z = 0;
-  const bool live = cell < ncell;
-  if (live) {
-    x = (int)(cell % g.nx);
-    y = (int)((cell / g.nx) % g.ny);
-    z = (int)(cell / ((long)g.nx * g.ny));
+  unsigned inside = 0;  // bit per tap
+  if (cell < ncell) {
+    int x, y, z;
+    coordinates(g, ncell, cell, x, y, z);
+    for (int t = 0; t < taps; ++t) {
+      const int X = x + t % 3 - 1, Y = y + (t / 3) % 3 - 1, Z = z + (g.dim == 3 ? t / 9 - 1 : 0);
+      if ((unsigned)X < (unsigned)g.nx && (unsigned)Y < (unsigned)g.ny && (unsigned)Z < (unsigned)g.nz) inside |= 1u << t;
+    }
   }
+  const uint16_t* own = in + cell * cin;
   const int ntiles = npad / 16;
   f32x4 acc0 = {0, 0, 0, 0}, acc1 = {0, 0, 0, 0};
   for (int k0 = 0; k0 < kpad; k0 += 16) {
     bf16x4 a;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int k = k0 + 4 * q + i;
-      uint16_t v = 0;
-      if (live && k < K) {
-        const int tap = k / cin, ci = k - tap * cin;
-        const long nb = neighbour(g, x, y, z, tap);
-        if (nb >= 0) v = in[nb * cin + ci];
-      }
-      a[i] = (short)v;
+      const TapRow row = rows[k0 + 4 * q + i];
+      a[i] = (inside >> row.tap) & 1u ? (short)own[row.off] : (short)0;
     }
     bf16x4 b0, b1;
 #pragma unroll
@@ -110,73 +126,37 @@ __global__ __launch_bounds__(256) void k_conv_fwd(Grid3 g, long ncell, int cin, 
   }
 }
 
-// The same layer when cin is a multiple of 4 (every layer of the 3D network and
-// its data gradients): a lane's four K entries of one MFMA step are four
-// consecutive channels of one tap, so the A fragment is one 8-byte load of the
-// neighbour's activations; W is staged transposed ([n][k]) so the B fragment
-// is one 8-byte LDS read.  Each wave computes CF_MT tiles of 16 cells, reusing
-// each B fragment CF_MT times, and a block stages W once for 64 CF_MT cells.
-// The K order of the accumulation is that of k_conv_fwd.
-constexpr int CF_MT = 4;
+// W [kpad][npad] -> LDS transposed, [n] rows of kpad + WPAD entries: four k of two n per
+// item, 8-byte stores.  The pad spreads the rows that a fragment read touches over the
+// banks (kpad alone is a multiple of 32 dwords for 32 channels).
+constexpr int WPAD = 8;
 
-template <int NT>
-__global__ __launch_bounds__(256) void k_conv_fwd_v(Grid3 g, long ncell, int cin, int cout, int kpad, int npad,
-                                                    const uint16_t* __restrict__ in, const uint16_t* __restrict__ W,
-                                                    const float* __restrict__ bias, int relu,
-                                                    float* __restrict__ out32, uint16_t* __restrict__ out16) {
-  extern __shared__ __align__(16) uint16_t Ws[];   // kpad * npad entries (dynamic: small layers keep occupancy)
-  for (int e = threadIdx.x; e < kpad * npad; e += 256) {
-    const int k = e / npad, n = e - k * npad;
-    Ws[n * kpad + k] = W[e];
-  }
-  __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int q = lane >> 4, r = lane & 15;
-  const int K = (g.dim == 3 ? 27 : 9) * cin;
-  const long base = ((long)blockIdx.x * 4 + wave) * (CF_MT * 16);
-  int xm[CF_MT], ym[CF_MT], zm[CF_MT];
-  bool livem[CF_MT];
+__device__ __forceinline__ void stage_weights(int kpad, int npad, const uint16_t* __restrict__ W,
+                                              uint16_t* __restrict__ Ws) {
+  const int kp = kpad + WPAD, half = npad / 2;
+  for (int e = threadIdx.x; e < kpad / 4 * half; e += blockDim.x) {
+    const int n = 2 * (e % half), k = 4 * (e / half);
+    bf16x4 lo, hi;
 #pragma unroll
-  for (int m = 0; m < CF_MT; ++m) {
-    const long cell = base + m * 16 + r;
-    livem[m] = cell < ncell;
-    const long c = livem[m] ? cell : 0;
-    xm[m] = (int)(c % g.nx);
-    ym[m] = (int)((c / g.nx) % g.ny);
-    zm[m] = (int)(c / ((long)g.nx * g.ny));
-  }
-  f32x4 acc[CF_MT][NT];
-#pragma unroll
-  for (int m = 0; m < CF_MT; ++m)
-#pragma unroll
-    for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0, 0, 0, 0};
-  for (int k0 = 0; k0 < kpad; k0 += 16) {
-    const int k = k0 + 4 * q;  // this lane's four K entries: channels ci..ci+3 of one tap
-    const bool kin = k < K;
-    const int tap = kin ? k / cin : 0;
-    const int ci = k - tap * cin;
-    const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = g.dim == 3 ? tap / 9 - 1 : 0;
-    bf16x4 b[NT];
-#pragma unroll
-    for (int t = 0; t < NT; ++t) b[t] = *reinterpret_cast<const bf16x4*>(&Ws[(t * 16 + r) * kpad + k]);
-    bf16x4 a[CF_MT];
-#pragma unroll
-    for (int m = 0; m < CF_MT; ++m) {
-      a[m] = bf16x4{0, 0, 0, 0};
-      const int X = xm[m] + dx, Y = ym[m] + dy, Z = zm[m] + dz;
-      if (kin && livem[m] && X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Z >= 0 && Z < g.nz) {
-        const long nb = (long)X + (long)g.nx * (Y + (long)g.ny * Z);
-        a[m] = *reinterpret_cast<const bf16x4*>(in + nb * cin + ci);
-      }
+    for (int i = 0; i < 4; ++i) {
+      const unsigned w = *reinterpret_cast<const unsigned*>(W + (k + i) * npad + n);
+      lo[i] = (short)(w & 0xffffu);
+      hi[i] = (short)(w >> 16);
     }
-#pragma unroll
-    for (int m = 0; m < CF_MT; ++m)
-#pragma unroll
-      for (int t = 0; t < NT; ++t) acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b[t], acc[m][t], 0, 0, 0);
+    *reinterpret_cast<bf16x4*>(Ws + n * kp + k) = lo;
+    *reinterpret_cast<bf16x4*>(Ws + (n + 1) * kp + k) = hi;
   }
-  // D[4 q + v][r]: cell base + 16 m + 4 q + v, output channel 16 t + r
+}
+
+// Bias, ReLU and the stores of MT x NT tiles: D[4 q + v][r] is cell base + 16 m + 4 q + v,
+// output channel 16 t + r.
+template <int MT, int NT>
+__device__ __forceinline__ void conv_store(const f32x4 (&acc)[MT][NT], long base, long ncell, int cout,
+                                           const float* __restrict__ bias, int relu, float* __restrict__ out32,
+                                           uint16_t* __restrict__ out16) {
+  const int lane = threadIdx.x & 63, q = lane >> 4, r = lane & 15;
 #pragma unroll
-  for (int m = 0; m < CF_MT; ++m)
+  for (int m = 0; m < MT; ++m)
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
       const int co = t * 16 + r;
@@ -194,150 +174,283 @@ __global__ __launch_bounds__(256) void k_conv_fwd_v(Grid3 g, long ncell, int cin
     }
 }
 
-// Partial weight gradients, one block per WG_CHUNK cells:
-//   partial[block][k][co] = sum over the block's cells of patch[cell][k] g[cell][co]
+// The same layer when cin is a multiple of 4 (every layer of the 3D network and
+// its data gradients): a lane's four K entries of one MFMA step are four
+// consecutive channels of one tap, so the A fragment is one 8-byte load of the
+// neighbour's activations; W is staged transposed ([n][k]) so the B fragment
+// is one 8-byte LDS read.  Each wave computes MT tiles of 16 cells, reusing
+// each B fragment MT times, and a block stages W once for 128 MT cells.
+// The K order of the accumulation is that of k_conv_fwd.
+// Bound by the latency of the neighbour loads: C32 (cin = 32) walks the taps with the
+// next tap's loads in flight and finds a neighbour once per tap, and small grids take
+// fewer tiles per wave, so that every CU has waves (conv_tiles).  32 -> 32 channels: 32^3 40 -> 15 us, 256^2
+// 31 -> 14 us against one step's loads at a time, 4 waves a block and four tiles always.
+template <int NT, int MT, bool C32>
+__global__ __launch_bounds__(512) void k_conv_fwd_v(Grid3 g, long ncell, int cin, int cout, int kpad, int npad,
+                                                    const uint16_t* __restrict__ in, const uint16_t* __restrict__ W,
+                                                    const float* __restrict__ bias, int relu,
+                                                    float* __restrict__ out32, uint16_t* __restrict__ out16) {
+  extern __shared__ __align__(16) uint16_t Ws[];   // npad rows of kpad + WPAD
+  stage_weights(kpad, npad, W, Ws);
+  const int kp = kpad + WPAD;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int q = lane >> 4, r = lane & 15;
+  const int taps = g.dim == 3 ? 27 : 9;
+  const long base = ((long)blockIdx.x * 8 + wave) * (MT * 16);
+  int xm[MT], ym[MT], zm[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    const long cell = base + m * 16 + r;
+    coordinates(g, ncell, cell < ncell ? cell : 0, xm[m], ym[m], zm[m]);
+    if (cell >= ncell) zm[m] = -4;  // no neighbour of a cell past the end is in the grid
+  }
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) acc[m][t] = f32x4{0, 0, 0, 0};
+  // four channels from ci of the neighbour through a tap (zero outside the grid)
+  auto piece = [&](int m, int tap, int ci, int channels) {
+    const int X = xm[m] + tap % 3 - 1, Y = ym[m] + (tap / 3) % 3 - 1, Z = zm[m] + (g.dim == 3 ? tap / 9 - 1 : 0);
+    bf16x4 a = {0, 0, 0, 0};
+    if ((unsigned)X < (unsigned)g.nx && (unsigned)Y < (unsigned)g.ny && (unsigned)Z < (unsigned)g.nz)
+      a = *reinterpret_cast<const bf16x4*>(in + ((long)X + (long)g.nx * (Y + (long)g.ny * Z)) * channels + ci);
+    return a;
+  };
+  if constexpr (C32) {
+    bf16x4 a[2][MT], nx[2][MT];
+    auto load = [&](int tap, bf16x4 (&to)[2][MT]) {
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        const int X = xm[m] + tap % 3 - 1, Y = ym[m] + (tap / 3) % 3 - 1, Z = zm[m] + (g.dim == 3 ? tap / 9 - 1 : 0);
+        to[0][m] = to[1][m] = bf16x4{0, 0, 0, 0};
+        if ((unsigned)X < (unsigned)g.nx && (unsigned)Y < (unsigned)g.ny && (unsigned)Z < (unsigned)g.nz) {
+          const uint16_t* p = in + ((long)X + (long)g.nx * (Y + (long)g.ny * Z)) * 32 + 4 * q;
+          to[0][m] = *reinterpret_cast<const bf16x4*>(p);
+          to[1][m] = *reinterpret_cast<const bf16x4*>(p + 16);
+        }
+      }
+    };
+    load(0, nx);
+    __syncthreads();
+    for (int tap = 0; tap < taps; ++tap) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) a[h][m] = nx[h][m];
+      if (tap + 1 < taps) load(tap + 1, nx);
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        bf16x4 b[NT];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          b[t] = *reinterpret_cast<const bf16x4*>(&Ws[(t * 16 + r) * kp + tap * 32 + 16 * h + 4 * q]);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+          for (int t = 0; t < NT; ++t)
+            acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[h][m], b[t], acc[m][t], 0, 0, 0);
+      }
+    }
+  } else {
+    __syncthreads();
+    const int K = taps * cin;
+#pragma unroll 2
+    for (int k0 = 0; k0 < kpad; k0 += 16) {
+      const int k = k0 + 4 * q;  // this lane's four K entries: channels ci..ci+3 of one tap
+      const int tap = k / cin;
+      bf16x4 b[NT], a[MT];
+#pragma unroll
+      for (int m = 0; m < MT; ++m) a[m] = k < K ? piece(m, tap, k - tap * cin, cin) : bf16x4{0, 0, 0, 0};
+#pragma unroll
+      for (int t = 0; t < NT; ++t) b[t] = *reinterpret_cast<const bf16x4*>(&Ws[(t * 16 + r) * kp + k]);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+          acc[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[m], b[t], acc[m][t], 0, 0, 0);
+    }
+  }
+  conv_store<MT, NT>(acc, base, ncell, cout, bias, relu, out32, out16);
+}
+
+// Tiles of 16 cells per wave: one while that gives at most two blocks of 128 cells per
+// CU, else four (a B fragment and a staging of W per four tiles).
+inline int conv_tiles(long ncell) { return ncell <= 512L * 128 ? 1 : 4; }
+
+// Partial weight and bias gradients, one block per chunk of cells:
+//   partial[block][k][co] = sum over the block's cells of patch[cell][k] g[cell][co],
+//   then 32 entries       sum over the block's cells of g32[cell][co] (the FP32 gradient)
 // as MFMAs with M = k, N = co and the cells as the reduction dimension.  The
 // block walks its cells WG_SUB at a time: the patch (all K values of WG_SUB
 // cells, zero outside the grid) and the gradient are staged transposed in LDS
 // ([k][cell], [co][cell]), so a lane's four reduction entries are one 8-byte
-// LDS read for A and for B.  The staging reads each (cell, tap) neighbour's
-// channels in 8- or 16-byte pieces.  Wave w of the WG_WAVES owns the output
-// tiles w, w + WG_WAVES, ... and keeps their accumulators in registers across
-// the whole chunk, so a block writes its partial once.
-constexpr int WG_CHUNK = 1024;
+// LDS read for A and for B.  A staging item is VEC channels of one tap for four
+// consecutive cells: four loads of VEC channels, VEC stores of four cells each.
+// Wave w of the WG_WAVES owns the k-tiles w, w + WG_WAVES, ... for both n-tiles and
+// keeps their accumulators in registers across the whole chunk, so a block writes its
+// partial once.
+// The staging bounds it (2-byte LDS stores of single cells took 331 us at 32^3 with 32
+// channels in and out, in 32 blocks); chunks are sized for about 256 blocks:
+// 20 us there, with the sum of the partials 26.
 constexpr int WG_SUB = 32;
+constexpr int WG_PITCH = WG_SUB + 4;  // LDS row pitch: 16 rows by 4 cells spread over the banks
 constexpr int WG_WAVES = 8;
-constexpr int WG_MAXT = 14;   // output tiles per wave: ceil(56 k-tiles x 2 n-tiles / 8)
+constexpr int WG_MAXT = 7;    // k-tiles per wave: 56 / 8
 constexpr int WG_KMAX = 896;  // staged K rows
 
+// cells per block (a multiple of WG_SUB) for about 256 blocks, at most 1024
+inline long wgrad_chunk(long ncell) {
+  const long c = ((ncell + 255) / 256 + WG_SUB - 1) / WG_SUB * WG_SUB;
+  return c < 1024 ? c : 1024;
+}
+inline long wgrad_blocks(long ncell) { return (ncell + wgrad_chunk(ncell) - 1) / wgrad_chunk(ncell); }
+inline size_t wgrad_lds(int kpad, int npad) { return sizeof(uint16_t) * (size_t)(kpad + npad) * WG_PITCH; }
+
 template <int VEC>   // channels per staging load: 8 (16 bytes), 4 (8 bytes) or 1
-__global__ __launch_bounds__(64 * WG_WAVES) void k_conv_wgrad(Grid3 g, long ncell, int cin, int cout, int kpad,
-                                                              int npad, const uint16_t* __restrict__ in,
+__global__ __launch_bounds__(64 * WG_WAVES) void k_conv_wgrad(Grid3 g, long ncell, int chunk, int cin, int cout,
+                                                              int kpad, int npad, const uint16_t* __restrict__ in,
                                                               const uint16_t* __restrict__ gout,
+                                                              const float* __restrict__ g32,
                                                               float* __restrict__ partial) {
-  __shared__ __align__(16) uint16_t pt[WG_KMAX * WG_SUB];   // [kpad][WG_SUB]
-  __shared__ __align__(16) uint16_t gt[32 * WG_SUB];        // [npad][WG_SUB]
+  extern __shared__ __align__(16) uint16_t lds[];
+  uint16_t* pt = lds;                     // [kpad][WG_PITCH]
+  uint16_t* gt = lds + kpad * WG_PITCH;   // [npad][WG_PITCH]
   constexpr int NT = 64 * WG_WAVES;
   const int taps = g.dim == 3 ? 27 : 9;
   const int K = taps * cin;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int q = lane >> 4, r = lane & 15;
-  const int ktiles = kpad / 16, ntiles = npad / 16, ntot = ktiles * ntiles;
+  const int ktiles = kpad / 16, ntiles = npad / 16;
   const int groups = cin / VEC;                 // channel pieces per (cell, tap)
-  const int staged_taps = (kpad + cin - 1) / cin;
-  const long c0 = (long)blockIdx.x * WG_CHUNK;
-  // K padding rows beyond the last staged tap stay zero for the whole chunk
-  for (int e = staged_taps * cin * WG_SUB + threadIdx.x; e < kpad * WG_SUB; e += NT) pt[e] = 0;
-  f32x4 acc[WG_MAXT];
+  const long c0 = (long)blockIdx.x * chunk;
+  const long c1 = c0 + chunk < ncell ? c0 + chunk : ncell;
+  // the K padding rows stay zero for the whole chunk
+  for (int e = K * WG_PITCH + threadIdx.x; e < kpad * WG_PITCH; e += NT) pt[e] = 0;
+  f32x4 acc[WG_MAXT][2];
 #pragma unroll
-  for (int t = 0; t < WG_MAXT; ++t) acc[t] = f32x4{0, 0, 0, 0};
-  for (int s0 = 0; s0 < WG_CHUNK && c0 + s0 < ncell; s0 += WG_SUB) {
-    // (piece, cell, tap) items: consecutive threads take consecutive pieces of one neighbour
-    for (int p = threadIdx.x; p < WG_SUB * staged_taps * groups; p += NT) {
+  for (int t = 0; t < WG_MAXT; ++t) acc[t][0] = acc[t][1] = f32x4{0, 0, 0, 0};
+  for (long s0 = c0; s0 < c1; s0 += WG_SUB) {
+    // (piece, four cells, tap) items: consecutive threads take consecutive pieces of one neighbour
+    for (int p = threadIdx.x; p < WG_SUB / 4 * taps * groups; p += NT) {
       const int gi = p % groups, rest = p / groups;
-      const int cl = rest % WG_SUB, tap = rest / WG_SUB;
-      const long cell = c0 + s0 + cl;
-      long nb = -1;
-      if (tap < taps && cell < ncell) {
-        const int ic = (int)cell;   // ncell < 2^31 (checked by the caller)
-        const int x = ic % g.nx, y = (ic / g.nx) % g.ny, z = ic / (g.nx * g.ny);
-        const int X = x + tap % 3 - 1, Y = y + (tap / 3) % 3 - 1, Z = z + (g.dim == 3 ? tap / 9 - 1 : 0);
-        if (X >= 0 && X < g.nx && Y >= 0 && Y < g.ny && Z >= 0 && Z < g.nz)
-          nb = (long)X + (long)g.nx * (Y + (long)g.ny * Z);
-      }
-      const int k0 = tap * cin + gi * VEC;
-      uint16_t v[VEC];
-      if (nb >= 0) {
-        const uint16_t* src = in + nb * cin + gi * VEC;
+      const int c4 = rest % (WG_SUB / 4), tap = rest / (WG_SUB / 4);
+      const int dx = tap % 3 - 1, dy = (tap / 3) % 3 - 1, dz = g.dim == 3 ? tap / 9 - 1 : 0;
+      unsigned ic = (unsigned)(s0 + 4 * c4);   // ncell < 2^31 (checked by the caller)
+      unsigned row = ic / (unsigned)g.nx;
+      int x = (int)(ic - row * (unsigned)g.nx), y = (int)(row % (unsigned)g.ny), z = (int)(row / (unsigned)g.ny);
+      uint16_t v[4][VEC];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int X = x + dx, Y = y + dy, Z = z + dz;
+        const bool inside = s0 + 4 * c4 + i < c1 && (unsigned)X < (unsigned)g.nx && (unsigned)Y < (unsigned)g.ny &&
+                            (unsigned)Z < (unsigned)g.nz;
+        const uint16_t* src = in + ((long)X + (long)g.nx * (Y + (long)g.ny * Z)) * cin + gi * VEC;
         if constexpr (VEC == 8) {
-          const uint4 w = *reinterpret_cast<const uint4*>(src);
+          uint4 w = {0, 0, 0, 0};
+          if (inside) w = *reinterpret_cast<const uint4*>(src);
           const unsigned u[4] = {w.x, w.y, w.z, w.w};
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            v[2 * j] = (uint16_t)(u[j] & 0xffffu);
-            v[2 * j + 1] = (uint16_t)(u[j] >> 16);
-          }
+          for (int j = 0; j < 8; ++j) v[i][j] = (uint16_t)(j & 1 ? u[j / 2] >> 16 : u[j / 2] & 0xffffu);
         } else if constexpr (VEC == 4) {
-          const uint2 w = *reinterpret_cast<const uint2*>(src);
-          v[0] = (uint16_t)(w.x & 0xffffu);
-          v[1] = (uint16_t)(w.x >> 16);
-          v[2] = (uint16_t)(w.y & 0xffffu);
-          v[3] = (uint16_t)(w.y >> 16);
+          uint2 w = {0, 0};
+          if (inside) w = *reinterpret_cast<const uint2*>(src);
+          const unsigned u[2] = {w.x, w.y};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i][j] = (uint16_t)(j & 1 ? u[j / 2] >> 16 : u[j / 2] & 0xffffu);
         } else {
-          v[0] = src[0];
+          v[i][0] = inside ? src[0] : (uint16_t)0;
         }
-      } else {
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) v[j] = 0;
+        if (++x == g.nx) {  // the next cell
+          x = 0;
+          if (++y == g.ny) {
+            y = 0;
+            ++z;
+          }
+        }
       }
+      const int k0 = tap * cin + gi * VEC;
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        const int k = k0 + j;
-        if (k < kpad) pt[k * WG_SUB + cl] = k < K ? v[j] : (uint16_t)0;
-      }
+      for (int j = 0; j < VEC; ++j)
+        *reinterpret_cast<bf16x4*>(&pt[(k0 + j) * WG_PITCH + 4 * c4]) =
+            bf16x4{(short)v[0][j], (short)v[1][j], (short)v[2][j], (short)v[3][j]};
     }
-    for (int e = threadIdx.x; e < npad * WG_SUB; e += NT) {
-      const int co = e / WG_SUB, cl = e % WG_SUB;
-      const long cell = c0 + s0 + cl;
-      gt[co * WG_SUB + cl] = (co < cout && cell < ncell) ? gout[cell * cout + co] : (uint16_t)0;
+    for (int e = threadIdx.x; e < npad * (WG_SUB / 4); e += NT) {
+      const int co = e % npad, c4 = e / npad;
+      bf16x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const long cell = s0 + 4 * c4 + i;
+        v[i] = (co < cout && cell < c1) ? (short)gout[cell * cout + co] : (short)0;
+      }
+      *reinterpret_cast<bf16x4*>(&gt[co * WG_PITCH + 4 * c4]) = v;
     }
     __syncthreads();
 #pragma unroll
-    for (int t = 0; t < WG_MAXT; ++t) {
-      const int tile = wave + WG_WAVES * t;
-      if (tile < ntot) {
-        const int kt = tile / ntiles, nt = tile - kt * ntiles;
+    for (int h = 0; h < WG_SUB; h += 16) {
+      const bf16x4 b0 = *reinterpret_cast<const bf16x4*>(&gt[r * WG_PITCH + h + 4 * q]);
+      bf16x4 b1 = {0, 0, 0, 0};
+      if (ntiles > 1) b1 = *reinterpret_cast<const bf16x4*>(&gt[(16 + r) * WG_PITCH + h + 4 * q]);
 #pragma unroll
-        for (int h = 0; h < WG_SUB; h += 16) {
-          const bf16x4 a = *reinterpret_cast<const bf16x4*>(&pt[(kt * 16 + r) * WG_SUB + h + 4 * q]);
-          const bf16x4 b = *reinterpret_cast<const bf16x4*>(&gt[(nt * 16 + r) * WG_SUB + h + 4 * q]);
-          acc[t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc[t], 0, 0, 0);
+      for (int t = 0; t < WG_MAXT; ++t) {
+        const int kt = wave + WG_WAVES * t;
+        if (kt < ktiles) {
+          const bf16x4 a = *reinterpret_cast<const bf16x4*>(&pt[(kt * 16 + r) * WG_PITCH + h + 4 * q]);
+          acc[t][0] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b0, acc[t][0], 0, 0, 0);
+          if (ntiles > 1) acc[t][1] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b1, acc[t][1], 0, 0, 0);
         }
       }
     }
     __syncthreads();
   }
-  float* P = partial + (long)blockIdx.x * kpad * npad;
+  const long len = (long)kpad * npad;
+  float* P = partial + (long)blockIdx.x * (len + 32);
 #pragma unroll
   for (int t = 0; t < WG_MAXT; ++t) {
-    const int tile = wave + WG_WAVES * t;
-    if (tile < ntot) {
-      const int kt = tile / ntiles, nt = tile - kt * ntiles;
+    const int kt = wave + WG_WAVES * t;
+    if (kt < ktiles) {
 #pragma unroll
-      for (int v = 0; v < 4; ++v) P[(long)(kt * 16 + 4 * q + v) * npad + nt * 16 + r] = acc[t][v];
+      for (int n = 0; n < 2; ++n)
+        if (n < ntiles)
+#pragma unroll
+          for (int v = 0; v < 4; ++v) P[(long)(kt * 16 + 4 * q + v) * npad + n * 16 + r] = acc[t][n][v];
     }
+  }
+  // bias: thread t sums channel t % cout of every (NT / cout)-th cell, then a tree per channel
+  float* red = (float*)lds;
+  const int rows = NT / cout, co = threadIdx.x % cout, first = threadIdx.x / cout;
+  float s = 0.f;
+  if (first < rows)
+    for (long c = c0 + first; c < c1; c += rows) s += g32[c * cout + co];
+  red[threadIdx.x] = s;
+  __syncthreads();
+  if (threadIdx.x < 32) {
+    float sum = 0.f;
+    if ((int)threadIdx.x < cout)
+      for (int i = 0; i < rows; ++i) sum += red[i * cout + threadIdx.x];
+    P[len + threadIdx.x] = sum;
   }
 }
 
-// out[e] = sum_b partial[b][e]  (fixed order: deterministic)
-__global__ __launch_bounds__(256) void k_sum_partials(int nb, long len, const float* __restrict__ partial,
-                                                      float* __restrict__ out) {
-  const long e = blockIdx.x * 256L + threadIdx.x;
-  if (e >= len) return;
-  float s = 0.f;
-  for (int b = 0; b < nb; ++b) s += partial[(long)b * len + e];
-  out[e] = s;
-}
-
-// bias partials: bp[block][co] = sum over the block's WG_CHUNK cells of g[cell][co] (FP32 gradient)
-__global__ __launch_bounds__(256) void k_bias_partial(long ncell, int cout, const float* __restrict__ g,
-                                                      float* __restrict__ bp) {
+// dW[e] (e < len), db[e - len] = sum_b partial[b][e]  (fixed order: deterministic).  64
+// entries per block, a quarter of the blocks' partials per wave.
+__global__ __launch_bounds__(256) void k_sum_partials(int nb, long len, int cout, const float* __restrict__ partial,
+                                                      float* __restrict__ dW, float* __restrict__ db) {
   __shared__ float sh[256];
-  const long c0 = (long)blockIdx.x * WG_CHUNK;
-  for (int co = 0; co < cout; ++co) {
-    float acc = 0.f;
-    for (int cl = threadIdx.x; cl < WG_CHUNK; cl += 256) {
-      const long cell = c0 + cl;
-      if (cell < ncell) acc += g[cell * cout + co];
-    }
-    sh[threadIdx.x] = acc;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-      if (threadIdx.x < s) sh[threadIdx.x] += sh[threadIdx.x + s];
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) bp[(long)blockIdx.x * cout + co] = sh[0];
-    __syncthreads();
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const long e = blockIdx.x * 64L + lane, pitch = len + 32;
+  float s = 0.f;
+  if (e < pitch) {
+    const float* p = partial + e;
+#pragma unroll 8
+    for (int b = wave; b < nb; b += 4) s += p[b * pitch];
+  }
+  sh[threadIdx.x] = s;
+  __syncthreads();
+  if (wave == 0) {
+    s = (sh[lane] + sh[64 + lane]) + (sh[128 + lane] + sh[192 + lane]);
+    if (e < len) dW[e] = s;
+    else if (db && e - len < cout) db[e - len] = s;
   }
 }
 
@@ -437,17 +550,29 @@ int tf_conv_fwd(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, in
   hipStream_t st = (hipStream_t)stream;
   const uint16_t* in16 = (const uint16_t*)in;
   const uint16_t* W16 = (const uint16_t*)W;
-  if (cin % 4 == 0 && ((uintptr_t)in % 8) == 0) {
-    const dim3 grid((unsigned)((ncell + 64 * CF_MT - 1) / (64 * CF_MT)));
-    const size_t lds = sizeof(uint16_t) * kpad * npad;
-    if (npad == 16)
-      hipLaunchKernelGGL(k_conv_fwd_v<1>, grid, dim3(256), lds, st, g, ncell, cin, cout, kpad, npad, in16, W16, bias,
-                         relu, out32, (uint16_t*)out16);
-    else
-      hipLaunchKernelGGL(k_conv_fwd_v<2>, grid, dim3(256), lds, st, g, ncell, cin, cout, kpad, npad, in16, W16, bias,
-                         relu, out32, (uint16_t*)out16);
+  size_t lds = (sizeof(TapRow) + sizeof(uint16_t) * npad) * (size_t)kpad;
+  if (cin % 4 == 0 && ((uintptr_t)in % 8) == 0 && ((uintptr_t)W % 4) == 0) {
+    const int mt = conv_tiles(ncell);
+    const dim3 grid((unsigned)((ncell + 128 * mt - 1) / (128 * mt)));
+    lds = sizeof(uint16_t) * (size_t)(kpad + WPAD) * npad;
+    auto go = [&](auto nt, auto tiles, auto c32) {
+      hipLaunchKernelGGL((k_conv_fwd_v<decltype(nt)::value, decltype(tiles)::value, decltype(c32)::value>), grid,
+                         dim3(512), lds, st, g, ncell, cin, cout, kpad, npad, in16, W16, bias, relu, out32,
+                         (uint16_t*)out16);
+    };
+    auto with_tiles = [&](auto nt, auto c32) {
+      if (mt == 1) go(nt, std::integral_constant<int, 1>(), c32);
+      else go(nt, std::integral_constant<int, 4>(), c32);
+    };
+    auto with_channels = [&](auto nt) {
+      if (cin == 32) with_tiles(nt, std::true_type());
+      else with_tiles(nt, std::false_type());
+    };
+    if (npad == 16) with_channels(std::integral_constant<int, 1>());
+    else with_channels(std::integral_constant<int, 2>());
   } else {
-    hipLaunchKernelGGL(k_conv_fwd, dim3((unsigned)((ncell + 63) / 64)), dim3(256), 0, st, g, ncell, cin, cout, kpad,
+    TF_HIP(hipFuncSetAttribute((const void*)k_conv_fwd, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_conv_fwd, dim3((unsigned)((ncell + 63) / 64)), dim3(256), lds, st, g, ncell, cin, cout, kpad,
                        npad, in16, W16, bias, relu, out32, (uint16_t*)out16);
   }
   TF_PROF_WORK(tf::PROF_CONV, 2.0 * ncell * (dim == 3 ? 27 : 9) * cin * cout);
@@ -456,8 +581,7 @@ int tf_conv_fwd(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, in
 }
 
 int tf_conv_wgrad_work_size(long ncell, int kpad, int npad) {
-  const long blocks = (ncell + WG_CHUNK - 1) / WG_CHUNK;
-  const long n = blocks * kpad * npad + blocks * 32;
+  const long n = wgrad_blocks(ncell) * ((long)kpad * npad + 32);
   return n > 2147483647L ? -1 : (int)n;
 }
 
@@ -469,26 +593,30 @@ int tf_conv_wgrad(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, 
   if (int e = check_layer(dim, cin, cout, kpad, npad)) return e;
   const long ncell = (long)nx * ny * nz;
   if (kpad > WG_KMAX || ncell >= (1L << 31)) return tf::fail("conv wgrad: K or the grid too large");
-  const long blocks = (ncell + WG_CHUNK - 1) / WG_CHUNK;
+  const long blocks = wgrad_blocks(ncell);
+  const int chunk = (int)wgrad_chunk(ncell);
   hipStream_t st = (hipStream_t)stream;
   Grid3 g{nx, ny, nz, dim};
   const dim3 wg_grid((unsigned)blocks), wg_block(64 * WG_WAVES);
+  const size_t lds = wgrad_lds(kpad, npad) < sizeof(float) * 64 * WG_WAVES ? sizeof(float) * 64 * WG_WAVES
+                                                                         : wgrad_lds(kpad, npad);
   const uint16_t* in16 = (const uint16_t*)in;
   const uint16_t* g16 = (const uint16_t*)gout16;
-  if (cin % 8 == 0 && ((uintptr_t)in % 16) == 0)
-    hipLaunchKernelGGL(k_conv_wgrad<8>, wg_grid, wg_block, 0, st, g, ncell, cin, cout, kpad, npad, in16, g16, work);
-  else if (cin % 4 == 0 && ((uintptr_t)in % 8) == 0)
-    hipLaunchKernelGGL(k_conv_wgrad<4>, wg_grid, wg_block, 0, st, g, ncell, cin, cout, kpad, npad, in16, g16, work);
-  else
-    hipLaunchKernelGGL(k_conv_wgrad<1>, wg_grid, wg_block, 0, st, g, ncell, cin, cout, kpad, npad, in16, g16, work);
+  auto go = [&](auto vec) {
+    constexpr int VEC = decltype(vec)::value;
+    TF_HIP(hipFuncSetAttribute((const void*)k_conv_wgrad<VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    hipLaunchKernelGGL(k_conv_wgrad<VEC>, wg_grid, wg_block, lds, st, g, ncell, chunk, cin, cout, kpad, npad, in16,
+                       g16, g32, work);
+    return 0;
+  };
+  int rc;
+  if (cin % 8 == 0 && ((uintptr_t)in % 16) == 0) rc = go(std::integral_constant<int, 8>());
+  else if (cin % 4 == 0 && ((uintptr_t)in % 8) == 0) rc = go(std::integral_constant<int, 4>());
+  else rc = go(std::integral_constant<int, 1>());
+  if (rc) return rc;
   const long len = (long)kpad * npad;
-  hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((len + 255) / 256)), dim3(256), 0, st, (int)blocks, len, work,
-                     dW);
-  float* bp = work + blocks * len;
-  if (db) {
-    hipLaunchKernelGGL(k_bias_partial, dim3((unsigned)blocks), dim3(256), 0, st, ncell, cout, g32, bp);
-    hipLaunchKernelGGL(k_sum_partials, dim3(1), dim3(256), 0, st, (int)blocks, (long)cout, bp, db);
-  }
+  hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((len + 32 + 63) / 64)), dim3(256), 0, st, (int)blocks, len, cout,
+                     work, dW, db);
   TF_PROF_WORK(tf::PROF_CONV, 2.0 * ncell * (dim == 3 ? 27 : 9) * cin * cout);
   TF_LAUNCH_CHECK("conv wgrad");
   return 0;
