@@ -17,6 +17,8 @@
 #include "tf_common.h"
 #include "transiflow_hip.h"
 
+#include <vector>
+
 using namespace tf;
 
 enum : int { MODE_RHS = 0, MODE_COUNT = 1, MODE_FILL = 2 };
@@ -26,7 +28,7 @@ struct tf_problem {
   int periodic[3];
   int dim, dof, buoy;
   int ncell, nrow, nblocks;
-  double* coord_d[3];
+  double* geom_d;     // axis tables of x, y, z (stencil.h), one after the other
   BcOp* ops_d;
   Physics ph;
   int* counts_d;      // nrow
@@ -36,26 +38,6 @@ struct tf_problem {
 };
 
 namespace {
-
-template <int DOF>
-__device__ __forceinline__ Cell<DOF> make_cell(const Grid& g, const double* state, int cell) {
-  Cell<DOF> c;
-  c.n[0] = g.n[0];
-  c.n[1] = g.n[1];
-  c.n[2] = g.n[2];
-  c.periodic[0] = g.periodic[0];
-  c.periodic[1] = g.periodic[1];
-  c.periodic[2] = g.periodic[2];
-  c.coord[0] = g.coord[0];
-  c.coord[1] = g.coord[1];
-  c.coord[2] = g.coord[2];
-  c.state = state;
-  c.idx[0] = cell % g.n[0];
-  const int rest = cell / g.n[0];
-  c.idx[1] = rest % g.n[1];
-  c.idx[2] = rest / g.n[1];
-  return c;
-}
 
 template <int DIM, int DOF, int BUOY, int D1, int MODE>
 __device__ __forceinline__ int row_work(const Cell<DOF>& c, const Physics& ph, int row, double* __restrict__ F,
@@ -89,16 +71,37 @@ __device__ __forceinline__ int dispatch_row(int d1, const Cell<DOF>& c, const Ph
   return 0;
 }
 
-// Inclusive scan of s[0..N) in LDS by all N threads of the block.
+// Inclusive scan of one value per thread over the N threads of the block (shuffles
+// within a wave, its totals through LDS: one barrier, where a scan in LDS took two for
+// every doubling and they were most of the kernels' time on small grids).
 template <int N>
-__device__ __forceinline__ void block_inclusive_scan(int* s, int t) {
+__device__ __forceinline__ int block_inclusive_scan(int v, int t) {
+  __shared__ int w[N / 64];
+  const int lane = t & 63, wave = t >> 6;
 #pragma unroll
-  for (int off = 1; off < N; off <<= 1) {
-    int v = t >= off ? s[t - off] : 0;
-    __syncthreads();
-    s[t] += v;
-    __syncthreads();
+  for (int off = 1; off < 64; off <<= 1) {
+    const int u = __shfl_up(v, off);
+    if (lane >= off) v += u;
   }
+  if (lane == 63) w[wave] = v;
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N / 64; ++i)
+    if (i < wave) v += w[i];
+  return v;
+}
+
+// The same over the rows of a workgroup, which thread t holds in equation order
+// (cnt is row lr's) and the CSR arrays in row order: returns the entries before row lr,
+// total those of the workgroup.  s is LDS of N entries.
+template <int N>
+__device__ __forceinline__ int scan_rows(int cnt, int lr, int t, int* s, int& total) {
+  s[lr] = cnt;
+  __syncthreads();
+  s[t] = block_inclusive_scan<N>(s[t], t);
+  __syncthreads();
+  total = s[N - 1];
+  return lr > 0 ? s[lr - 1] : 0;
 }
 
 template <int DIM, int DOF, int BUOY, int MODE>
@@ -108,7 +111,6 @@ __global__ __launch_bounds__(64 * DOF) void k_assemble(Grid g, Physics ph, const
                                                        int* __restrict__ row_ptr, int* __restrict__ col,
                                                        double* __restrict__ val, int ncell) {
   constexpr int NT = 64 * DOF;
-  __shared__ int s[NT];
   const int t = threadIdx.x;
   const int d1 = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lane = t & 63;
@@ -116,17 +118,15 @@ __global__ __launch_bounds__(64 * DOF) void k_assemble(Grid g, Physics ph, const
   const bool active = cell < ncell;
   const int row = cell * DOF + d1;
   const int lr = lane * DOF + d1;  // row index local to the workgroup
-  const Cell<DOF> c = make_cell<DOF>(g, state, active ? cell : 0);
+  const Cell<DOF> c(g, state, active ? cell : 0);
 
   if constexpr (MODE == MODE_RHS) {
     if (active) dispatch_row<DIM, DOF, BUOY, MODE>(d1, c, ph, row, F, nullptr, nullptr, 0);
   } else if constexpr (MODE == MODE_COUNT) {
     int cnt = active ? dispatch_row<DIM, DOF, BUOY, MODE>(d1, c, ph, row, nullptr, nullptr, nullptr, 0) : 0;
     if (active) counts[row] = cnt;
-    s[lr] = cnt;
-    __syncthreads();
-    block_inclusive_scan<NT>(s, t);
-    if (t == NT - 1) block_sums[blockIdx.x] = s[NT - 1];
+    const int sum = block_inclusive_scan<NT>(cnt, t);
+    if (t == NT - 1) block_sums[blockIdx.x] = sum;
   } else {
     // The workgroup's rows are contiguous in the CSR arrays: when its entries fit,
     // the rows are emitted into LDS and the segment is written out coalesced.  The
@@ -136,12 +136,10 @@ __global__ __launch_bounds__(64 * DOF) void k_assemble(Grid g, Physics ph, const
     constexpr int CAP = NT * (DIM == 3 ? 16 : 12);
     __shared__ int s_col[CAP];
     __shared__ double s_val[CAP];
-    s[lr] = active ? counts[row] : 0;
-    __syncthreads();
-    block_inclusive_scan<NT>(s, t);
+    __shared__ int s[NT];
+    int total;
     const int base = block_off[blockIdx.x];
-    const int total = s[NT - 1];
-    const int loc = lr > 0 ? s[lr - 1] : 0;
+    const int loc = scan_rows<NT>(active ? counts[row] : 0, lr, t, s, total);
     if (active) row_ptr[row] = base + loc;
     if (total <= CAP) {
       if (active) dispatch_row<DIM, DOF, BUOY, MODE>(d1, c, ph, row, nullptr, s_col, s_val, loc);
@@ -160,23 +158,20 @@ __global__ __launch_bounds__(64 * DOF) void k_assemble(Grid g, Physics ph, const
 // grand total to row_ptr[nrow] and to host-visible memory.
 __global__ __launch_bounds__(1024) void k_scan_blocks(const int* __restrict__ sums, int* __restrict__ off, int nb,
                                                       int* __restrict__ row_ptr_end, int* __restrict__ total_host) {
-  __shared__ int s[1024];
   const int t = threadIdx.x;
   const int chunk = (nb + 1023) / 1024;
   const int b0 = min(t * chunk, nb), b1 = min(b0 + chunk, nb);
   int acc = 0;
   for (int b = b0; b < b1; ++b) acc += sums[b];
-  s[t] = acc;
-  __syncthreads();
-  block_inclusive_scan<1024>(s, t);
-  int run = t > 0 ? s[t - 1] : 0;
+  const int incl = block_inclusive_scan<1024>(acc, t);
+  int run = incl - acc;
   for (int b = b0; b < b1; ++b) {
     off[b] = run;
     run += sums[b];
   }
   if (t == 1023) {
-    *row_ptr_end = s[1023];
-    if (total_host) *total_host = s[1023];
+    *row_ptr_end = incl;
+    if (total_host) *total_host = incl;
   }
 }
 
@@ -184,10 +179,10 @@ __global__ __launch_bounds__(1024) void k_scan_blocks(const int* __restrict__ su
 // u, v, w (staggered) and T, S (centred); pressure rows are empty.
 template <int DOF>
 __device__ __forceinline__ double mass_value(const Cell<DOF>& c, int d, int dim) {
-  if (d == 0) return c.hdiff(0, -1, 1) * c.diff(1, -1, 0) * c.diff(2, -1, 0);
-  if (d == 1) return c.hdiff(1, -1, 1) * c.diff(0, -1, 0) * c.diff(2, -1, 0);
-  if (d == 2 && dim == 3) return c.hdiff(2, -1, 1) * c.diff(1, -1, 0) * c.diff(0, -1, 0);
-  if (d == dim + 1 || d == dim + 2) return c.diff(0, -1, 0) * c.diff(1, -1, 0) * c.diff(2, -1, 0);
+  if (d == 0) return c.span(0) * c.width(1) * c.width(2);
+  if (d == 1) return c.span(1) * c.width(0) * c.width(2);
+  if (d == 2 && dim == 3) return c.span(2) * c.width(1) * c.width(0);
+  if (d == dim + 1 || d == dim + 2) return c.width(0) * c.width(1) * c.width(2);
   return 0.0;
 }
 
@@ -197,7 +192,6 @@ __global__ __launch_bounds__(64 * DOF) void k_mass(Grid g, int dim, int* __restr
                                                    int* __restrict__ row_ptr, int* __restrict__ col,
                                                    double* __restrict__ val, int ncell) {
   constexpr int NT = 64 * DOF;
-  __shared__ int s[NT];
   const int t = threadIdx.x;
   const int d1 = t >> 6;
   const int lane = t & 63;
@@ -205,20 +199,17 @@ __global__ __launch_bounds__(64 * DOF) void k_mass(Grid g, int dim, int* __restr
   const bool active = cell < ncell;
   const int row = cell * DOF + d1;
   const int lr = lane * DOF + d1;
-  const Cell<DOF> c = make_cell<DOF>(g, nullptr, active ? cell : 0);
+  const Cell<DOF> c(g, nullptr, active ? cell : 0);
   const double v = mass_value<DOF>(c, d1, dim);
   const int cnt = (active && fabs(v) > DROP) ? 1 : 0;
   if constexpr (MODE == MODE_COUNT) {
     if (active) counts[row] = cnt;
-    s[lr] = cnt;
-    __syncthreads();
-    block_inclusive_scan<NT>(s, t);
-    if (t == NT - 1) block_sums[blockIdx.x] = s[NT - 1];
+    const int sum = block_inclusive_scan<NT>(cnt, t);
+    if (t == NT - 1) block_sums[blockIdx.x] = sum;
   } else {
-    s[lr] = cnt;
-    __syncthreads();
-    block_inclusive_scan<NT>(s, t);
-    const int off = block_off[blockIdx.x] + (lr > 0 ? s[lr - 1] : 0);
+    __shared__ int s[NT];
+    int total;
+    const int off = block_off[blockIdx.x] + scan_rows<NT>(cnt, lr, t, s, total);
     if (active) {
       row_ptr[row] = off;
       if (cnt) {
@@ -234,7 +225,7 @@ Grid grid_of(const tf_problem* p) {
   for (int a = 0; a < 3; ++a) {
     g.n[a] = p->n[a];
     g.periodic[a] = p->periodic[a];
-    g.coord[a] = p->coord_d[a];
+    g.geom[a] = p->geom_d + G_FIELDS * (a > 0 ? p->n[0] + (a > 1 ? p->n[1] : 0) : 0);
   }
   return g;
 }
@@ -278,11 +269,11 @@ int scan_blocks(tf_problem* p, int* row_ptr, hipStream_t st) {
 // Device buffers of a problem; on failure the caller frees the partial set
 // (every pointer starts null, and hipFree/hipHostFree accept null).
 static int problem_alloc(tf_problem* p, const double* const host[3]) {
-  for (int a = 0; a < 3; ++a) {
-    const size_t bytes = sizeof(double) * (p->n[a] + 3);
-    TF_HIP(hipMalloc(&p->coord_d[a], bytes));
-    TF_HIP(tf::upload(p->coord_d[a], host[a], bytes));
-  }
+  std::vector<double> geom((size_t)G_FIELDS * (p->n[0] + p->n[1] + p->n[2]));
+  double* at = geom.data();
+  for (int a = 0; a < 3; at += G_FIELDS * (size_t)p->n[a++]) axis_geometry(host[a], p->n[a], at);
+  TF_HIP(hipMalloc(&p->geom_d, sizeof(double) * geom.size()));
+  TF_HIP(tf::upload(p->geom_d, geom.data(), sizeof(double) * geom.size()));
   TF_HIP(hipMalloc(&p->ops_d, sizeof(BcOp) * MAX_BC_OPS));
   TF_HIP(hipMalloc(&p->counts_d, sizeof(int) * p->nrow));
   TF_HIP(hipMalloc(&p->block_sums_d, sizeof(int) * p->nblocks));
@@ -336,7 +327,7 @@ int tf_problem_create(tf_problem** out, int nx, int ny, int nz, int dim, int dof
 
 int tf_problem_destroy(tf_problem* p) {
   if (!p) return 0;
-  for (int a = 0; a < 3; ++a) (void)hipFree(p->coord_d[a]);
+  (void)hipFree(p->geom_d);
   (void)hipFree(p->ops_d);
   (void)hipFree(p->counts_d);
   (void)hipFree(p->block_sums_d);

@@ -3,7 +3,7 @@
 // One row = equation d1 of one cell.  The row's atom is the dof x 3x3x3 block
 // A[d2][sx][sy][sz] of coefficients on variable d2 of the neighbour at slot
 // offset (sx-1, sy-1, sz-1) (transiflow/Discretization.py:71-102).  It is
-// built in registers from the coordinate vectors and the state, term by term,
+// built in registers from the axis tables and the state, term by term,
 // in the same floating-point order as the reference's whole-grid atom sums:
 //
 //   linear part     Discretization.py:229-317 (and the term builders :740-1084)
@@ -40,10 +40,46 @@ struct BcOp {
   double sign, fc, ac;
 };
 
+// Per index of an axis, the functions of its coordinates that the terms use (made once
+// per problem on the host, by the operations the reference applies in place, so that
+// the products they enter round as there): field f of index i is at geom[axis][f n + i].
+// Formed per cell they cost a dozen FP64 divisions a row, which with the checks and
+// 64-bit index products of every state access bounded the kernels: 64^3 cells of dof 4,
+// rhs 41 -> 19.5 us, count 55 -> 27, fill 88 -> 58 (150 MB written: 2.6 TB/s).
+enum : int {
+  G_D,    // x[i] - x[i-1]
+  G_H,    // (x[i+1] - x[i-1]) / 2
+  G_RD0,  // 1 / (x[i] - x[i-1])
+  G_RD1,  // 1 / (x[i+1] - x[i])
+  G_RH0,  // 1 / ((x[i] - x[i-2]) / 2)
+  G_RH1,  // 1 / ((x[i+1] - x[i-1]) / 2)
+  G_W0,   // 1/2 (x[i] - x[i-1]) / ((x[i+1] - x[i-1]) / 2)
+  G_W1,   // 1/2 (x[i+1] - x[i]) / ((x[i+1] - x[i-1]) / 2)
+  G_FIELDS
+};
+
+// the table of an axis of n cells from its coordinate vector (n+3 entries, negative
+// indices wrap as in Python)
+inline void axis_geometry(const double* x, int n, double* t) {
+  auto X = [&](int i) { return x[i < 0 ? i + n + 3 : i]; };
+  for (int i = 0; i < n; ++i) {
+    const double d0 = X(i) - X(i - 1), d1 = X(i + 1) - X(i);
+    const double h0 = (X(i) - X(i - 2)) / 2.0, h1 = (X(i + 1) - X(i - 1)) / 2.0;
+    t[G_D * n + i] = d0;
+    t[G_H * n + i] = h1;
+    t[G_RD0 * n + i] = 1.0 / d0;
+    t[G_RD1 * n + i] = 1.0 / d1;
+    t[G_RH0 * n + i] = 1.0 / h0;
+    t[G_RH1 * n + i] = 1.0 / h1;
+    t[G_W0 * n + i] = 1.0 / 2.0 * d0 / h1;
+    t[G_W1 * n + i] = 1.0 / 2.0 * d1 / h1;
+  }
+}
+
 struct Grid {
   int n[3];
   int periodic[3];
-  const double* coord[3];  // device coordinate vectors, length n+3 each
+  const double* geom[3];  // device tables, G_FIELDS n entries each
 };
 
 struct Physics {
@@ -85,42 +121,56 @@ template <int DOF>
 struct Cell {
   int idx[3];
   int n[3];
-  int periodic[3];
-  const double* coord[3];
-  const double* __restrict__ state;
+  const double* __restrict__ geom[3];
+  const double* __restrict__ state;  // of this cell
+  // neighbour s (0, 1, 2: before, own, after) along each axis: the offset of its state
+  // from this cell's, whether it exists, and whether the axis's velocity there is not a
+  // wall's (see P)
+  long off[3][3];
+  bool ok[3][3], open[3][3];
 
-  // coordinate vector entry idx+off with Python negative-index wrap
-  __device__ __forceinline__ double X(int axis, int off) const {
-    int t = idx[axis] + off;
-    if (t < 0) t += n[axis] + 3;
-    return coord[axis][t];
+  __device__ __forceinline__ Cell(const Grid& g, const double* st, int cell) {
+    idx[0] = cell % g.n[0];
+    const int rest = cell / g.n[0];
+    idx[1] = rest % g.n[1];
+    idx[2] = rest / g.n[1];
+    state = st + (size_t)cell * DOF;
+    long stride = DOF;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {
+      n[a] = g.n[a];
+      geom[a] = g.geom[a];
+      const bool per = g.periodic[a] != 0;
+      const bool first = idx[a] == 0, last = idx[a] == n[a] - 1;
+      off[a][0] = first ? (per ? (n[a] - 1) * stride : 0) : -stride;
+      off[a][1] = 0;
+      off[a][2] = last ? (per ? -(n[a] - 1) * stride : 0) : stride;
+      ok[a][0] = per || !first;
+      ok[a][1] = true;
+      ok[a][2] = per || !last;
+      open[a][0] = true;
+      open[a][1] = per || !last;
+      open[a][2] = per || idx[a] != n[a] - 2;
+      stride *= n[a];
+    }
   }
-  __device__ __forceinline__ double diff(int axis, int lo, int hi) const {
-    return X(axis, hi) - X(axis, lo);
-  }
-  __device__ __forceinline__ double hdiff(int axis, int lo, int hi) const {
-    return (X(axis, hi) - X(axis, lo)) / 2.0;
-  }
+
+  __device__ __forceinline__ double G(int axis, int field) const { return geom[axis][field * n[axis] + idx[axis]]; }
+  __device__ __forceinline__ double width(int axis) const { return G(axis, G_D); }
+  __device__ __forceinline__ double span(int axis) const { return G(axis, G_H); }
 
   // Padded state (utils.create_padded_state_mtx, utils.py:62-133): component
   // c of the cell at offset (rx, ry, rz).  Ghosts are zero unless the axis is
   // periodic; on a non-periodic axis the wall-normal velocity of the last
-  // interior cell is zero.
+  // interior cell is zero.  (An entry that is zero is loaded from this cell instead: no
+  // branch around the load.)
   __device__ __forceinline__ double P(int c, int rx, int ry, int rz) const {
-    int p[3] = {idx[0] + 1 + rx, idx[1] + 1 + ry, idx[2] + 1 + rz};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-      if (p[a] == 0) {
-        if (!periodic[a]) return 0.0;
-        p[a] = n[a];
-      } else if (p[a] == n[a] + 1) {
-        if (!periodic[a]) return 0.0;
-        p[a] = 1;
-      }
-    }
-    if (c < 3 && !periodic[c < 3 ? c : 0] && p[c < 3 ? c : 0] == n[c < 3 ? c : 0]) return 0.0;
-    size_t cell = ((size_t)(p[2] - 1) * n[1] + (p[1] - 1)) * n[0] + (p[0] - 1);
-    return state[cell * DOF + c];
+    const int r[3] = {rx + 1, ry + 1, rz + 1};
+    bool v = ok[0][r[0]] && ok[1][r[1]] && ok[2][r[2]];
+    if (c < 3) v = v && open[c < 3 ? c : 0][r[c < 3 ? c : 0]];
+    const long o = off[0][r[0]] + off[1][r[1]] + off[2][r[2]];
+    const double x = state[(v ? o : 0) + c];
+    return v ? x : 0.0;
   }
 };
 
@@ -141,10 +191,9 @@ __device__ __forceinline__ void add_line(double* acc, double a0, double a1, doub
 template <int R, int DOF>
 __device__ __forceinline__ void face_lap(const Cell<DOF>& c, double& a0, double& a1, double& a2) {
   constexpr int r0 = Role<R>::r0, r1 = Role<R>::r1, r2 = Role<R>::r2;
-  double dx = c.diff(r0, -1, 0), dxp1 = c.diff(r0, 0, 1);
-  double dy = c.diff(r1, -1, 0), dz = c.diff(r2, -1, 0);
-  a0 = 1.0 / dx * dy * dz;
-  a2 = 1.0 / dxp1 * dy * dz;
+  const double dy = c.width(r1), dz = c.width(r2);
+  a0 = c.G(r0, G_RD0) * dy * dz;
+  a2 = c.G(r0, G_RD1) * dy * dz;
   a1 = -a0 - a2;
 }
 
@@ -152,10 +201,9 @@ __device__ __forceinline__ void face_lap(const Cell<DOF>& c, double& a0, double&
 template <int R, int DOF>
 __device__ __forceinline__ void centre_lap_y(const Cell<DOF>& c, double& a0, double& a1, double& a2) {
   constexpr int r0 = Role<R>::r0, r1 = Role<R>::r1, r2 = Role<R>::r2;
-  double dy = c.hdiff(r1, -2, 0), dyp1 = c.hdiff(r1, -1, 1);
-  double dx = c.hdiff(r0, -1, 1), dz = c.diff(r2, -1, 0);
-  a0 = 1.0 / dy * dx * dz;
-  a2 = 1.0 / dyp1 * dx * dz;
+  const double dx = c.span(r0), dz = c.width(r2);
+  a0 = c.G(r1, G_RH0) * dx * dz;
+  a2 = c.G(r1, G_RH1) * dx * dz;
   a1 = -a0 - a2;
 }
 
@@ -163,10 +211,9 @@ __device__ __forceinline__ void centre_lap_y(const Cell<DOF>& c, double& a0, dou
 template <int R, int DOF>
 __device__ __forceinline__ void centre_lap_z(const Cell<DOF>& c, double& a0, double& a1, double& a2) {
   constexpr int r0 = Role<R>::r0, r1 = Role<R>::r1, r2 = Role<R>::r2;
-  double dz = c.hdiff(r2, -2, 0), dzp1 = c.hdiff(r2, -1, 1);
-  double dx = c.hdiff(r0, -1, 1), dy = c.diff(r1, -1, 0);
-  a0 = 1.0 / dz * dx * dy;
-  a2 = 1.0 / dzp1 * dx * dy;
+  const double dx = c.span(r0), dy = c.width(r1);
+  a0 = c.G(r2, G_RH0) * dx * dy;
+  a2 = c.G(r2, G_RH1) * dx * dy;
   a1 = -a0 - a2;
 }
 
@@ -174,23 +221,22 @@ __device__ __forceinline__ void centre_lap_z(const Cell<DOF>& c, double& a0, dou
 template <int R, int DOF>
 __device__ __forceinline__ void scalar_lap(const Cell<DOF>& c, double& a0, double& a1, double& a2) {
   constexpr int r0 = Role<R>::r0, r1 = Role<R>::r1, r2 = Role<R>::r2;
-  double dx = c.hdiff(r0, -2, 0), dxp1 = c.hdiff(r0, -1, 1);
-  double dy = c.diff(r1, -1, 0), dz = c.diff(r2, -1, 0);
-  a0 = 1.0 / dx * dy * dz;
-  a2 = 1.0 / dxp1 * dy * dz;
+  const double dy = c.width(r1), dz = c.width(r2);
+  a0 = c.G(r0, G_RH0) * dy * dz;
+  a2 = c.G(r0, G_RH1) * dy * dz;
   a1 = -a0 - a2;
 }
 
 // dy*dz of _forward_u_x / _backward_u_x for role R
 template <int R, int DOF>
 __device__ __forceinline__ double face_area(const Cell<DOF>& c) {
-  return c.diff(Role<R>::r1, -1, 0) * c.diff(Role<R>::r2, -1, 0);
+  return c.width(Role<R>::r1) * c.width(Role<R>::r2);
 }
 
 // dx*dy*dz/2 of _forward_average_x / _backward_average_x for role R
 template <int R, int DOF>
 __device__ __forceinline__ double half_volume(const Cell<DOF>& c) {
-  return c.hdiff(Role<R>::r0, -1, 1) * c.diff(Role<R>::r1, -1, 0) * c.diff(Role<R>::r2, -1, 0) / 2.0;
+  return c.span(Role<R>::r0) * c.width(Role<R>::r1) * c.width(Role<R>::r2) / 2.0;
 }
 
 // Velocity Laplacian terms of component V along axis AX (V's own axis ->
@@ -347,12 +393,10 @@ template <int D1, int A, int B, int DOF>
 __device__ __forceinline__ void cross_adv(const Cell<DOF>& c, double* Fn, double* Jn) {
   if constexpr (D1 == B) {
     constexpr int third = 3 - A - B;
-    double area = c.hdiff(B, -1, 1) * c.diff(third, -1, 0);
+    double area = c.span(B) * c.width(third);
     double a1 = area, a0 = -area;
     // _weighted_average along B at this cell (Discretization.py:1212-1221)
-    double dxb = (c.X(B, 1) - c.X(B, -1)) / 2.0;
-    double w0 = 1.0 / 2.0 * (c.X(B, 0) - c.X(B, -1)) / dxb;
-    double w1 = 1.0 / 2.0 * (c.X(B, 1) - c.X(B, 0)) / dxb;
+    double w0 = c.G(B, G_W0), w1 = c.G(B, G_W1);
     // velocity A weighted-averaged to the B location, on the lower and upper A face
     double wav_lo = w0 * Pe2<A, B>(c, A, -1, 0) + w1 * Pe2<A, B>(c, A, -1, 1);
     double wav_hi = w0 * Pe2<A, B>(c, A, 0, 0) + w1 * Pe2<A, B>(c, A, 0, 1);
