@@ -184,3 +184,54 @@ def test_continuation_3d_multigrid_matches_plane_factor(hip):
           flush=True)
     numpy.testing.assert_allclose(musm, musl, rtol=1e-9)
     assert abs(mm - 300) <= 1e-3 and err <= 1e-8
+
+
+@pytest.mark.parametrize('nx,dof,ny,nz', [(5, 1, 3, 3), (16, 4, 3, 2), (65, 1, 2, 3), (64, 4, 2, 2), (257, 1, 3, 2),
+                                          (69, 4, 3, 1)])
+@pytest.mark.parametrize('single', [False, True])
+def test_line_ilu_schur_sizes(hip, nx, dof, ny, nz, single):
+    """The pivots' Schur updates at line lengths around the row tile (16), the wave and
+    the block's columns (256), with columns of 11 couplings into one line (more than a
+    thread holds).  Rows sum to less than half their diagonal, so the pivots are as well
+    conditioned as the matrix and the inverses' error is m units of rounding times a
+    constant below ten: 280 * 1.1e-16 * 10 < 1e-12, 280 * 6e-8 * 10 < 2e-4."""
+    import types
+
+    import torch
+    from transiflow_amd.solver import LineILU
+    from transiflow_amd.vector import DeviceCsrMatrix
+    rng = numpy.random.default_rng(nx + dof)
+    m, N = nx * dof, ny * nz
+    I, J, V = [], [], []
+
+    def add(i, j):
+        I.extend(i)
+        J.extend(j)
+        V.extend(rng.uniform(-1, 1, len(i)) * 0.03)
+
+    for line in range(N):
+        i = line * m + numpy.arange(m)
+        for off in (-3, -1, 1, 2):
+            add(i, line * m + (numpy.arange(m) + off) % m)
+        for dj, dk in ((-1, 0), (1, 0), (0, -1), (0, 1), (-1, 1), (1, -1)):
+            j, k = line % ny + dj, line // ny + dk
+            if 0 <= j < ny and 0 <= k < nz:
+                add(i, (j + ny * k) * m + rng.permutation(m))
+                if (dj, dk) in ((-1, 0), (1, 0)) and min(j, line % ny) % 2 == 0:
+                    hot = min(m, 10)
+                    add(i[:hot], [(j + ny * k) * m + m - 1] * hot)
+    A = sparse.csr_matrix((V, (I, J)), shape=(N * m, N * m)) + sparse.identity(N * m)
+    A = sparse.csr_matrix(A)
+    A.sort_indices()
+    t = lambda v, dt: torch.from_numpy(numpy.ascontiguousarray(v)).to(dt).cuda()
+    M = DeviceCsrMatrix(t(A.indptr, torch.int32), t(A.indices, torch.int32), t(A.data, torch.float64), N * m)
+    P = LineILU(types.SimpleNamespace(nx=nx, ny=ny, nz=nz, dof=dof), single)
+    P.refactor(M, -1)
+    r = rng.uniform(-1, 1, N * m)
+    z = linegrid.dilu_apply(A, r, nx, ny, nz, dof)
+    rt = t(r, torch.float32 if single else torch.float64)
+    out = torch.empty_like(rt)
+    (P.apply32 if single else P.apply)(rt, out)
+    err = numpy.max(numpy.abs(out.double().cpu().numpy() - z)) / numpy.max(numpy.abs(z))
+    assert P.perturbed == 0
+    assert err <= (2e-4 if single else 1e-12), err
