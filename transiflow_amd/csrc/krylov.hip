@@ -15,6 +15,7 @@
 #include "tf_common.h"
 
 #include <type_traits>
+#include <utility>
 
 namespace {
 
@@ -55,20 +56,8 @@ int md_blocks(long n) {
 // wavefront shuffles and then across the block's waves in a fixed order.
 // VEC: 16-byte loads over entries [b0, b1) counted in vectors (rows of V and w
 // 16-byte aligned, n a multiple of the vector width); else one entry per lane.
-// A grid with gridDim.y == 2 does the same for a second system: blockIdx.y 1
-// takes V1, w1 and partial1 (the other kernels below follow the same rule).
 template <typename T, bool VEC>
-__global__ __launch_bounds__(MD_THREADS) void k_multidot_partial(int n, int k, const T* __restrict__ V, long ldv,
-                                                                 const T* __restrict__ w,
-                                                                 double* __restrict__ partial,
-                                                                 const T* __restrict__ V1 = nullptr,
-                                                                 const T* __restrict__ w1 = nullptr,
-                                                                 double* __restrict__ partial1 = nullptr) {
-  if (blockIdx.y) {
-    V = V1;
-    w = w1;
-    partial = partial1;
-  }
+__device__ __forceinline__ void dot_body(int n, int k, const T* V, long ldv, const T* w, double* partial) {
   using Acc = typename std::conditional<sizeof(T) == 8, double, float>::type;
   using VT = typename Vec16<T>::type;
   constexpr int VN = VEC ? Vec16<T>::N : 1;
@@ -118,6 +107,24 @@ __global__ __launch_bounds__(MD_THREADS) void k_multidot_partial(int n, int k, c
   }
 }
 
+// dot_body as a launch.  A grid with gridDim.y == 2 does the same for a second
+// system: blockIdx.y 1 takes V1, w1 and partial1 (the other kernels below follow the
+// same rule).
+template <typename T, bool VEC>
+__global__ __launch_bounds__(MD_THREADS) void k_multidot_partial(int n, int k, const T* __restrict__ V, long ldv,
+                                                                 const T* __restrict__ w,
+                                                                 double* __restrict__ partial,
+                                                                 const T* __restrict__ V1 = nullptr,
+                                                                 const T* __restrict__ w1 = nullptr,
+                                                                 double* __restrict__ partial1 = nullptr) {
+  if (blockIdx.y) {
+    V = V1;
+    w = w1;
+    partial = partial1;
+  }
+  dot_body<T, VEC>(n, k, V, ldv, w, partial);
+}
+
 // h[i] (+)= sum_b partial[i][b]; one workgroup per i, wavefront reductions.
 __global__ __launch_bounds__(MD_THREADS) void k_multidot_final(int k, int nb, const double* __restrict__ partial,
                                                                double* __restrict__ h, int accumulate,
@@ -143,14 +150,13 @@ __global__ __launch_bounds__(MD_THREADS) void k_multidot_final(int k, int nb, co
 
 // w += sum_i c[i] V[i] with the coefficients c (sign applied) in LDS: accumulation
 // in FP64 in the order i = 0, 1, ...; VEC: 16-byte loads, four basis vectors' loads
-// issued together.  Grid-stride over the entries.
+// issued together.  Units (vectors or entries) e0, e0 + step, ... below e1.
 template <typename T, bool VEC>
-__device__ __forceinline__ void axpy_body(int n, int k, const T* __restrict__ V, long ldv, const double* c,
-                                          T* __restrict__ w) {
+__device__ __forceinline__ void axpy_body(int e0, int e1, int step, int k, const T* V, long ldv, const double* c,
+                                          T* w) {
   using VT = typename Vec16<T>::type;
   constexpr int VN = VEC ? Vec16<T>::N : 1;
-  const int units = n / VN;
-  for (int e = blockIdx.x * blockDim.x + threadIdx.x; e < units; e += gridDim.x * blockDim.x) {
+  for (int e = e0; e < e1; e += step) {
     if constexpr (VEC) {
       VT wv = reinterpret_cast<const VT*>(w)[e];
       double acc[VN];
@@ -197,7 +203,8 @@ __global__ __launch_bounds__(256) void k_multiaxpy(int n, int k, const T* __rest
   __shared__ double c[MAX_BASIS];
   for (int i = threadIdx.x; i < k; i += blockDim.x) c[i] = sign * coef[i];
   __syncthreads();
-  axpy_body<T, VEC>(n, k, V, ldv, c, w);
+  axpy_body<T, VEC>(blockIdx.x * blockDim.x + threadIdx.x, n / (VEC ? Vec16<T>::N : 1), gridDim.x * blockDim.x, k, V,
+                    ldv, c, w);
 }
 
 // ---- CGS2 with the block sums reduced where they are consumed --------------------
@@ -221,20 +228,29 @@ __device__ __forceinline__ void fin_sums(int k, int nb, const double* __restrict
   __syncthreads();
 }
 
-// c = the sums of partial (k x nb); block 0: hout[i] = c[i] (add: hout[i] += c[i]);
-// then w -= sum_i c[i] V[i].  blockIdx.y 1 takes the second system.
+// One Gram-Schmidt pass: c = the sums of partial (k x nb); block 0: hout[i] = c[i]
+// (add: hout[i] += c[i]); w -= sum_i c[i] V[i]; then the block sums of the next
+// reduction, V^T w (self: w . w), into next.  A block updates the entries it then sums
+// (dot_body's chunk, and each thread the ones it reads), so the next reduction needs no
+// launch of its own: a step of the 64 x 64 grid is six dependent launches of 4 us
+// instead of eight, with the second reading of V from the L2.  blockIdx.y 1 takes the
+// second system.
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256) void k_multiaxpy_fin(int n, int k, int nb, const T* __restrict__ V, long ldv,
-                                                       const double* __restrict__ partial, double* __restrict__ hout,
-                                                       int add, T* __restrict__ w, const T* __restrict__ V1,
-                                                       const double* __restrict__ partial1,
-                                                       double* __restrict__ hout1, T* __restrict__ w1) {
+__global__ __launch_bounds__(MD_THREADS) void k_gram_schmidt(int n, int k, const T* V, long ldv,
+                                                             const double* __restrict__ partial,
+                                                             double* __restrict__ hout, int add, T* w, int self,
+                                                             double* __restrict__ next, const T* V1,
+                                                             const double* __restrict__ partial1,
+                                                             double* __restrict__ hout1, T* w1,
+                                                             double* __restrict__ next1) {
   if (blockIdx.y) {
     V = V1;
     partial = partial1;
     hout = hout1;
     w = w1;
+    next = next1;
   }
+  const int nb = gridDim.x;
   __shared__ double sp[FIN_LDS];
   __shared__ double c[MAX_BASIS];
   fin_sums(k, nb, partial, sp, c);
@@ -243,7 +259,12 @@ __global__ __launch_bounds__(256) void k_multiaxpy_fin(int n, int k, int nb, con
   __syncthreads();
   for (int i = threadIdx.x; i < k; i += blockDim.x) c[i] = -c[i];
   __syncthreads();
-  axpy_body<T, VEC>(n, k, V, ldv, c, w);
+  const int units = n / (VEC ? Vec16<T>::N : 1);
+  const int chunk = (units + nb - 1) / nb;
+  const int b0 = blockIdx.x * chunk, b1 = min(units, b0 + chunk);
+  axpy_body<T, VEC>(b0 + threadIdx.x, b1, MD_THREADS, k, V, ldv, c, w);
+  if (self) dot_body<T, VEC>(n, 1, w, (long)n, w, next);
+  else dot_body<T, VEC>(n, k, V, ldv, w, next);
 }
 
 // nrm = sqrt(sum of partial[0..nb)) (block 0 stores it in h[k]), out = w / nrm.
@@ -516,11 +537,11 @@ __global__ void k_add_pair(int k, double* h0, const double* y0, double* h1, cons
 // in the same launches (blockIdx.y picks the system; the second system's pointers
 // are unused for one): h = V^T w, w -= V h, y = V^T w, w -= V y, h += y,
 // h[j+1] = |w|, V[j+1] = w / |w|.  With the partials in LDS reach (k nb <= FIN_LDS)
-// the sums are reduced by the consuming kernels (k_multiaxpy_fin, k_scale_fin:
-// five launches); else by separate kernels (k_multidot_final, k_add_pair,
-// k_norm_final: eight).  The choice depends on n and j only, so one system and
+// the sums are reduced by the consuming kernels (k_gram_schmidt, k_scale_fin:
+// four launches); else by separate kernels (k_multidot_final, k_add_pair,
+// k_norm_final: ten).  The choice depends on n and j only, so one system and
 // two systems take the same arithmetic.  hh0, hh1 (pinned host memory, or null):
-// on the five-launch path the last launch also writes each column h[0..j+1] there
+// on the four-launch path the last launch also writes each column h[0..j+1] there
 // (*to_host = 1); otherwise *to_host = 0 and the caller copies it.
 template <typename T>
 int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, double* work0, double* work1,
@@ -543,25 +564,43 @@ int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, dou
   const bool fused = (long)k * nb <= FIN_LDS;
   const dim3 md(nb, nsys), blk(MD_THREADS), fin(k, nsys);
   const dim3 ew(grid_for(vec ? n / Vec16<T>::N : n), nsys);
+  auto dots = [&](int kk, const T* A0, const T* A1) {
+    if (vec)
+      hipLaunchKernelGGL((k_multidot_partial<T, true>), md, blk, 0, st, n, kk, A0, (long)n, (const T*)w0, work0, A1,
+                         (const T*)w1, work1);
+    else
+      hipLaunchKernelGGL((k_multidot_partial<T, false>), md, blk, 0, st, n, kk, A0, (long)n, (const T*)w0, work0, A1,
+                         (const T*)w1, work1);
+  };
+  if (fused) {
+    // the partial sums alternate between two halves of work: a pass reads one while
+    // other blocks write the other
+    double *in0 = work0, *in1 = work1, *out0 = work0 + FIN_LDS, *out1 = work1 + FIN_LDS;
+    dots(k, V0, V1);
+    for (int pass = 0; pass < 2; ++pass) {
+      if (vec)
+        hipLaunchKernelGGL((k_gram_schmidt<T, true>), md, blk, 0, st, n, k, V0, (long)n, (const double*)in0, h0, pass,
+                           w0, pass, out0, V1, (const double*)in1, h1, w1, out1);
+      else
+        hipLaunchKernelGGL((k_gram_schmidt<T, false>), md, blk, 0, st, n, k, V0, (long)n, (const double*)in0, h0,
+                           pass, w0, pass, out0, V1, (const double*)in1, h1, w1, out1);
+      std::swap(in0, out0);
+      std::swap(in1, out1);
+    }
+    if (vec)
+      hipLaunchKernelGGL((k_scale_fin<T, true>), ew, dim3(256), 0, st, n, nb, k, (const double*)in0, h0, hh0,
+                         (const T*)w0, v0, (const double*)in1, h1, hh1, (const T*)w1, v1);
+    else
+      hipLaunchKernelGGL((k_scale_fin<T, false>), ew, dim3(256), 0, st, n, nb, k, (const double*)in0, h0, hh0,
+                         (const T*)w0, v0, (const double*)in1, h1, hh1, (const T*)w1, v1);
+    TF_LAUNCH_CHECK("cgs2");
+    *to_host = hh0 != nullptr && hh1 != nullptr;
+    return 0;
+  }
   for (int pass = 0; pass < 2; ++pass) {
     double* c0 = pass ? y0 : h0;
     double* c1 = pass ? y1 : h1;
-    if (vec)
-      hipLaunchKernelGGL((k_multidot_partial<T, true>), md, blk, 0, st, n, k, V0, (long)n, (const T*)w0, work0, V1,
-                         (const T*)w1, work1);
-    else
-      hipLaunchKernelGGL((k_multidot_partial<T, false>), md, blk, 0, st, n, k, V0, (long)n, (const T*)w0, work0, V1,
-                         (const T*)w1, work1);
-    if (fused) {
-      // pass 0: h = sums; pass 1: h += sums (y is not needed further)
-      if (vec)
-        hipLaunchKernelGGL((k_multiaxpy_fin<T, true>), ew, dim3(256), 0, st, n, k, nb, V0, (long)n,
-                           (const double*)work0, h0, pass, w0, V1, (const double*)work1, h1, w1);
-      else
-        hipLaunchKernelGGL((k_multiaxpy_fin<T, false>), ew, dim3(256), 0, st, n, k, nb, V0, (long)n,
-                           (const double*)work0, h0, pass, w0, V1, (const double*)work1, h1, w1);
-      continue;
-    }
+    dots(k, V0, V1);
     hipLaunchKernelGGL(k_multidot_final, fin, blk, 0, st, k, nb, (const double*)work0, c0, 0, (const double*)work1,
                        c1);
     if (vec)
@@ -571,25 +610,9 @@ int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, dou
       hipLaunchKernelGGL((k_multiaxpy<T, false>), ew, dim3(256), 0, st, n, k, V0, (long)n, (const double*)c0, w0,
                          -1.0, V1, (const double*)c1, w1);
   }
-  if (!fused) hipLaunchKernelGGL(k_add_pair, dim3(nsys), dim3(64), 0, st, k, h0, (const double*)y0, h1, (const double*)y1);
+  hipLaunchKernelGGL(k_add_pair, dim3(nsys), dim3(64), 0, st, k, h0, (const double*)y0, h1, (const double*)y1);
   // |w| into h[j+1], V[j+1] = w / |w|
-  if (vec)
-    hipLaunchKernelGGL((k_multidot_partial<T, true>), md, blk, 0, st, n, 1, (const T*)w0, (long)n, (const T*)w0,
-                       work0, (const T*)w1, (const T*)w1, work1);
-  else
-    hipLaunchKernelGGL((k_multidot_partial<T, false>), md, blk, 0, st, n, 1, (const T*)w0, (long)n, (const T*)w0,
-                       work0, (const T*)w1, (const T*)w1, work1);
-  if (fused) {
-    if (vec)
-      hipLaunchKernelGGL((k_scale_fin<T, true>), ew, dim3(256), 0, st, n, nb, k, (const double*)work0, h0, hh0,
-                         (const T*)w0, v0, (const double*)work1, h1, hh1, (const T*)w1, v1);
-    else
-      hipLaunchKernelGGL((k_scale_fin<T, false>), ew, dim3(256), 0, st, n, nb, k, (const double*)work0, h0, hh0,
-                         (const T*)w0, v0, (const double*)work1, h1, hh1, (const T*)w1, v1);
-    TF_LAUNCH_CHECK("cgs2");
-    *to_host = hh0 != nullptr && hh1 != nullptr;
-    return 0;
-  }
+  dots(1, w0, w1);
   hipLaunchKernelGGL(k_norm_final, dim3(1, nsys), blk, 0, st, nb, (const double*)work0, h0 + k, (const double*)work1,
                      h1 + k);
   if (vec)
