@@ -114,3 +114,31 @@ def test_multidot_deterministic(hip):
         _lib.call('tf_multidot_f32', n, k, ptr(V), n, ptr(w), ptr(work), ptr(h), 0, stream())
         hs.append(h.cpu().numpy())
     assert all(numpy.array_equal(hs[0], x) for x in hs[1:])
+
+
+@pytest.mark.parametrize('shape', [(12, 12), (9, 14), (14, 9), (5, 7), (4, 3, 3)])
+@pytest.mark.parametrize('restart', [3, 30])
+def test_replayed_iterations_match_eager(hip, shape, restart):
+    """Iterations of a lagged line factor replayed whole (apply and Arnoldi step), issued
+    one by one and captured on their third use, in cycles of 3 (restarts) and 30, one
+    system and two, against the launches without graphs: the same bits at every solve,
+    with lines along x and y and sizes with and without 16-byte columns."""
+    got = {}
+    for graphs in (False, True):
+        itf = hip.Interface({'Reynolds Number': 300,
+                             'HIP Solver': {'Preconditioner': 'line', 'Precision': 'mixed', 'Reuse Limit': 1000,
+                                            'Restart': restart, 'Apply Graph': graphs, 'Step Graphs': graphs}},
+                            *shape)
+        rng = numpy.random.default_rng(5)
+        vec = lambda s: itf.vector_from_array(rng.uniform(-1, 1, itf.n) * s)
+        itf.solve(itf.jacobian(vec(0.0)), vec(1.0))
+        out = []
+        for i in range(5):
+            J = itf.jacobian(vec(0.05))
+            out += [itf.array_from_vector(v) for v in itf.solve_pair(J, vec(1.0), vec(1e-3))]
+            out.append(itf.array_from_vector(itf.solve(J, vec(1.0))))
+        got[graphs] = (out, [e[0] for e in itf.solver.log])
+    assert got[True][1] == got[False][1]
+    assert max(got[True][1]) > 3
+    for a, b in zip(got[True][0], got[False][0]):
+        assert numpy.isfinite(a).all() and numpy.array_equal(a, b)

@@ -38,6 +38,7 @@
 
 #include <algorithm>
 #include <array>
+#include <atomic>
 #include <cstdint>
 #include <type_traits>
 #include <vector>
@@ -547,7 +548,8 @@ __device__ __forceinline__ void group_rows(int m, int G, int (&rr)[R], bool (&li
   }
 }
 
-// Every vector argument below holds NC columns at stride cs.
+// Every vector argument below holds NC columns: r and x, which may be the caller's, at
+// strides rs and xs, the others at stride cs.
 
 // rw[k] -= P1 rw[e1] + P2 rw[e2] (terms with a missing neighbour dropped) for a batch of kept lines
 template <typename B, typename V, int NC, int R>
@@ -594,7 +596,7 @@ template <typename B, typename V, int NC, int R>
 __global__ __launch_bounds__(256) void k_bwd_t(int m, int G, int vec, const int* __restrict__ e_line,
                                                const int* __restrict__ a_line, const int* __restrict__ b_line,
                                                B Lb, B Ub, const V* __restrict__ rw, const V* __restrict__ x,
-                                               V* __restrict__ tbuf, long cs) {
+                                               V* __restrict__ tbuf, long cs, long xs) {
   const int bi = blockIdx.y;
   const int g = threadIdx.x % G;
   int rr[R];
@@ -608,14 +610,14 @@ __global__ __launch_bounds__(256) void k_bwd_t(int m, int G, int vec, const int*
 #pragma unroll
     for (int j = 0; j < NC; ++j) acc[i][j] = 0.0;
   if (a >= 0) {
-    row_dot<NC, R>(Lb, bi, rr, x + (long)a * m, cs, m, g, G, vec, d);
+    row_dot<NC, R>(Lb, bi, rr, x + (long)a * m, xs, m, g, G, vec, d);
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
       for (int j = 0; j < NC; ++j) acc[i][j] += d[i][j];
   }
   if (bb >= 0) {
-    row_dot<NC, R>(Ub, bi, rr, x + (long)bb * m, cs, m, g, G, vec, d);
+    row_dot<NC, R>(Ub, bi, rr, x + (long)bb * m, xs, m, g, G, vec, d);
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
@@ -632,7 +634,7 @@ __global__ __launch_bounds__(256) void k_bwd_t(int m, int G, int vec, const int*
         }
 }
 
-// Level 0: t[e] = rw[e] - L_e x[a] - U_e x[b] with the sparse couplings.  Thread per
+// Level 0: t[e] = r[e] - L_e x[a] - U_e x[b] with the sparse couplings.  Thread per
 // row; the row's couplings are loaded once for all columns, each column's sum keeps
 // the coupling order.
 template <typename V, int NC>
@@ -640,12 +642,12 @@ __global__ __launch_bounds__(256) void k_bwd_t_sparse(int m, const int* __restri
                                                       const int* __restrict__ a_line, const int* __restrict__ b_line,
                                                       const Cpl* __restrict__ Lr, const int* __restrict__ nLr,
                                                       const Cpl* __restrict__ Ur, const int* __restrict__ nUr,
-                                                      const V* __restrict__ rw, const V* __restrict__ x,
-                                                      V* __restrict__ tbuf, long cs) {
+                                                      const V* __restrict__ r, long rs, const V* __restrict__ x,
+                                                      long xs, V* __restrict__ tbuf, long cs) {
   const int bi = blockIdx.y;
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= m) return;
-  const long row = (long)e_line[bi] * m + r;
+  const int loc = blockIdx.x * blockDim.x + threadIdx.x;
+  if (loc >= m) return;
+  const long row = (long)e_line[bi] * m + loc;
   const int a = a_line[bi], bb = b_line[bi];
   const int nl = a >= 0 ? nLr[row] : 0, nu = bb >= 0 ? nUr[row] : 0;
   Cpl lc[KC], uc[KC];
@@ -656,7 +658,7 @@ __global__ __launch_bounds__(256) void k_bwd_t_sparse(int m, const int* __restri
   }
 #pragma unroll
   for (int j = 0; j < NC; ++j) {
-    const V* xj = x + j * cs;
+    const V* xj = x + j * xs;
     double acc = 0.0;
 #pragma unroll
     for (int q = 0; q < KC; ++q)
@@ -664,14 +666,14 @@ __global__ __launch_bounds__(256) void k_bwd_t_sparse(int m, const int* __restri
 #pragma unroll
     for (int q = 0; q < KC; ++q)
       if (q < nu) acc += uc[q].val * (double)xj[(long)bb * m + uc[q].idx];
-    tbuf[j * cs + row] = (V)((double)rw[j * cs + row] - acc);
+    tbuf[j * cs + row] = (V)((double)r[j * rs + row] - acc);
   }
 }
 
 // x[e] = Y_e t[e]
 template <typename B, typename V, int NC, int R>
 __global__ __launch_bounds__(256) void k_bwd_x(int m, int G, int vec, const int* __restrict__ e_line, B Yb,
-                                               const V* __restrict__ tbuf, V* __restrict__ x, long cs) {
+                                               const V* __restrict__ tbuf, long cs, V* __restrict__ x, long xs) {
   const int bi = blockIdx.y;
   const int g = threadIdx.x % G;
   int rr[R];
@@ -685,7 +687,7 @@ __global__ __launch_bounds__(256) void k_bwd_x(int m, int G, int vec, const int*
     for (int i = 0; i < R; ++i)
       if (live[i])
 #pragma unroll
-        for (int j = 0; j < NC; ++j) x[j * cs + base + rr[i]] = (V)d[i][j];
+        for (int j = 0; j < NC; ++j) x[j * xs + base + rr[i]] = (V)d[i][j];
 }
 
 // Levels >= 1 of a factor made with the products Y L and Y U in place of L and U
@@ -694,8 +696,8 @@ __global__ __launch_bounds__(256) void k_bwd_x(int m, int G, int vec, const int*
 template <typename B, typename V, int NC, int R>
 __global__ __launch_bounds__(256) void k_bwd_fused(int m, int G, int vec, const int* __restrict__ e_line,
                                                    const int* __restrict__ a_line, const int* __restrict__ b_line,
-                                                   B Yb, B YLb, B YUb, const V* __restrict__ rw, V* __restrict__ x,
-                                                   long cs) {
+                                                   B Yb, B YLb, B YUb, const V* __restrict__ rw, long cs,
+                                                   V* __restrict__ x, long xs) {
   const int bi = blockIdx.y;
   const int g = threadIdx.x % G;
   int rr[R];
@@ -706,14 +708,14 @@ __global__ __launch_bounds__(256) void k_bwd_fused(int m, int G, int vec, const 
   double acc[R][NC], d[R][NC];
   row_dot<NC, R>(Yb, bi, rr, rw + base, cs, m, g, G, vec, acc);
   if (a >= 0) {
-    row_dot<NC, R>(YLb, bi, rr, x + (long)a * m, cs, m, g, G, vec, d);
+    row_dot<NC, R>(YLb, bi, rr, x + (long)a * m, xs, m, g, G, vec, d);
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
       for (int j = 0; j < NC; ++j) acc[i][j] -= d[i][j];
   }
   if (bb >= 0) {
-    row_dot<NC, R>(YUb, bi, rr, x + (long)bb * m, cs, m, g, G, vec, d);
+    row_dot<NC, R>(YUb, bi, rr, x + (long)bb * m, xs, m, g, G, vec, d);
 #pragma unroll
     for (int i = 0; i < R; ++i)
 #pragma unroll
@@ -724,7 +726,7 @@ __global__ __launch_bounds__(256) void k_bwd_fused(int m, int G, int vec, const 
     for (int i = 0; i < R; ++i)
       if (live[i])
 #pragma unroll
-        for (int j = 0; j < NC; ++j) x[j * cs + base + rr[i]] = (V)acc[i][j];
+        for (int j = 0; j < NC; ++j) x[j * xs + base + rr[i]] = (V)acc[i][j];
 }
 
 // ---- the few-line levels with their operands by value ----------------------------
@@ -756,7 +758,7 @@ __device__ __forceinline__ void small_dot(const Row& row, int r, const V* __rest
 
 template <typename B, typename V, int NC>
 __global__ __launch_bounds__(256) void k_small(int m, int G, int vec, int dir, SmallLevel<B> a, V* __restrict__ rw,
-                                               V* __restrict__ xo, long cs) {
+                                               long cs, V* __restrict__ xo, long xs) {
   const int b = blockIdx.y;
   const int g = threadIdx.x % G;
   const int r = blockIdx.x * rows_per_block(G) + (int)threadIdx.x / G;
@@ -787,18 +789,18 @@ __global__ __launch_bounds__(256) void k_small(int m, int G, int vec, int dir, S
     const long base = (long)a.line[b] * m;
     small_dot<NC>(a.blk[0][b], rr, rw + base, cs, m, g, G, vec, acc);
     if (n1 >= 0) {
-      small_dot<NC>(a.blk[1][b], rr, xo + (long)n1 * m, cs, m, g, G, vec, d);
+      small_dot<NC>(a.blk[1][b], rr, xo + (long)n1 * m, xs, m, g, G, vec, d);
 #pragma unroll
       for (int j = 0; j < NC; ++j) acc[j] -= d[j];
     }
     if (n2 >= 0) {
-      small_dot<NC>(a.blk[2][b], rr, xo + (long)n2 * m, cs, m, g, G, vec, d);
+      small_dot<NC>(a.blk[2][b], rr, xo + (long)n2 * m, xs, m, g, G, vec, d);
 #pragma unroll
       for (int j = 0; j < NC; ++j) acc[j] -= d[j];
     }
     if (live && g == 0)
 #pragma unroll
-      for (int j = 0; j < NC; ++j) xo[j * cs + base + r] = (V)acc[j];
+      for (int j = 0; j < NC; ++j) xo[j * xs + base + r] = (V)acc[j];
   }
 }
 
@@ -822,7 +824,7 @@ struct DenseTop {
 
 template <typename B, typename V, int NC>
 __global__ __launch_bounds__(256) void k_dense_top(int m, int G, int vec, DenseTop<B> a, const V* __restrict__ rw,
-                                                   V* __restrict__ xo, long cs) {
+                                                   long cs, V* __restrict__ xo, long xs) {
   const int b = blockIdx.y;
   const int g = threadIdx.x % G;
   const int r = blockIdx.x * rows_per_block(G) + (int)threadIdx.x / G;
@@ -841,7 +843,7 @@ __global__ __launch_bounds__(256) void k_dense_top(int m, int G, int vec, DenseT
   }
   if (live && g == 0)
 #pragma unroll
-    for (int j = 0; j < NC; ++j) xo[j * cs + (long)a.line[b] * m + r] = (V)acc[j];
+    for (int j = 0; j < NC; ++j) xo[j * xs + (long)a.line[b] * m + r] = (V)acc[j];
 }
 
 // ---- the upper levels in one launch ---------------------------------------------
@@ -887,8 +889,8 @@ struct TopPlan {
 };
 
 template <typename B, typename V, int NC>
-__global__ __launch_bounds__(256) void k_top(int m, int vec, TopPlan<B> tp, V* __restrict__ rw, V* __restrict__ xo,
-                                             long cs, unsigned* __restrict__ sync) {
+__global__ __launch_bounds__(256) void k_top(int m, int vec, TopPlan<B> tp, V* __restrict__ rw, long cs,
+                                             V* __restrict__ xo, long xs, unsigned* __restrict__ sync) {
   __shared__ int s_t;
   for (;;) {
     if (threadIdx.x == 0) s_t = (int)atomicAdd(&sync[0], 1u);
@@ -952,18 +954,18 @@ __global__ __launch_bounds__(256) void k_top(int m, int vec, TopPlan<B> tp, V* _
       double acc[1][NC];
       row_dot<NC, 1>(S.blk[0], b, rr, rw + base, cs, m, g, G, vec, acc);
       if (a >= 0) {
-        row_dot<NC, 1>(S.blk[1], b, rr, xo + (long)a * m, cs, m, g, G, vec, d);
+        row_dot<NC, 1>(S.blk[1], b, rr, xo + (long)a * m, xs, m, g, G, vec, d);
 #pragma unroll
         for (int j = 0; j < NC; ++j) acc[0][j] -= d[0][j];
       }
       if (bb >= 0) {
-        row_dot<NC, 1>(S.blk[2], b, rr, xo + (long)bb * m, cs, m, g, G, vec, d);
+        row_dot<NC, 1>(S.blk[2], b, rr, xo + (long)bb * m, xs, m, g, G, vec, d);
 #pragma unroll
         for (int j = 0; j < NC; ++j) acc[0][j] -= d[0][j];
       }
       if (live && g == 0)
 #pragma unroll
-        for (int j = 0; j < NC; ++j) xo[j * cs + base + r] = (V)acc[0][j];
+        for (int j = 0; j < NC; ++j) xo[j * xs + base + r] = (V)acc[0][j];
     }
     __syncthreads();  // the block's writes of this task are done
     if (threadIdx.x == 0) {
@@ -987,7 +989,7 @@ __global__ __launch_bounds__(256) void k_copy_blocks(long mm, T* const* __restri
   for (long e = blockIdx.x * (long)blockDim.x + threadIdx.x; e < mm; e += (long)gridDim.x * blockDim.x) d[e] = s[e];
 }
 
-// Level 0, kept lines: rw[k] -= L_k y[e1] + U_k y[e2] with the sparse couplings and
+// Level 0, kept lines: rw[k] = r[k] - (L_k y[e1] + U_k y[e2]) with the sparse couplings and
 // y[e] = Y_e rw[e] (so P1 rw[e1] = L_k Y_e1 rw[e1] without reading P1).  Thread per
 // row; the row's couplings are loaded once for all columns.
 template <typename V, int NC>
@@ -995,11 +997,12 @@ __global__ __launch_bounds__(256) void k_fwd_sparse(int m, const int* __restrict
                                                     const int* __restrict__ e1, const int* __restrict__ e2,
                                                     const Cpl* __restrict__ Lr, const int* __restrict__ nLr,
                                                     const Cpl* __restrict__ Ur, const int* __restrict__ nUr,
-                                                    const V* __restrict__ y, V* __restrict__ rw, long cs) {
+                                                    const V* __restrict__ y, const V* __restrict__ r, long rs,
+                                                    V* __restrict__ rw, long cs) {
   const int b = blockIdx.y;
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= m) return;
-  const long row = (long)k_line[b] * m + r;
+  const int loc = blockIdx.x * blockDim.x + threadIdx.x;
+  if (loc >= m) return;
+  const long row = (long)k_line[b] * m + loc;
   const int a = e1[b], c = e2[b];
   const int nl = a >= 0 ? nLr[row] : 0, nu = c >= 0 ? nUr[row] : 0;
   Cpl lc[KC], uc[KC];
@@ -1018,7 +1021,7 @@ __global__ __launch_bounds__(256) void k_fwd_sparse(int m, const int* __restrict
 #pragma unroll
     for (int q = 0; q < KC; ++q)
       if (q < nu) acc += uc[q].val * (double)yj[(long)c * m + uc[q].idx];
-    rw[j * cs + row] = (V)((double)rw[j * cs + row] - acc);
+    rw[j * cs + row] = (V)((double)r[j * rs + row] - acc);
   }
 }
 
@@ -1206,6 +1209,7 @@ struct tf_bcr {
   void* xtab;  // 2 pointers: the outputs of the current graph apply (k_stage_in -> k_stage_out_tab)
   // captured apply: the sweeps rw -> xw replayed as one graph launch (per vector type and column count)
   int use_graph;
+  unsigned long long gen;    // unique to this handle and to what an apply of it launches
   hipStream_t cap;
   BcrGraph g64[2], g32[2];   // [columns - 1]
   size_t es;
@@ -1281,8 +1285,15 @@ void level_gemm(tf_bcr* h, void** A, void** B, void** C, double alpha, double be
   TF_PROF_END(tf::PROF_GEMM, st);
 }
 
-// the captured applies (every vector type and column count) are made again on next use
+unsigned long long new_gen() {
+  static std::atomic<unsigned long long> next{1};
+  return next++;
+}
+
+// what an apply launches changes: the captured applies (every vector type and column
+// count) are made again on next use, also those that a Krylov handle captured
 void drop_graphs(tf_bcr* h) {
+  h->gen = new_gen();
   for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
     if (g->exec) (void)hipGraphExecDestroy(g->exec);
     if (g->graph) (void)hipGraphDestroy(g->graph);
@@ -1471,11 +1482,25 @@ bool dense_top(const tf_bcr* h, DenseTop<B>& a) {
   return true;
 }
 
-// forward and backward sweeps over the levels, rows read through the block
-// source B, for NC columns at stride cs in rw, tb, xo (and the handle's yb)
+// Vectors of an apply, line-major, NC columns each: the right-hand sides r at stride rs
+// (the caller's, or rw), the work vectors rw and tb (and the handle's yb) at stride cs,
+// the solutions x at stride xs (the caller's, or xw).
+template <typename V>
+struct ApplyVecs {
+  const V* r;
+  long rs;
+  V *rw, *tb;
+  long cs;
+  V* x;
+  long xs;
+};
+
+// forward and backward sweeps over the levels, rows read through the block source B
 template <typename B, typename V, int NC>
 void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&), B Lb(const BcrLevelDev&),
-           B Ub(const BcrLevelDev&), B Yb(const BcrLevelDev&), V* rw, V* tb, V* xo, long cs, hipStream_t st) {
+           B Ub(const BcrLevelDev&), B Yb(const BcrLevelDev&), const ApplyVecs<V>& v, hipStream_t st) {
+  V *rw = v.rw, *tb = v.tb, *xo = v.x;
+  const long cs = v.cs, xs = v.xs;
   const int m = h->m;
   const dim3 blk(256);
   auto gx = [m](int G, int R) { return (unsigned)((m + R * rows_per_block(G) - 1) / (R * rows_per_block(G))); };
@@ -1534,14 +1559,14 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
       with_rows(rows_for<B>(L.ne, m), [&](auto Rc) {
         constexpr int R = decltype(Rc)::value;
         hipLaunchKernelGGL((k_bwd_x<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, Yb(L),
-                           (const V*)rw, yb, cs);
+                           v.r, v.rs, yb, cs);
       });
       hipLaunchKernelGGL((k_fwd_sparse<V, NC>), dim3(gs, L.nk), blk, 0, st, m, L.k, L.k1, L.k2, h->Lr, h->nLr, h->Ur,
-                         h->nUr, (const V*)yb, rw, cs);
+                         h->nUr, (const V*)yb, v.r, v.rs, rw, cs);
     } else if (SmallLevel<B> sa; h->use_small && L.nk <= SMALL_MAX && rows_for<B>(L.nk, m) == 1 &&
                                  small_level<B>(h, L.nk, L.k, L.k1, L.k2, P1(L), P2(L), nullptr, sa)) {
       hipLaunchKernelGGL((k_small<B, V, NC>), dim3(gx(group_for(L.nk), 1), L.nk), blk, 0, st, m, group_for(L.nk),
-                         vec, 0, sa, rw, xo, cs);
+                         vec, 0, sa, rw, cs, xo, xs);
     } else {
       const int G = group_for(L.nk);
       with_rows(rows_for<B>(L.nk, m), [&](auto Rc) {
@@ -1552,11 +1577,11 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
     }
   }
   if (top)
-    hipLaunchKernelGGL((k_top<B, V, NC>), dim3(TOP_BLOCKS), blk, 0, st, m, vec, tp, rw, xo, cs, h->topsync);
+    hipLaunchKernelGGL((k_top<B, V, NC>), dim3(TOP_BLOCKS), blk, 0, st, m, vec, tp, rw, cs, xo, xs, h->topsync);
   if (dense) {
     const int G = group_for(zt.n);
-    hipLaunchKernelGGL((k_dense_top<ZB, V, NC>), dim3(gx(G, 1), zt.n), blk, 0, st, m, G, vec, zt, (const V*)rw, xo,
-                       cs);
+    hipLaunchKernelGGL((k_dense_top<ZB, V, NC>), dim3(gx(G, 1), zt.n), blk, 0, st, m, G, vec, zt, (const V*)rw, cs,
+                       xo, xs);
   }
   for (int l = dense ? h->zl - 1 : (top ? lt - 1 : nlev - 1); l >= 0; --l) {
     const BcrLevelDev& L = h->lev[l];
@@ -1564,7 +1589,7 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
     if (SmallLevel<B> sa; l > 0 && h->fused && h->use_small && L.ne <= SMALL_MAX && rows_for<B>(L.ne, m) == 1) {
       const B ub = Ub(L);
       if (small_level<B>(h, L.ne, L.e, L.ea, L.eb, Yb(L), Lb(L), &ub, sa)) {
-        hipLaunchKernelGGL((k_small<B, V, NC>), dim3(gx(G, 1), L.ne), blk, 0, st, m, G, vec, 1, sa, rw, xo, cs);
+        hipLaunchKernelGGL((k_small<B, V, NC>), dim3(gx(G, 1), L.ne), blk, 0, st, m, G, vec, 1, sa, rw, cs, xo, xs);
         continue;
       }
     }
@@ -1572,17 +1597,17 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
       constexpr int R = decltype(Rc)::value;
       if (l > 0 && h->fused) {
         hipLaunchKernelGGL((k_bwd_fused<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, L.ea, L.eb,
-                           Yb(L), Lb(L), Ub(L), (const V*)rw, xo, cs);
+                           Yb(L), Lb(L), Ub(L), (const V*)rw, cs, xo, xs);
         return;
       }
       if (l == 0)
         hipLaunchKernelGGL((k_bwd_t_sparse<V, NC>), dim3(gs, L.ne), blk, 0, st, m, L.e, L.ea, L.eb, h->Lr, h->nLr,
-                           h->Ur, h->nUr, (const V*)rw, (const V*)xo, tb, cs);
+                           h->Ur, h->nUr, v.r, v.rs, (const V*)xo, xs, tb, cs);
       else
         hipLaunchKernelGGL((k_bwd_t<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, L.ea, L.eb, Lb(L),
-                           Ub(L), (const V*)rw, (const V*)xo, tb, cs);
+                           Ub(L), (const V*)rw, (const V*)xo, tb, cs, xs);
       hipLaunchKernelGGL((k_bwd_x<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, Yb(L),
-                         (const V*)tb, xo, cs);
+                         (const V*)tb, cs, xo, xs);
     });
   }
 }
@@ -1593,28 +1618,34 @@ inline bool aligned16(const void* p, long cs, int nc, size_t es) {
   return ((uintptr_t)p & 15) == 0 && (nc == 1 || (cs * (long)es) % 16 == 0);
 }
 
+template <typename V, int NC>
+bool vectors_aligned16(const ApplyVecs<V>& v) {
+  return aligned16(v.r, v.rs, NC, sizeof(V)) && aligned16(v.rw, v.cs, NC, sizeof(V)) &&
+         aligned16(v.x, v.xs, NC, sizeof(V));
+}
+
 template <typename T, typename V, int NC>
-void levels(tf_bcr* h, V* rw, V* tb, V* xo, long cs, hipStream_t st) {
+void levels(tf_bcr* h, const ApplyVecs<V>& v, hipStream_t st) {
   constexpr int W = 16 / (int)sizeof(T);
-  const int vec = (sizeof(T) == sizeof(V) && h->m % W == 0 && aligned16(xo, cs, NC, sizeof(V))) ? 1 : 0;
+  const int vec = (sizeof(T) == sizeof(V) && h->m % W == 0 && vectors_aligned16<V, NC>(v)) ? 1 : 0;
   typedef Blocks<T> B;
   sweep<B, V, NC>(
       h, vec, [](const BcrLevelDev& L) { return B{(T* const*)L.P1}; },
       [](const BcrLevelDev& L) { return B{(T* const*)L.P2}; }, [](const BcrLevelDev& L) { return B{(T* const*)L.Le}; },
       [](const BcrLevelDev& L) { return B{(T* const*)L.Ue}; }, [](const BcrLevelDev& L) { return B{(T* const*)L.Ye}; },
-      rw, tb, xo, cs, st);
+      v, st);
 }
 
 template <int NC>
-void levels_half(tf_bcr* h, float* rw, float* tb, float* xo, long cs, hipStream_t st) {
-  const int vec = (h->m % 8 == 0 && aligned16(xo, cs, NC, sizeof(float))) ? 1 : 0;
+void levels_half(tf_bcr* h, const ApplyVecs<float>& v, hipStream_t st) {
+  const int vec = (h->m % 8 == 0 && vectors_aligned16<float, NC>(v)) ? 1 : 0;
   typedef HalfBlocks B;
   sweep<B, float, NC>(
       h, vec, [](const BcrLevelDev& L) { return B{(f16* const*)L.P1h, (float* const*)L.P1s}; },
       [](const BcrLevelDev& L) { return B{(f16* const*)L.P2h, (float* const*)L.P2s}; },
       [](const BcrLevelDev& L) { return B{(f16* const*)L.Lh, (float* const*)L.Ls}; },
       [](const BcrLevelDev& L) { return B{(f16* const*)L.Uh, (float* const*)L.Us}; },
-      [](const BcrLevelDev& L) { return B{(f16* const*)L.Yh, (float* const*)L.Ys}; }, rw, tb, xo, cs, st);
+      [](const BcrLevelDev& L) { return B{(f16* const*)L.Yh, (float* const*)L.Ys}; }, v, st);
 }
 
 // algorithmic bytes of an NC-column apply: the factor blocks once (the dense top's in
@@ -1633,18 +1664,23 @@ double solve_work(const tf_bcr* h) {
 
 constexpr int solve_prof_id(int nc) { return nc == 1 ? tf::PROF_SOLVE : tf::PROF_SOLVE2; }
 
-// The sweeps of an apply on the work vectors: rw (right-hand sides, line-major,
-// overwritten) -> xo (solutions, line-major), NC columns at stride n.
+// The sweeps of an apply.
 template <typename T, typename V, int NC>
-void run_levels(tf_bcr* h, V* rw, V* xo, hipStream_t st) {
-  const long n = h->n;
-  V* tb = (V*)h->tb;
-  bool half = false;
-  if constexpr (sizeof(T) == 4 && sizeof(V) == 4) half = h->half != 0;
+void run_levels(tf_bcr* h, const ApplyVecs<V>& v, hipStream_t st) {
   if constexpr (sizeof(T) == 4 && sizeof(V) == 4) {
-    if (half) levels_half<NC>(h, (float*)rw, (float*)tb, (float*)xo, n, st);
+    if (h->half) {
+      levels_half<NC>(h, v, st);
+      return;
+    }
   }
-  if (!half) levels<T, V, NC>(h, rw, tb, xo, n, st);
+  levels<T, V, NC>(h, v, st);
+}
+
+// the apply on the handle's own vectors: rw (overwritten) -> xw
+template <typename V>
+ApplyVecs<V> own_vecs(tf_bcr* h) {
+  const long n = h->n;
+  return ApplyVecs<V>{(const V*)h->rw, n, (V*)h->rw, (V*)h->tb, n, (V*)h->xw, n};
 }
 
 // r[j] (natural order) -> the work vector rw, one launch for all columns; x (or null):
@@ -1669,18 +1705,45 @@ void stage_out(const tf_bcr* h, const V* xo, V* const (&x)[NC], hipStream_t st) 
   hipLaunchKernelGGL((k_stage_out<V, NC>), dim3(1024), dim3(256), 0, st, h->n, h->order, xo, (long)h->n, c);
 }
 
+// Whether the sweeps can work on the caller's vectors: lines in natural order, columns
+// that do not overlap one another (a solution line is written before the last
+// right-hand side is read) and are aligned as the handle's own are.
+template <typename V, int NC>
+bool direct_vecs(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], ApplyVecs<V>& v) {
+  if (h->order.ylines) return false;
+  const uintptr_t bytes = sizeof(V) * (uintptr_t)h->n;
+  auto apart = [bytes](const void* a, const void* b) {
+    return (uintptr_t)a + bytes <= (uintptr_t)b || (uintptr_t)b + bytes <= (uintptr_t)a;
+  };
+  for (int i = 0; i < NC; ++i)
+    for (int j = 0; j < NC; ++j)
+      if (!apart(r[i], x[j]) || (i < j && !apart(x[i], x[j]))) return false;
+  const intptr_t dr = (intptr_t)r[NC - 1] - (intptr_t)r[0], dx = (intptr_t)x[NC - 1] - (intptr_t)x[0];
+  if (dr % (intptr_t)sizeof(V) || dx % (intptr_t)sizeof(V)) return false;
+  v = own_vecs<V>(h);
+  const bool own = vectors_aligned16<V, NC>(v);
+  v.r = r[0];
+  v.rs = (long)(dr / (intptr_t)sizeof(V));
+  v.x = x[0];
+  v.xs = (long)(dx / (intptr_t)sizeof(V));
+  return !own || vectors_aligned16<V, NC>(v);
+}
+
 // NC right-hand sides r[j] -> solutions x[j] (host arrays of device pointers), eager.
+// Where they can be read and written in place, the gather and the scatter (2.5 us each
+// at 64 x 64, 4 at 256 x 256, and as much again to start them) are left out.
 template <typename T, typename V, int NC>
 int solve_impl(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream_t st) {
-  V* rw = (V*)h->rw;
   TF_PROF_WORK(solve_prof_id(NC), (solve_work<T, V, NC>(h)));
   TF_PROF_BEGIN(solve_prof_id(NC), st);
-  // one column in natural order: the kernels write the solution in place
-  const bool direct = !h->order.ylines && NC == 1;
-  V* xo = direct ? x[0] : (V*)h->xw;
-  stage_in<V, NC>(h, r, rw, nullptr, st);
-  run_levels<T, V, NC>(h, rw, xo, st);
-  if (!direct) stage_out<V, NC>(h, xo, x, st);
+  if (ApplyVecs<V> v; direct_vecs<V, NC>(h, r, x, v)) {
+    run_levels<T, V, NC>(h, v, st);
+  } else {
+    v = own_vecs<V>(h);
+    stage_in<V, NC>(h, r, v.rw, nullptr, st);
+    run_levels<T, V, NC>(h, v, st);
+    stage_out<V, NC>(h, v.x, x, st);
+  }
   TF_PROF_END(solve_prof_id(NC), st);
   TF_LAUNCH_CHECK("bcr solve");
   return 0;
@@ -1707,7 +1770,7 @@ int solve_graph(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream
     {
       std::lock_guard<std::mutex> lock(tf::capture_mutex());
       TF_HIP(hipStreamBeginCapture(h->cap, hipStreamCaptureModeThreadLocal));
-      run_levels<T, V, NC>(h, rw, xw, h->cap);
+      run_levels<T, V, NC>(h, own_vecs<V>(h), h->cap);
       hipLaunchKernelGGL((k_stage_out_tab<V, NC>), dim3(1024), dim3(256), 0, h->cap, h->n, h->order,
                          (const V*)xw, (long)h->n, (V* const*)h->xtab);
       le = hipGetLastError();
@@ -1743,6 +1806,28 @@ int solve_any(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream_t
 }
 
 }  // namespace
+
+namespace tf {
+// For callers that capture an apply in a graph of their own: whether this handle's
+// applies are to be replayed, and the number under which that stays the same apply.
+bool bcr_replays(const tf_bcr* h, unsigned long long* gen) {
+  *gen = h->gen;
+  return h->use_graph != 0;
+}
+// the launches of one apply of nc (1 or 2) columns (single: FP32 vectors)
+int bcr_apply(tf_bcr* h, int single, int nc, const void* r0, const void* r1, void* x0, void* x1, hipStream_t st) {
+  auto go = [&](auto* t) -> int {
+    typedef typename std::remove_pointer<decltype(t)>::type V;
+    const V* const r1c[1] = {(const V*)r0};
+    V* const x1c[1] = {(V*)x0};
+    const V* const r2c[2] = {(const V*)r0, (const V*)r1};
+    V* const x2c[2] = {(V*)x0, (V*)x1};
+    if (h->single) return nc == 2 ? solve_impl<float, V, 2>(h, r2c, x2c, st) : solve_impl<float, V, 1>(h, r1c, x1c, st);
+    return nc == 2 ? solve_impl<double, V, 2>(h, r2c, x2c, st) : solve_impl<double, V, 1>(h, r1c, x1c, st);
+  };
+  return single ? go((float*)nullptr) : go((double*)nullptr);
+}
+}  // namespace tf
 
 // ---- C ABI -----------------------------------------------------------------------
 
@@ -1786,6 +1871,7 @@ int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int y
   if (ylines && (nx < 1 || dof < 1 || m % dof != 0 || (long)nx * m != n))
     return tf::fail("y-line order needs n = nx * m with m = ny * dof");
   tf_bcr* h = new tf_bcr();
+  h->gen = new_gen();
   const int rc = bcr_create_impl(h, n, m, single, nx, dof, ylines);
   if (rc) {
     // frees whatever was allocated before the failure (unset members are null)
@@ -2115,13 +2201,7 @@ int tf_bcr_status(tf_bcr* h, int* flags_host, void* stream) {
 int tf_bcr_set_top(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
   if (on) return tf::fail("tf_bcr_set_top: the one-launch upper levels are disabled (they did not finish on the GPU)");
-  if ((on != 0) != (h->use_top != 0)) {
-    for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
-      if (g->exec) (void)hipGraphExecDestroy(g->exec);
-      if (g->graph) (void)hipGraphDestroy(g->graph);
-      *g = BcrGraph{};
-    }
-  }
+  if ((on != 0) != (h->use_top != 0)) drop_graphs(h);
   h->use_top = on ? 1 : 0;
   return 0;
 }
@@ -2131,13 +2211,7 @@ int tf_bcr_set_top(tf_bcr* h, int on) {
 // other levels.  The results are the same bit for bit.
 int tf_bcr_set_small(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
-  if ((on != 0) != (h->use_small != 0)) {
-    for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
-      if (g->exec) (void)hipGraphExecDestroy(g->exec);
-      if (g->graph) (void)hipGraphDestroy(g->graph);
-      *g = BcrGraph{};
-    }
-  }
+  if ((on != 0) != (h->use_small != 0)) drop_graphs(h);
   h->use_small = on ? 1 : 0;
   return 0;
 }
@@ -2286,14 +2360,7 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
     h->cv_scl = (void**)(P + occ);
     h->ncv = (int)cs.size();
   }
-  if ((on != 0) != (h->half != 0)) {
-    // the captured FP32 applies read the other storage: capture them again
-    for (BcrGraph& g : h->g32) {
-      if (g.exec) (void)hipGraphExecDestroy(g.exec);
-      if (g.graph) (void)hipGraphDestroy(g.graph);
-      g = BcrGraph{};
-    }
-  }
+  if ((on != 0) != (h->half != 0)) drop_graphs(h);  // the FP32 applies read the other storage
   h->half = on ? 1 : 0;
   if (h->half && h->factored && h->ncv > 0) {
     hipLaunchKernelGGL(k_to_half, dim3((m + 3) / 4, h->ncv), dim3(256), 0, st, m, (float* const*)h->cv_src,
@@ -2321,6 +2388,7 @@ int tf_bcr_set_fused(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
   if (h->factored && (on != 0) != (h->fused != 0))
     return tf::fail("tf_bcr_set_fused: the handle already holds a factor of the other form");
+  if ((on != 0) != (h->fused != 0)) drop_graphs(h);
   h->fused = on ? 1 : 0;
   return 0;
 }

@@ -9,15 +9,16 @@
 // FGMRES: stop when the residual estimate |g_{j+1}| <= tol ||b||, restart with
 // the true residual b - A x.
 //
-// The device part of Arnoldi step j (SpMV of Z[j], two Gram-Schmidt passes
-// against V[0..j], the normalisation into V[j+1] and the copy of the (j+2)-entry
-// column to pinned host memory) is captured once per j into a hipGraph and
-// replayed with one launch; the SpMV reads the matrix through a small device
-// descriptor that each solve points at its own CSR arrays, so the graphs stay
-// valid across Jacobians.  The host then waits for the column by polling (no
-// blocking wait, whose wake-up would leave the GPU idle longer); while the
-// residual estimate is far from the tolerance, the preconditioner on the new basis
-// vector is queued before that wait, so the device is busy through the host's part.
+// The device part of Arnoldi step j is the SpMV of Z[j], two Gram-Schmidt passes
+// against V[0..j], the normalisation into V[j+1] and the (j+2)-entry column into pinned
+// host memory.  With a line factor it is captured together with the preconditioner's
+// apply V[j] -> Z[j] before it, on the third use of a basis index, and the whole
+// iteration replayed with one launch; with the other preconditioners the step alone is.
+// The SpMV reads the matrix through a small device descriptor that each solve points at
+// its own CSR arrays, so the graphs stay valid across Jacobians.  The host then waits
+// for the column by polling a word that the step sets behind it; while the residual
+// estimate is far from the tolerance, the next iteration (other preconditioners: its
+// apply) is queued before that wait, so the device is busy through the host's part.
 #include "spmv.h"
 #include "tf_common.h"
 #include "transiflow_hip.h"
@@ -28,6 +29,8 @@
 
 namespace {
 constexpr int MAX_STEPS = 256;   // Arnoldi steps per restart cycle (tf_krylov_max_basis)
+constexpr int HSLOT = tf::HFLAG + 1;  // words of a pinned column
+constexpr int CAPTURE_USE = 3;   // use of a basis index on which its iteration is captured
 
 struct MatrixDesc {
   const int* rp;
@@ -46,7 +49,7 @@ struct tf_krylov {
   double* h;   // m+2 (device)
   double* y;   // m+1 (device)
   double* work;
-  double* h_host;      // m+2 (pinned, coherent)
+  double* h_host;      // two columns of m+2 and the word HFLAG, of the even and the odd steps (pinned, coherent)
   double* h_host_dev;  // h_host as kernels address it
   MatrixDesc* desc;          // the matrix of the current solve (device)
   hipStream_t cap;           // private stream the step graphs are captured on
@@ -57,12 +60,22 @@ struct tf_krylov {
   hipGraph_t step2_graph[MAX_STEPS];
   unsigned long long uid;            // unique per handle (a freed handle's address can come back)
   unsigned long long step2_partner;  // uid of the partner the step2 graphs were captured with
+  // iterations of one and of two systems (captured on the first one's handle): the line
+  // factor's apply and the step.  iter_key: the apply's number (tf::bcr_replays) and,
+  // for two, the partner's uid.
+  hipGraphExec_t iter[2][MAX_STEPS];
+  int iter_uses[2][MAX_STEPS];
+  unsigned long long iter_key[2][2];
   hipEvent_t step_done;              // recorded after a step's Hessenberg column is queued to the host
   double last_sn0;                   // |sine| of the first rotation of the last cycle (0: none yet)
   int use_graph;
 };
 
 namespace tf {
+// whether step j of n entries writes its column to hh itself and then sets its HFLAG
+bool cgs2_to_host(int n, int j);
+bool bcr_replays(const tf_bcr* h, unsigned long long* gen);
+int bcr_apply(tf_bcr* h, int single, int nc, const void* r0, const void* r1, void* x0, void* x1, hipStream_t st);
 // hh0, hh1: the device address of pinned host copies of h (or null); *to_host = 1
 // when the launches wrote the column there
 int cgs2_pair_f64(int n, int j, const double* V0, const double* V1, double* w0, double* w1, double* work0,
@@ -158,6 +171,10 @@ int norm(const tf_krylov* k, int n, const void* x, double* out, hipStream_t st) 
   return 0;
 }
 
+// the pinned column of step j, for the host and for kernels
+double* hh(const tf_krylov* k, int j) { return k->h_host + (j & 1) * HSLOT; }
+double* hh_dev(const tf_krylov* k, int j) { return k->h_host_dev + (j & 1) * HSLOT; }
+
 // The device part of Arnoldi step j on stream st: w = A Z[j] (through the
 // descriptor), CGS2 h = V^T w, w -= V h, y = V^T w, w -= V y, h += y, V[j+1] =
 // w / |w| with |w| into h[j+1], and h[0..j+1] into h_host (written there by the
@@ -174,11 +191,11 @@ int arnoldi_step(tf_krylov* k, int j, hipStream_t st) {
   TF_LAUNCH_CHECK("fgmres spmv");
   int to_host = 0;
   if (int e = k->single ? tf::cgs2_one_f32(n, j, (const float*)k->V, (float*)k->w, k->work, k->h, k->y,
-                                           (float*)o.V(j + 1), k->h_host_dev, &to_host, st)
+                                           (float*)o.V(j + 1), hh_dev(k, j), &to_host, st)
                         : tf::cgs2_one_f64(n, j, (const double*)k->V, (double*)k->w, k->work, k->h, k->y,
-                                           (double*)o.V(j + 1), k->h_host_dev, &to_host, st))
+                                           (double*)o.V(j + 1), hh_dev(k, j), &to_host, st))
     return e;
-  if (!to_host) TF_HIP(hipMemcpyAsync(k->h_host, k->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
+  if (!to_host) TF_HIP(hipMemcpyAsync(hh(k, j), k->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
   return 0;
 }
 
@@ -229,15 +246,15 @@ int arnoldi_step2(tf_krylov* a, tf_krylov* b, int j, hipStream_t st) {
   int to_host = 0;
   if (int e = a->single ? tf::cgs2_pair_f32(n, j, (const float*)a->V, (const float*)b->V, (float*)a->w, (float*)b->w,
                                             a->work, b->work, a->h, b->h, a->y, b->y, (float*)oa.V(j + 1),
-                                            (float*)ob.V(j + 1), a->h_host_dev, b->h_host_dev, &to_host, st)
+                                            (float*)ob.V(j + 1), hh_dev(a, j), hh_dev(b, j), &to_host, st)
                         : tf::cgs2_pair_f64(n, j, (const double*)a->V, (const double*)b->V, (double*)a->w,
                                             (double*)b->w, a->work, b->work, a->h, b->h, a->y, b->y,
-                                            (double*)oa.V(j + 1), (double*)ob.V(j + 1), a->h_host_dev, b->h_host_dev,
+                                            (double*)oa.V(j + 1), (double*)ob.V(j + 1), hh_dev(a, j), hh_dev(b, j),
                                             &to_host, st))
     return e;
   if (!to_host) {
-    TF_HIP(hipMemcpyAsync(a->h_host, a->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
-    TF_HIP(hipMemcpyAsync(b->h_host, b->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
+    TF_HIP(hipMemcpyAsync(hh(a, j), a->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
+    TF_HIP(hipMemcpyAsync(hh(b, j), b->h, sizeof(double) * (j + 2), hipMemcpyDeviceToHost, st));
   }
   return 0;
 }
@@ -278,6 +295,82 @@ int arnoldi_step2_graph(tf_krylov* a, tf_krylov* b, int j, hipStream_t st) {
     a->step2[j] = ex;
   }
   TF_HIP(hipGraphLaunch(a->step2[j], st));
+  return 0;
+}
+
+// The word of handle k that the last launch of step j sets once its column is in host memory.
+unsigned long long* column_flag(const tf_krylov* k, int j) { return (unsigned long long*)(hh(k, j) + tf::HFLAG); }
+
+// Wait until the columns of step j of the nk handles are in host memory, by polling
+// their words (the stream's own state, looked at now and then, ends the wait if the
+// step failed).
+int poll_columns(tf_krylov* const* k, int nk, int j, hipStream_t st) {
+  for (int q = 0; q < nk; ++q)
+    for (unsigned spins = 1; !__atomic_load_n(column_flag(k[q], j), __ATOMIC_ACQUIRE); ++spins) {
+      if (spins % (1u << 16)) continue;
+      const hipError_t e = hipStreamQuery(st);
+      if (e == hipErrorNotReady) continue;
+      if (e != hipSuccess) return tf::fail_hip(e, "Arnoldi step");
+      if (!__atomic_load_n(column_flag(k[q], j), __ATOMIC_ACQUIRE))
+        return tf::fail("the Arnoldi step ended without its column");
+    }
+  return 0;
+}
+
+// Iteration j of one handle or two (nk): the line factor's apply V[j] -> Z[j] and the
+// Arnoldi step.
+int iteration(tf_krylov* const* k, int nk, int j, tf_bcr* prec, hipStream_t st) {
+  Ops a{k[0], k[0]->n, st}, b{k[nk - 1], k[0]->n, st};
+  if (int e = tf::bcr_apply(prec, k[0]->single, nk, a.V(j), b.V(j), a.Z(j), b.Z(j), st)) return e;
+  return nk == 2 ? arnoldi_step2(k[0], k[1], j, st) : arnoldi_step(k[0], j, st);
+}
+
+void drop_iterations(tf_krylov* k, int which) {
+  for (int j = 0; j < MAX_STEPS; ++j) {
+    if (k->iter[which][j]) (void)hipGraphExecDestroy(k->iter[which][j]);
+    k->iter[which][j] = nullptr;
+    k->iter_uses[which][j] = 0;
+  }
+}
+
+// Iteration j, its launches issued one by one the first times (a solve that is not
+// repeated pays for no capture) and replayed from then on.  gen: the apply's number; when
+// it or the partner changes, no earlier replay is in flight (a solve ends with a wait).
+// A replay starts about 8 us after what precedes it: with one for the apply and one for
+// the step, and the gather, the scatter and the event between them, an iteration of the
+// 64 x 64 grid took 137 us for about 100 us of kernels (continuation 71.4 -> 67.2 ms,
+// 256 x 256 Newton step 11.27 -> 10.87 ms).
+int iteration_replay(tf_krylov* const* k, int nk, int j, tf_bcr* prec, unsigned long long gen, hipStream_t st) {
+  tf_krylov* a = k[0];
+  const int w = nk - 1;
+  const unsigned long long key[2] = {gen, nk == 2 ? k[1]->uid : 0};
+  if (a->iter_key[w][0] != key[0] || a->iter_key[w][1] != key[1]) {
+    drop_iterations(a, w);
+    a->iter_key[w][0] = key[0];
+    a->iter_key[w][1] = key[1];
+  }
+  if (!a->iter[w][j] && ++a->iter_uses[w][j] >= CAPTURE_USE) {
+    if (!a->cap) TF_HIP(hipStreamCreateWithFlags(&a->cap, hipStreamNonBlocking));
+    hipGraph_t g = nullptr;
+    hipGraphExec_t ex = nullptr;
+    bool ok = false;
+    {
+      std::lock_guard<std::mutex> lock(tf::capture_mutex());
+      TF_HIP(hipStreamBeginCapture(a->cap, hipStreamCaptureModeThreadLocal));
+      const int e = iteration(k, nk, j, prec, a->cap);
+      const hipError_t ce = hipStreamEndCapture(a->cap, &g);
+      ok = !e && ce == hipSuccess && g && hipGraphInstantiate(&ex, g, nullptr, nullptr, 0) == hipSuccess;
+    }
+    if (g) (void)hipGraphDestroy(g);
+    if (ok) {
+      a->iter[w][j] = ex;
+    } else {
+      (void)hipGetLastError();  // issued one by one, and captured again next time
+      tf::note_capture_fallback();
+    }
+  }
+  if (!a->iter[w][j]) return iteration(k, nk, j, prec, st);
+  TF_HIP(hipGraphLaunch(a->iter[w][j], st));
   return 0;
 }
 
@@ -379,7 +472,7 @@ int col_begin_cycle(Column& c, const int* rp, const int* ci, const void* val, in
 // estimate, the iteration limit, a breakdown or a non-finite estimate.
 void col_givens(Column& c, int j, int maxit) {
   const double tol = c.tol;
-  for (int i = 0; i <= j + 1; ++i) c.Hij(i, j) = c.k->h_host[i];
+  for (int i = 0; i <= j + 1; ++i) c.Hij(i, j) = hh(c.k, j)[i];
   for (int i = 0; i < j; ++i) {
     const double t = c.cs[i] * c.Hij(i, j) + c.sn[i] * c.Hij(i + 1, j);
     c.Hij(i + 1, j) = -c.sn[i] * c.Hij(i, j) + c.cs[i] * c.Hij(i + 1, j);
@@ -472,6 +565,10 @@ int fgmres_columns(Column* c, int nc, const int* rp, const int* ci, const void* 
     hipLaunchKernelGGL(k_set_desc, dim3(1), dim3(1), 0, st, c[q].k->desc, rp, ci, val, gauge);
   TF_LAUNCH_CHECK("fgmres descriptor");
   const int m = c[0].k->m;
+  // a line factor whose applies are replayed: whole iterations are
+  unsigned long long gen = 0;
+  bool whole = prec_kind == 1 && prec && tf::bcr_replays((const tf_bcr*)prec, &gen) && !tf::prof_on();
+  for (int q = 0; q < nc; ++q) whole = whole && c[q].k->use_graph;
   for (;;) {
     bool any = false;
     for (int q = 0; q < nc; ++q) {
@@ -480,42 +577,56 @@ int fgmres_columns(Column* c, int nc, const int* rp, const int* ci, const void* 
       any = any || c[q].in_cycle;
     }
     if (!any) break;
-    // Z[j] of the stepping columns already queued by the previous step's look-ahead
-    bool have_z = false;
+    // queued by the previous step's look-ahead: Z[j] of the stepping columns, and (line
+    // factor) all of iteration j
+    bool have_z = false, have_step = false;
     for (int j = 0; j < m; ++j) {
-      bool stepping = false;
-      for (int q = 0; q < nc; ++q) stepping = stepping || c[q].stepping;
-      if (!stepping) break;
-      if (!have_z)
-        if (int e = precond_columns(c, nc, j, prec_kind, prec, ncell, dof, st)) return e;
-      if (nc == 2 && c[0].stepping && c[1].stepping) {
-        tf_krylov* a = c[0].k;
-        tf_krylov* b = c[1].k;
-        if (int e = (a->use_graph && !tf::prof_on()) ? arnoldi_step2_graph(a, b, j, st) : arnoldi_step2(a, b, j, st))
-          return e;
+      // the stepping columns' handles; their words cleared for step i
+      tf_krylov* active[2];
+      int na = 0;
+      for (int q = 0; q < nc; ++q)
+        if (c[q].stepping) active[na++] = c[q].k;
+      if (na == 0) break;
+      auto clear = [&](int i) {
+        for (int q = 0; q < na; ++q) __atomic_store_n(column_flag(active[q], i), 0ull, __ATOMIC_RELEASE);
+      };
+      const bool flagged = tf::cgs2_to_host(active[0]->n, j);
+      if (!have_step) clear(j);
+      if (whole) {
+        if (!have_step)
+          if (int e = iteration_replay(active, na, j, (tf_bcr*)prec, gen, st)) return e;
       } else {
-        for (int q = 0; q < nc; ++q) {
-          if (!c[q].stepping) continue;
-          tf_krylov* k = c[q].k;
-          if (int e = (k->use_graph && !tf::prof_on()) ? arnoldi_step_graph(k, j, st) : arnoldi_step(k, j, st))
+        if (!have_z)
+          if (int e = precond_columns(c, nc, j, prec_kind, prec, ncell, dof, st)) return e;
+        const bool replay = active[0]->use_graph && !tf::prof_on();
+        if (na == 2) {
+          if (int e = replay ? arnoldi_step2_graph(active[0], active[1], j, st)
+                             : arnoldi_step2(active[0], active[1], j, st))
             return e;
+        } else if (int e = replay ? arnoldi_step_graph(active[0], j, st) : arnoldi_step(active[0], j, st)) {
+          return e;
         }
       }
-      // Look-ahead: when every stepping column will most likely go on, the
-      // preconditioner on V[j+1] (written by the step just queued) is queued before
-      // the host waits for the Hessenberg column, so the device works through the
-      // host's Givens update.  The arithmetic is unchanged; a wrong guess costs one
-      // unused Z[j+1].
+      // Look-ahead: when every stepping column will most likely go on, the next
+      // iteration (or the preconditioner on V[j+1], written by the step just queued) is
+      // queued before the host waits for the Hessenberg column, so the device works
+      // through the host's Givens update.  The arithmetic is unchanged; a wrong guess
+      // costs one unused iteration (a column that stops at j uses nothing of j + 1).
       bool ahead = j + 1 < m;
       for (int q = 0; q < nc; ++q)
         if (c[q].stepping && !col_continues(c[q], j, maxit)) ahead = false;
       have_z = ahead;
-      // the event marks the step's Hessenberg columns as visible to the host
+      have_step = ahead && whole;
+      // columns that are copied: an event marks them as visible to the host
       hipEvent_t ev = c[0].k->step_done;
-      TF_HIP(hipEventRecord(ev, st));
-      if (ahead)
+      if (!flagged) TF_HIP(hipEventRecord(ev, st));
+      if (have_step) {
+        clear(j + 1);
+        if (int e = iteration_replay(active, na, j + 1, (tf_bcr*)prec, gen, st)) return e;
+      } else if (ahead) {
         if (int e = precond_columns(c, nc, j + 1, prec_kind, prec, ncell, dof, st)) return e;
-      if (int e = poll_event(ev)) return e;
+      }
+      if (int e = flagged ? poll_columns(active, na, j, st) : poll_event(ev)) return e;
       for (int q = 0; q < nc; ++q)
         if (c[q].stepping) col_givens(c[q], j, maxit);
     }
@@ -550,7 +661,7 @@ int tf_krylov_create(tf_krylov** out, int n, int restart, int single) {
     TF_HIP(hipMalloc(&k->work, sizeof(double) * (size_t)tf_krylov_work_size()));
     // coherent: the Arnoldi step's last kernel writes the Hessenberg column here
     // and the host reads it as soon as the step's completion is seen
-    TF_HIP(hipHostMalloc(&k->h_host, sizeof(double) * (restart + 2), hipHostMallocCoherent));
+    TF_HIP(hipHostMalloc(&k->h_host, sizeof(double) * 2 * HSLOT, hipHostMallocCoherent));
     TF_HIP(hipHostGetDevicePointer((void**)&k->h_host_dev, k->h_host, 0));
     TF_HIP(hipMalloc(&k->desc, sizeof(MatrixDesc)));
     TF_HIP(hipEventCreateWithFlags(&k->step_done, hipEventDisableTiming));
@@ -581,6 +692,7 @@ int tf_krylov_destroy(tf_krylov* k) {
     if (k->step2[j]) (void)hipGraphExecDestroy(k->step2[j]);
     if (k->step2_graph[j]) (void)hipGraphDestroy(k->step2_graph[j]);
   }
+  for (int w = 0; w < 2; ++w) drop_iterations(k, w);
   if (k->cap) (void)hipStreamDestroy(k->cap);
   if (k->step_done) (void)hipEventDestroy(k->step_done);
   for (void* p : {k->V, k->Z, k->w, (void*)k->h, (void*)k->y, (void*)k->work, (void*)k->desc}) (void)hipFree(p);

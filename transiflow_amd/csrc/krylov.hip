@@ -17,6 +17,10 @@
 #include <type_traits>
 #include <utility>
 
+namespace tf {
+bool cgs2_to_host(int n, int j);
+}
+
 namespace {
 
 constexpr int MD_THREADS = 256;
@@ -232,8 +236,8 @@ __device__ __forceinline__ void fin_sums(int k, int nb, const double* __restrict
 // (add: hout[i] += c[i]); w -= sum_i c[i] V[i]; then the block sums of the next
 // reduction, V^T w (self: w . w), into next.  A block updates the entries it then sums
 // (dot_body's chunk, and each thread the ones it reads), so the next reduction needs no
-// launch of its own: a step of the 64 x 64 grid is six dependent launches of 4 us
-// instead of eight, with the second reading of V from the L2.  blockIdx.y 1 takes the
+// launch of its own: a step of the 64 x 64 grid is five dependent launches of 4 us
+// instead of seven, with the second reading of V from the L2.  blockIdx.y 1 takes the
 // second system.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(MD_THREADS) void k_gram_schmidt(int n, int k, const T* V, long ldv,
@@ -268,8 +272,8 @@ __global__ __launch_bounds__(MD_THREADS) void k_gram_schmidt(int n, int k, const
 }
 
 // nrm = sqrt(sum of partial[0..nb)) (block 0 stores it in h[k]), out = w / nrm.
-// hhost (pinned host memory, or null): block 0 also writes the column h[0..k] there,
-// so the host reads it without a copy after the launch.
+// hhost (pinned, coherent host memory, or null): block 0 also writes the column h[0..k]
+// there and then sets hhost[HFLAG], so the host reads it without a copy or an event.
 template <typename T, bool VEC>
 __global__ __launch_bounds__(256) void k_scale_fin(int n, int nb, int k, const double* __restrict__ partial,
                                                    double* __restrict__ h, double* __restrict__ hhost,
@@ -294,6 +298,11 @@ __global__ __launch_bounds__(256) void k_scale_fin(int n, int nb, int k, const d
       // h[0..k) is final since the previous launch
       for (int i = threadIdx.x; i < k; i += blockDim.x) hhost[i] = h[i];
       if (threadIdx.x == 0) hhost[k] = nrm;
+      __threadfence_system();
+      __syncthreads();
+      if (threadIdx.x == 0)
+        __hip_atomic_store((unsigned long long*)(hhost + tf::HFLAG), 1ull, __ATOMIC_RELEASE,
+                           __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
   using VT = typename Vec16<T>::type;
@@ -541,8 +550,8 @@ __global__ void k_add_pair(int k, double* h0, const double* y0, double* h1, cons
 // four launches); else by separate kernels (k_multidot_final, k_add_pair,
 // k_norm_final: ten).  The choice depends on n and j only, so one system and
 // two systems take the same arithmetic.  hh0, hh1 (pinned host memory, or null):
-// on the four-launch path the last launch also writes each column h[0..j+1] there
-// (*to_host = 1); otherwise *to_host = 0 and the caller copies it.
+// on the four-launch path the last launch also writes each column h[0..j+1] there and
+// sets the word HFLAG (*to_host = 1); otherwise *to_host = 0 and the caller copies it.
 template <typename T>
 int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, double* work0, double* work1,
              double* h0, double* h1, double* y0, double* y1, T* v0, T* v1, double* hh0, double* hh1, int* to_host,
@@ -561,7 +570,7 @@ int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, dou
   }
   const int nb = md_blocks(n);
   const bool vec = vec_ok<T>(n, n, V0, w0) && vec_ok<T>(n, n, V1, w1) && vec_ok<T>(n, n, v0, v1);
-  const bool fused = (long)k * nb <= FIN_LDS;
+  const bool fused = tf::cgs2_to_host(n, j);
   const dim3 md(nb, nsys), blk(MD_THREADS), fin(k, nsys);
   const dim3 ew(grid_for(vec ? n / Vec16<T>::N : n), nsys);
   auto dots = [&](int kk, const T* A0, const T* A1) {
@@ -628,6 +637,8 @@ int cgs2_sys(int nsys, int n, int j, const T* V0, const T* V1, T* w0, T* w1, dou
 }  // namespace
 
 namespace tf {
+// Whether step j of n entries writes its column to the host itself.
+bool cgs2_to_host(int n, int j) { return (long)(j + 1) * md_blocks(n) <= FIN_LDS; }
 // One CGS2 Arnoldi orthogonalisation and normalisation (cgs2_sys) for two systems
 // in the same launches, or for one; the same arithmetic either way.
 int cgs2_pair_f64(int n, int j, const double* V0, const double* V1, double* w0, double* w1, double* work0,

@@ -43,6 +43,10 @@ __device__ __forceinline__ typename Global<T>::type* global_ptr(T* p) {
 }
 #endif
 
+// Word of a pinned Hessenberg column that the Arnoldi step sets once the column is there
+// (behind a column of the largest basis).
+constexpr int HFLAG = 264;
+
 // ---- opt-in kernel timing -------------------------------------------------
 // When enabled (tf_prof_enable), launches wrapped in TF_PROF_BEGIN/END record
 // a pair of HIP events on the launch stream; tf_prof_read() synchronises and
