@@ -241,10 +241,11 @@ __device__ __forceinline__ void invert64(T (&cur)[NS], T (&nxt)[NS], int& mystep
 // identity), into P_b (PB x PB; in place when Pb is null and k0 = 0): one block of 8 waves
 // per matrix.  The block
 // is held in LDS as 2 x 2 blocks of 64 and inverted by two Gauss-Jordan steps of width
-// 64 (invert64 each), their block products on the matrix cores.The block of 128 takes 68 us in
-// FP64 and 53 us in FP32, for one matrix or 128 (of it 2 x 21 and 2 x 16 us the
-// invert64 chains); the earlier panels of 64, in registers with the identity beside
-// them, LDS shuffles and the division on the chain, took 60 and 46 us each.
+// 64 (invert64 each), their block products on the matrix cores.  The block of 128 takes
+// 61 us in FP64 and 44 us in FP32, for one matrix or 128 (of it 2 x 21 and 2 x 16 us the
+// invert64 chains, 14 and 8 the products, which one CU's matrix units bound); the earlier
+// panels of 64, in registers with the identity beside them, LDS shuffles and the division
+// on the chain, took 60 and 46 us each.
 template <typename T>
 struct BlockLds {
   static constexpr int LD = PB + 1;  // a column of 64 rows meets every bank
@@ -267,10 +268,19 @@ __global__ __launch_bounds__(512) void k_gj_block(int m, int k0, int pb, T* cons
   const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
   const int lr = lane & 15, lk = lane >> 4;
   const int nb = pb > 64 ? 2 : 1;
-  for (int e = t; e < nb * 64 * PB; e += 512) {
-    const int r = e >> 7, c = e & 127;
-    if (c < nb * 64)
-      S[r * LD + c] = (r < pb && c < pb) ? X[(long)(k0 + r) * m + k0 + c] : (r == c ? (T)1 : (T)0);
+  // sixteen loads in flight a thread (one at a time, the loop took 6 us of the block's 65)
+  for (int q = 0; q < nb; ++q) {
+    T v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = q * 64 + (t >> 7) + 4 * i, c = t & 127;
+      v[i] = X[(long)(k0 + min(r, pb - 1)) * m + k0 + min(c, pb - 1)];
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = q * 64 + (t >> 7) + 4 * i, c = t & 127;
+      if (c < nb * 64) S[r * LD + c] = (r < pb && c < pb) ? v[i] : (r == c ? (T)1 : (T)0);
+    }
   }
   __syncthreads();
   // the 64 x 64 block at (o, o) <- its inverse
@@ -331,9 +341,15 @@ __global__ __launch_bounds__(512) void k_gj_block(int m, int k0, int pb, T* cons
     put(0, 64, w, (T)-1, (T)0);
     __syncthreads();
   }
-  for (int e = t; e < nb * 64 * PB; e += 512) {
-    const int r = e >> 7, c = e & 127;
-    if (r < pb && c < pb) P[(long)r * pp + c] = S[r * LD + c];
+  for (int q = 0; q < nb; ++q) {
+    T v[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = S[(q * 64 + (t >> 7) + 4 * i) * LD + (t & 127)];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int r = q * 64 + (t >> 7) + 4 * i, c = t & 127;
+      if (r < pb && c < pb) P[(long)r * pp + c] = v[i];
+    }
   }
 }
 
@@ -430,10 +446,10 @@ inline size_t scratch_P() { return (size_t)PB * PB; }
 inline size_t scratch_K(int m) { return (size_t)PB * m; }
 
 // X_b <- X_b^-1 for the matrices of a device pointer list.  Up to 128 rows: one launch;
-// otherwise three per panel of 128 columns.The
+// otherwise three per panel of 128 columns.  The
 // update reads and writes the whole matrix once per panel, and HBM bounds it: with
 // panels of 64 and separate copies and stores (five launches a panel) the 128 matrices
-// of 768 took 540 us per 64 columns in FP64, now 280 (update 366 us, rows 115, block 77
+// of 768 took 540 us per 64 columns in FP64, now 280 (update 366 us, rows 115, block 70
 // per 128 columns); one matrix of 768 takes 110 us per 128 columns (170).
 template <typename T>
 int invert(int m, T* const* Xp, int batch, const Scratch<T>& w, int* nperturb, double repl, hipStream_t st) {
