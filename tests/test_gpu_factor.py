@@ -47,3 +47,46 @@ def test_line_factor_applies_the_inverse(hip, problem, nx, single):
     tol = factor.m * cond * numpy.finfo(numpy.float32 if single else numpy.float64).eps
     print('%s m %d single %s: cond %.1e, error %.1e, bound %.1e' % (problem, factor.m, single, cond, err, tol), flush=True)
     assert err <= min(tol, 0.1)
+
+
+@pytest.mark.parametrize('shape', [(32, 24, 5), (64, 12, 3), (28, 28, 2), (56, 14, 4)])
+def test_chain_matches_reduction(hip, shape):
+    """Planes of 3072 rows and more, eliminated one after the other when the factor does
+    not keep Y L and Y U, against the reduction that does: the same inverse to rounding
+    (1e-10, as for the two forms of the reduction), the same bits for one column and two,
+    replayed and eager; a handle that is set back and forth before it is factored ends up
+    with the order of its last setting."""
+    import torch
+    from transiflow_amd.solver import LineFactor
+    itf = hip.Interface({'Reynolds Number': 100}, *shape)
+    g = itf.solver.gauge()
+    rng = numpy.random.default_rng(9)
+    J = itf.jacobian(itf.vector_from_array(rng.uniform(-1, 1, itf.n) * 0.1))
+    r = [torch.from_numpy(rng.uniform(-1, 1, itf.n)).cuda() for _ in range(2)]
+    for v in r:
+        v[g] = 0.0
+    out = {}
+    for order in ((True,), (False,), (True, False), (False, True)):
+        f = LineFactor(itf, J, g, single=False, factor=False)
+        for fused in order:
+            f.set_fused(fused)
+        f.refactor(J, g)
+        got = []
+        for graph in (False, True, True):
+            f.set_graph(graph)
+            z = [torch.full_like(v, numpy.nan) for v in r]
+            p = [torch.full_like(v, numpy.nan) for v in r]
+            for a, b in zip(r, z):
+                f.apply(a, b)
+            f.apply_pair(r[0], r[1], p[0], p[1], single=False)
+            torch.cuda.synchronize()
+            got.append([v.cpu().numpy() for v in z + p])
+        for zs in got:
+            for i in range(2):
+                assert numpy.isfinite(zs[i]).all()
+                assert numpy.array_equal(zs[i], got[0][i]) and numpy.array_equal(zs[2 + i], got[0][i])
+        out[order] = got[0][0]
+    diff = numpy.linalg.norm(out[(False,)] - out[(True,)]) / numpy.linalg.norm(out[(True,)])
+    assert diff <= 1e-10
+    assert numpy.array_equal(out[(True, False)], out[(False,)])
+    assert numpy.array_equal(out[(False, True)], out[(True,)])

@@ -1125,6 +1125,37 @@ struct LevelPlan {
   std::vector<int> k, k1, k2, kfa, kfb, kslot;
 };
 
+// Lines of CHAIN_M rows and more are eliminated one after the other (the chain) unless
+// the factor keeps Y L and Y U: the couplings then stay sparse, and a line costs one
+// inversion and its neighbour a sparse update, where the reduction multiplies five to six
+// dense blocks per line (32 against 122 products of 2 m^3 at 32 lines).  One such matrix
+// fills the device; shorter lines need the reduction's batches.  Factorisation and apply
+// in FP64, chain against reduction: 24^3 (2304 rows) 47.6 / 44.9 ms and 747 / 602 us,
+// 28^3 (3136 rows) 93 / 119 ms and 1246 / 1229 us, 32^3 165 / 264 ms and 1908 / 2221 us.
+// Long chains can round more than the reduction (2D grids of 48 lines up to a hundred
+// times more in FP32; planes of 3D grids as much, but for states of noise at Re 1000 up to
+// ten times): FP64 only, where the solves refine that away, and up to CHAIN_N lines.
+constexpr int CHAIN_M = 3072, CHAIN_N = 64;
+
+bool chain_pays(int m, int N, int single) { return !single && m >= CHAIN_M && N > 1 && N <= CHAIN_N; }
+
+std::vector<LevelPlan> chain_plan(int N) {
+  std::vector<LevelPlan> plan(N);
+  for (int j = 0; j < N; ++j) {
+    LevelPlan& L = plan[j];
+    const int next = j + 1 < N ? j + 1 : -1;
+    L.e = {j};
+    L.ea = {-1};
+    L.eb = {next};
+    if (next < 0) continue;
+    L.k = {next};
+    L.k1 = {j};
+    L.k2 = L.kfa = L.kfb = {-1};
+    L.kslot = {0};
+  }
+  return plan;
+}
+
 std::vector<LevelPlan> make_plan(int N) {
   // The last active line is always kept (it is eliminated alone at the final
   // level): with a no-slip lid its raw diagonal block carries the 1D pressure
@@ -1241,6 +1272,7 @@ struct tf_bcr {
   size_t slots;
   size_t solve_bytes_half;
   int split;           // level GEMMs of an FP32 factor on BF16 terms: 0 off, 1 or 3 terms
+  int chain;           // the lines one after the other (chain_plan): every level's couplings are the sparse ones
   int fused;           // L, U of the levels >= 1 hold Y L, Y U (one backward kernel per level)
   int use_top;         // the upper levels of the fused backward and their forward levels in one k_top launch
   int use_small;       // levels with at most SMALL_MAX lines through k_small (operands by value)
@@ -1359,7 +1391,7 @@ int factor_impl(tf_bcr* h, const int* rp, const int* ci, const double* v, int ga
     // 1. invert the eliminated lines' diagonal blocks in place
     if (int e = tf::gj::invert<T>(m, (T* const*)L.Ye, L.ne, w, h->flags + 1, 0.0, st)) return e;
     if (L.nk == 0) continue;
-    if (l == 0) {
+    if (l == 0 || h->chain) {
       level0<T>(h, L, st);
       continue;
     }
@@ -1552,14 +1584,15 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
   for (int l = 0; l < fwd_end; ++l) {
     const BcrLevelDev& L = h->lev[l];
     if (!L.nk) continue;
-    if (l == 0) {
+    if (l == 0 || h->chain) {
       // the level-0 couplings are sparse: y_e = Y_e r_e, then r_k -= L_k y_e1 + U_k y_e2
-      // (one Y block per eliminated line instead of two multipliers per kept line)
+      // (one Y block per eliminated line instead of two multipliers per kept line); a
+      // chain's kept line is the next one, still as given
       const int G = group_for(L.ne);
       with_rows(rows_for<B>(L.ne, m), [&](auto Rc) {
         constexpr int R = decltype(Rc)::value;
         hipLaunchKernelGGL((k_bwd_x<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, Yb(L),
-                           v.r, v.rs, yb, cs);
+                           l == 0 ? v.r : (const V*)rw, l == 0 ? v.rs : cs, yb, cs);
       });
       hipLaunchKernelGGL((k_fwd_sparse<V, NC>), dim3(gs, L.nk), blk, 0, st, m, L.k, L.k1, L.k2, h->Lr, h->nLr, h->Ur,
                          h->nUr, (const V*)yb, v.r, v.rs, rw, cs);
@@ -1600,9 +1633,9 @@ void sweep(tf_bcr* h, int vec, B P1(const BcrLevelDev&), B P2(const BcrLevelDev&
                            Yb(L), Lb(L), Ub(L), (const V*)rw, cs, xo, xs);
         return;
       }
-      if (l == 0)
+      if (l == 0 || h->chain)
         hipLaunchKernelGGL((k_bwd_t_sparse<V, NC>), dim3(gs, L.ne), blk, 0, st, m, L.e, L.ea, L.eb, h->Lr, h->nLr,
-                           h->Ur, h->nUr, v.r, v.rs, (const V*)xo, xs, tb, cs);
+                           h->Ur, h->nUr, l == 0 ? v.r : (const V*)rw, l == 0 ? v.rs : cs, (const V*)xo, xs, tb, cs);
       else
         hipLaunchKernelGGL((k_bwd_t<B, V, NC, R>), dim3(gx(G, R), L.ne), blk, 0, st, m, G, vec, L.e, L.ea, L.eb, Lb(L),
                            Ub(L), (const V*)rw, (const V*)xo, tb, cs, xs);
@@ -1800,6 +1833,7 @@ int solve_graph(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream
 
 template <typename V, int NC>
 int solve_any(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream_t st) {
+  if (h->lev.empty()) return tf::fail("tf_bcr_solve: the handle was lost to a failed allocation");
   if (h->use_graph)
     return h->single ? solve_graph<float, V, NC>(h, r, x, st) : solve_graph<double, V, NC>(h, r, x, st);
   return h->single ? solve_impl<float, V, NC>(h, r, x, st) : solve_impl<double, V, NC>(h, r, x, st);
@@ -1812,7 +1846,7 @@ namespace tf {
 // applies are to be replayed, and the number under which that stays the same apply.
 bool bcr_replays(const tf_bcr* h, unsigned long long* gen) {
   *gen = h->gen;
-  return h->use_graph != 0;
+  return h->use_graph != 0 && !h->lev.empty();
 }
 // the launches of one apply of nc (1 or 2) columns (single: FP32 vectors)
 int bcr_apply(tf_bcr* h, int single, int nc, const void* r0, const void* r1, void* x0, void* x1, hipStream_t st) {
@@ -1862,7 +1896,9 @@ extern "C" {
 // ylines != 0 (2D only): lines are the grid columns i (m = ny dof rows each, nx
 // lines) instead of the rows j; n = nx ny dof.
 int tf_bcr_destroy(tf_bcr* h);
-static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines);
+static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines, bool chain);
+int tf_bcr_set_dense_top(tf_bcr* h, int lines);
+int tf_bcr_set_half(tf_bcr* h, int on, void* stream);
 
 int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines) {
   if (!out) return tf::fail("null handle");
@@ -1872,7 +1908,7 @@ int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int y
     return tf::fail("y-line order needs n = nx * m with m = ny * dof");
   tf_bcr* h = new tf_bcr();
   h->gen = new_gen();
-  const int rc = bcr_create_impl(h, n, m, single, nx, dof, ylines);
+  const int rc = bcr_create_impl(h, n, m, single, nx, dof, ylines, chain_pays(m, n / m, single));
   if (rc) {
     // frees whatever was allocated before the failure (unset members are null)
     tf_bcr_destroy(h);
@@ -1882,7 +1918,39 @@ int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int y
   return 0;
 }
 
-static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines) {
+// everything the handle owns
+static void bcr_release(tf_bcr* h) {
+  for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
+    if (g->exec) (void)hipGraphExecDestroy(g->exec);
+    if (g->graph) (void)hipGraphDestroy(g->graph);
+  }
+  if (h->cap) (void)hipStreamDestroy(h->cap);
+  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
+                  (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
+                  (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
+                  (void*)h->topsync, h->Z, h->zpool, h->xtab})
+    (void)hipFree(p);
+  (void)hipHostFree(h->host_flags);
+}
+
+// An unfactored handle made again with the other elimination order, its settings kept.
+static int bcr_rebuild(tf_bcr* h, bool chain) {
+  const tf_bcr old = *h;
+  bcr_release(h);
+  *h = tf_bcr{};
+  h->gen = new_gen();
+  const Order& o = old.order;
+  if (int e = bcr_create_impl(h, old.n, old.m, old.single, o.nx, o.dof, o.ylines, chain)) return e;
+  h->use_graph = old.use_graph;
+  h->use_small = old.use_small;
+  h->split = old.split;
+  h->fused = old.fused;
+  if (old.zmax)
+    if (int e = tf_bcr_set_dense_top(h, old.zmax)) return e;
+  return old.half ? tf_bcr_set_half(h, 1, nullptr) : 0;
+}
+
+static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines, bool chain) {
   h->order = Order{ylines ? 1 : 0, nx, dof, m};
   h->n = n;
   h->m = m;
@@ -1890,19 +1958,22 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   h->single = single;
   h->es = single ? sizeof(float) : sizeof(double);
   const size_t mm = (size_t)m * m, N = h->N;
-  const size_t maxb = (N + 1) / 2;
+  h->chain = chain ? 1 : 0;
+  const size_t maxb = chain ? 1 : (N + 1) / 2;
   TF_HIP(hipMalloc(&h->D, h->es * mm * N));
-  TF_HIP(hipMalloc(&h->Lm, h->es * mm * N));
-  TF_HIP(hipMalloc(&h->Um, h->es * mm * N));
+  if (!chain) {
+    TF_HIP(hipMalloc(&h->Lm, h->es * mm * N));
+    TF_HIP(hipMalloc(&h->Um, h->es * mm * N));
+  }
   // one multiplier pair per kept line per level (more than N - 1 when the
   // active count is odd at some level)
-  h->plan = make_plan(h->N);
+  h->plan = chain ? chain_plan(h->N) : make_plan(h->N);
   size_t slots = 0;
   for (const LevelPlan& L : h->plan) slots += L.k.size();
-  if (slots < 1) slots = 1;
+  if (slots < 1 || chain) slots = 1;  // a chain's multiplier is used at once
   h->slots = slots;
   TF_HIP(hipMalloc(&h->P1, h->es * mm * slots));
-  TF_HIP(hipMalloc(&h->P2, h->es * mm * slots));
+  if (!chain) TF_HIP(hipMalloc(&h->P2, h->es * mm * slots));
   TF_HIP(hipMalloc(&h->Pinv, h->es * tf::gj::scratch_P() * maxb));
   TF_HIP(hipMalloc(&h->Kc, h->es * tf::gj::scratch_K(m) * maxb));
   TF_HIP(hipMalloc(&h->Tb, h->es * tf::gj::scratch_K(m) * maxb));
@@ -1932,7 +2003,7 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   char* P1 = (char*)h->P1;
   char* P2 = (char*)h->P2;
   const size_t bm = h->es * mm;
-  auto blk = [&](char* base, int j) -> void* { return (void*)(base + bm * (size_t)j); };
+  auto blk = [&](char* base, int j) -> void* { return base ? (void*)(base + bm * (size_t)j) : nullptr; };
   PoolBuilder pb;
   struct Off {
     size_t e, ea, eb, Ye, Le, Ue, k, k1, k2, P1, P2, pA, pB, pC, dA1, dB1, dA2, dB2, dC, d1A, d2A, fA, fB, fC, zY1, zY2, zL, zU, zfa, zfb, hase1, hase2, faline, fbline, ylA, ylB, ylC, yuA, yuB, yuC;
@@ -1941,7 +2012,7 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   std::vector<Off> offs;
   // scratch of the fused products: the largest batch of one level (levels >= 1)
   size_t wslots = 0;
-  for (size_t l = 1; l < h->plan.size(); ++l) {
+  for (size_t l = 1; l < h->plan.size() && !chain; ++l) {
     size_t na = 0, nb = 0;
     for (size_t b = 0; b < h->plan[l].e.size(); ++b) {
       na += h->plan[l].ea[b] >= 0;
@@ -2051,7 +2122,7 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
     o.zfb = pb.add_ints(zfb);
     // fused products Y_e L_e, Y_e U_e of the eliminated lines at levels >= 1 (W: scratch slots)
     std::vector<void*> ylA, ylB, ylC, yuA, yuB, yuC;
-    if (l_index > 0) {
+    if (l_index > 0 && !chain) {
       for (int b = 0; b < o.ne; ++b) {
         const int e = L.e[b];
         if (L.ea[b] >= 0) {
@@ -2085,7 +2156,7 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
     for (size_t l = 0; l < h->plan.size(); ++l) {
       const LevelPlan& L = h->plan[l];
       blocks += L.e.size();
-      if (l > 0) {
+      if (l > 0 && !chain) {
         for (size_t b = 0; b < L.e.size(); ++b) blocks += (L.ea[b] >= 0) + (L.eb[b] >= 0);
         for (size_t b = 0; b < L.k.size(); ++b) blocks += (L.k1[b] >= 0) + (L.k2[b] >= 0);
       } else if (!L.k.empty()) {
@@ -2159,17 +2230,7 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
 
 int tf_bcr_destroy(tf_bcr* h) {
   if (!h) return 0;
-  for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
-    if (g->exec) (void)hipGraphExecDestroy(g->exec);
-    if (g->graph) (void)hipGraphDestroy(g->graph);
-  }
-  if (h->cap) (void)hipStreamDestroy(h->cap);
-  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
-                  (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
-                  (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
-                  (void*)h->topsync, h->Z, h->zpool, h->xtab})
-    (void)hipFree(p);
-  (void)hipHostFree(h->host_flags);
+  bcr_release(h);
   delete h;
   return 0;
 }
@@ -2177,6 +2238,7 @@ int tf_bcr_destroy(tf_bcr* h) {
 // Factor the gauged matrix (CSR, gauge row or -1).  Asynchronous on ``stream``.
 int tf_bcr_factor(tf_bcr* h, const int* rp, const int* ci, const double* v, int gauge, void* stream) {
   if (!h) return tf::fail("null handle");
+  if (h->lev.empty()) return tf::fail("tf_bcr_factor: the handle was lost to a failed allocation");
   hipStream_t st = (hipStream_t)stream;
   return h->single ? factor_impl<float>(h, rp, ci, v, gauge, st) : factor_impl<double>(h, rp, ci, v, gauge, st);
 }
@@ -2256,8 +2318,9 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
   if (on && !h->H) {
     // all three allocations succeed before any is kept (a failed call leaves no copies)
     void *H_ = nullptr, *S_ = nullptr;
-    hipError_t e = hipMalloc(&H_, sizeof(f16) * mm * (3 * N + 2 * slots));
-    if (e == hipSuccess) e = hipMalloc(&S_, sizeof(float) * (size_t)m * (3 * N + 2 * slots));
+    const size_t copies = h->chain ? N : 3 * N + 2 * slots;  // (a chain reads D only)
+    hipError_t e = hipMalloc(&H_, sizeof(f16) * mm * copies);
+    if (e == hipSuccess) e = hipMalloc(&S_, sizeof(float) * (size_t)m * copies);
     if (e != hipSuccess) {
       (void)hipFree(H_);
       (void)hipFree(S_);
@@ -2299,8 +2362,8 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
         uh.push_back(hb(2, e));
         us.push_back(sb(2, e));
         conv(0, e);
-        if (l > 0 && L.ea[b] >= 0) conv(1, e);
-        if (l > 0 && L.eb[b] >= 0) conv(2, e);
+        if (l > 0 && !h->chain && L.ea[b] >= 0) conv(1, e);
+        if (l > 0 && !h->chain && L.eb[b] >= 0) conv(2, e);
       }
       for (size_t b = 0; b < L.k.size(); ++b) {
         const int sl = L.kslot[b];
@@ -2309,8 +2372,8 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
         p2h.push_back(hb(4, sl));
         p2s.push_back(sb(4, sl));
         // (level 0 applies its multipliers through Y and the sparse couplings)
-        if (l > 0 && L.k1[b] >= 0) conv(3, sl);
-        if (l > 0 && L.k2[b] >= 0) conv(4, sl);
+        if (l > 0 && !h->chain && L.k1[b] >= 0) conv(3, sl);
+        if (l > 0 && !h->chain && L.k2[b] >= 0) conv(4, sl);
       }
       HOff o;
       o.Yh = pb.add_ptrs(yh);
@@ -2388,7 +2451,13 @@ int tf_bcr_set_fused(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
   if (h->factored && (on != 0) != (h->fused != 0))
     return tf::fail("tf_bcr_set_fused: the handle already holds a factor of the other form");
-  if ((on != 0) != (h->fused != 0)) drop_graphs(h);
+  if ((on != 0) != (h->fused != 0)) {
+    drop_graphs(h);
+    h->fused = on ? 1 : 0;
+    const bool chain = !on && chain_pays(h->m, h->N, h->single);
+    if (chain != (h->chain != 0))
+      if (int e = bcr_rebuild(h, chain)) return e;
+  }
   h->fused = on ? 1 : 0;
   return 0;
 }
