@@ -90,3 +90,38 @@ def test_chain_matches_reduction(hip, shape):
     assert diff <= 1e-10
     assert numpy.array_equal(out[(True, False)], out[(False,)])
     assert numpy.array_equal(out[(False, True)], out[(True,)])
+
+
+@pytest.mark.parametrize('shape,single', [((32, 24, 5), False), ((56, 14, 4), True), ((40, 20, 9), True),
+                                          ((40, 20, 9), False)])
+def test_look_ahead_keeps_the_bits(hip, shape, single):
+    """Inversions whose next diagonal block is updated and inverted beside the rest of the
+    update (3072 and 3136 rows, the last panel half filled; 3200 rows with a batch of up to
+    five), against the same launches one after the other, which the kernel profiler asks
+    for: the same bits, also from a factor made twice."""
+    import torch
+    from transiflow_amd import _lib
+    from transiflow_amd.solver import LineFactor
+    itf = hip.Interface({'Reynolds Number': 100}, *shape)
+    g = itf.solver.gauge()
+    rng = numpy.random.default_rng(10)
+    J = itf.jacobian(itf.vector_from_array(rng.uniform(-1, 1, itf.n) * 0.1))
+    r = torch.from_numpy(rng.uniform(-1, 1, itf.n)).cuda()
+    r[g] = 0.0
+    r = r.float() if single else r
+    out = []
+    f = LineFactor(itf, J, g, single=single, factor=False)
+    f.set_fused(True)
+    f.set_graph(False)
+    for prof in (1, 0, 0):
+        _lib.call('tf_prof_enable', prof)
+        try:
+            f.refactor(J, g)
+        finally:
+            _lib.call('tf_prof_enable', 0)
+        z = torch.empty_like(r)
+        (f.apply32 if single else f.apply)(r, z)
+        torch.cuda.synchronize()
+        out.append(z.cpu().numpy())
+    assert numpy.isfinite(out[0]).all()
+    assert numpy.array_equal(out[1], out[0]) and numpy.array_equal(out[2], out[0])

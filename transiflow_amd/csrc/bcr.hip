@@ -1250,6 +1250,8 @@ struct tf_bcr {
   void* P1;   // slots m^2 (one per kept line per level)
   void* P2;   // slots m^2
   void *Pinv, *Kc, *Tb;  // scratch of the inversions (gj.h), largest level
+  void* Nx;              // ... of those that look ahead (null: none does)
+  tf::gj::Side side;
   Cpl *Lr, *Ur, *Ut, *Lt;
   int *nLr, *nUr, *nUt, *nLt;
   int* flags;  // [err, nperturb]
@@ -1385,7 +1387,7 @@ int factor_impl(tf_bcr* h, const int* rp, const int* ci, const double* v, int ga
   hipLaunchKernelGGL(k_sort_cols, dim3((n + 255) / 256), dim3(256), 0, st, n, h->Ut, h->nUt);
   hipLaunchKernelGGL(k_sort_cols, dim3((n + 255) / 256), dim3(256), 0, st, n, h->Lt, h->nLt);
   hipLaunchKernelGGL(k_diag_blocks<T>, dim3(m, N), dim3(256), 0, st, m, h->order, rp, ci, v, gauge, (T*)h->D);
-  const tf::gj::Scratch<T> w{(T*)h->Pinv, (T*)h->Kc, (T*)h->Tb};
+  const tf::gj::Scratch<T> w{(T*)h->Pinv, (T*)h->Kc, (T*)h->Tb, (T*)h->Nx, &h->side};
   for (size_t l = 0; l < h->lev.size(); ++l) {
     BcrLevelDev& L = h->lev[l];
     // 1. invert the eliminated lines' diagonal blocks in place
@@ -1928,9 +1930,10 @@ static void bcr_release(tf_bcr* h) {
   for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
                   (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
                   (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
-                  (void*)h->topsync, h->Z, h->zpool, h->xtab})
+                  (void*)h->topsync, h->Z, h->zpool, h->xtab, h->Nx})
     (void)hipFree(p);
   (void)hipHostFree(h->host_flags);
+  h->side.release();
 }
 
 // An unfactored handle made again with the other elimination order, its settings kept.
@@ -1977,6 +1980,10 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   TF_HIP(hipMalloc(&h->Pinv, h->es * tf::gj::scratch_P() * maxb));
   TF_HIP(hipMalloc(&h->Kc, h->es * tf::gj::scratch_K(m) * maxb));
   TF_HIP(hipMalloc(&h->Tb, h->es * tf::gj::scratch_K(m) * maxb));
+  size_t ahead = 0;
+  for (const LevelPlan& L : h->plan)
+    if (tf::gj::look_ahead(m, (int)L.e.size(), h->es)) ahead = std::max(ahead, L.e.size());
+  if (ahead) TF_HIP(hipMalloc(&h->Nx, h->es * tf::gj::scratch_P() * ahead));
   for (Cpl** c : {&h->Lr, &h->Ur, &h->Ut, &h->Lt}) TF_HIP(hipMalloc(c, sizeof(Cpl) * KC * (size_t)n));
   for (int** c : {&h->nLr, &h->nUr, &h->nUt, &h->nLt}) TF_HIP(hipMalloc(c, sizeof(int) * (size_t)n));
   TF_HIP(hipMalloc(&h->flags, sizeof(int) * 2));
