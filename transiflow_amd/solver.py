@@ -71,7 +71,8 @@ Options (``parameters['HIP Solver']``, all optional):
                        scaled from 'Inner Tolerance' to 'Tolerance' (30 by
                        default) or does not converge;
 ``'Fused Apply'``      (line factor) True or False (default: True for a factor
-                       that is reused -- mixed, or 'Reuse Factor' -- else
+                       that is reused -- mixed, or 'Reuse Factor' -- and whose
+                       lines or planes have less than 3072 rows, else
                        False): the factorisation also forms Y L and Y U so
                        that each backward level of the apply is one kernel;
 ``'Dense Top'``        (line factor with 'Fused Apply') 0 (default), 2, 3 or 4:
@@ -153,12 +154,24 @@ def _opts(parameters):
 _SPLITS = {'fp32': 0, 'bf16x3': 3, 'bf16': 1}
 
 
-def _fused_apply(opts, single):
+# Rows per line from which a reused factor is made without Y L and Y U by default.  The
+# two more products per line grow with the cube of the rows and save one launch per level
+# and apply: FP32 factor and two-column FP16 apply with and without, 24^3 (2304 rows) 29.8
+# / 25.7 ms and 252 / 270 us (even after 230 applies), 28^3 (3136) 77.7 / 65.0 ms and 465 /
+# 479 us (900), 32^3 (4096) 173.9 / 145.3 ms and 714 / 731 us (1700).  In FP64 the lines
+# are then eliminated one after the other: 32^3 315.5 / 141.6 ms and 2345 / 2194 us.
+FUSED_ROWS = 3072
+
+
+def _fused_apply(opts, single, m):
     """One-kernel backward levels (two more GEMMs per line at factor time) pay for a
     factor applied many times: the lagged factor of the mixed or factor-reusing
-    solves; a factor made for every Jacobian is applied only a few times."""
+    solves, unless its lines are long; a factor made for every Jacobian is applied only
+    a few times.  (The dense top is made from those products.)"""
     o = opts['Fused Apply']
-    return (single or opts['Reuse Factor']) if o is None else bool(o)
+    if o is not None:
+        return bool(o)
+    return bool(single or opts['Reuse Factor']) and (m < FUSED_ROWS or bool(opts['Dense Top']))
 
 
 def _dense_top(opts, fused):
@@ -171,7 +184,7 @@ def _dense_top(opts, fused):
 
 def _configure_line(f, opts, single):
     """Backward form and dense top of a line factor (before its first factorisation)."""
-    fused = _fused_apply(opts, single)
+    fused = _fused_apply(opts, single, f.m)
     f.set_fused(fused)
     f.set_dense_top(_dense_top(opts, fused))
 
