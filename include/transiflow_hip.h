@@ -67,8 +67,11 @@ int tf_rhs(tf_problem* p, const double* state, double* F, void* stream);
  * Discretization.py:392-415,474-524, CrsMatrix.py:52-71; SciPy.Interface.jacobian, SciPy.py:43-45).
  * count: row_ptr[0..n] is filled by the fill pass except row_ptr[n] = nnz,
  * which count writes; nnz_host (optional) receives nnz after a stream sync.
+ * count_copy: the same, and copy[0..n) = state in the same launch (not overlapping state; may be null).
  * fill: writes row_ptr[0..n-1], col[0..nnz), val[0..nnz). */
 int tf_jacobian_count(tf_problem* p, const double* state, int* row_ptr, int* nnz_host, void* stream);
+int tf_jacobian_count_copy(tf_problem* p, const double* state, double* copy, int* row_ptr, int* nnz_host,
+                           void* stream);
 int tf_jacobian_fill(tf_problem* p, const double* state, int* row_ptr, int* col, double* val,
                      void* stream);
 

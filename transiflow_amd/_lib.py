@@ -33,6 +33,7 @@ SIGNATURES = {
     'tf_problem_rows': (_c_int, [_vp]),
     'tf_rhs': (_c_int, [_vp, _vp, _vp, _vp]),
     'tf_jacobian_count': (_c_int, [_vp, _vp, _vp, _ip, _vp]),
+    'tf_jacobian_count_copy': (_c_int, [_vp, _vp, _vp, _vp, _ip, _vp]),
     'tf_jacobian_fill': (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp]),
     'tf_mass_count': (_c_int, [_vp, _vp, _ip, _vp]),
     'tf_mass_fill': (_c_int, [_vp, _vp, _vp, _vp, _vp]),

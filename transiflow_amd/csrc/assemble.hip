@@ -125,6 +125,7 @@ __global__ __launch_bounds__(64 * DOF) void k_assemble(Grid g, Physics ph, const
   } else if constexpr (MODE == MODE_COUNT) {
     int cnt = active ? dispatch_row<DIM, DOF, BUOY, MODE>(d1, c, ph, row, nullptr, nullptr, nullptr, 0) : 0;
     if (active) counts[row] = cnt;
+    if (F && active) F[row] = state[row];  // the caller's copy of the state
     const int sum = block_inclusive_scan<NT>(cnt, t);
     if (t == NT - 1) block_sums[blockIdx.x] = sum;
   } else {
@@ -373,9 +374,14 @@ int tf_rhs(tf_problem* p, const double* state, double* F, void* stream) {
 }
 
 int tf_jacobian_count(tf_problem* p, const double* state, int* row_ptr, int* nnz_host, void* stream) {
+  return tf_jacobian_count_copy(p, state, nullptr, row_ptr, nnz_host, stream);
+}
+
+int tf_jacobian_count_copy(tf_problem* p, const double* state, double* copy, int* row_ptr, int* nnz_host,
+                           void* stream) {
   if (!p || !state || !row_ptr) return fail("null argument");
   hipStream_t st = (hipStream_t)stream;
-  int rc = launch_assemble<MODE_COUNT>(p, state, nullptr, row_ptr, nullptr, nullptr, st);
+  int rc = launch_assemble<MODE_COUNT>(p, state, copy, row_ptr, nullptr, nullptr, st);
   if (rc) return rc;
   rc = scan_blocks(p, row_ptr, st);
   if (rc) return rc;

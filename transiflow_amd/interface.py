@@ -142,14 +142,16 @@ class Interface:
         x = self._device(state)
         row_ptr = T.empty(self.n + 1, dtype=T.int32, device='cuda')
         nnz = ctypes.c_int()
-        _lib.call('tf_jacobian_count', self._handle, ptr(x.data), ptr(row_ptr), ctypes.byref(nnz), stream())
+        # where the Jacobian is taken: the two-grid preconditioner re-assembles it on the
+        # coarse grid at the restricted state with the same parameters
+        state = T.empty(self.n, dtype=T.float64, device='cuda')
+        _lib.call('tf_jacobian_count_copy', self._handle, ptr(x.data), ptr(state), ptr(row_ptr), ctypes.byref(nnz),
+                  stream())
         col = T.empty(max(nnz.value, 1), dtype=T.int32, device='cuda')[:nnz.value]
         val = T.empty(max(nnz.value, 1), dtype=T.float64, device='cuda')[:nnz.value]
         _lib.call('tf_jacobian_fill', self._handle, ptr(x.data), ptr(row_ptr), ptr(col), ptr(val), stream())
         J = DeviceCsrMatrix(row_ptr, col, val, self.n)
-        # where the Jacobian was taken: the two-grid preconditioner re-assembles it
-        # on the coarse grid at the restricted state with the same parameters
-        J.state = x.data.clone()
+        J.state = state
         J.parameters = dict(self.parameters)
         return J
 
