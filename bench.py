@@ -293,8 +293,8 @@ def assembly_roofline(tf, torch, itf, x, reps=20):
 
 # profiled kernels: id -> (kernel name(s) as rocprofv3 lists them, bound, unit of the work figure)
 PROFILED = {
-    5: ('k_gemm_mfma', 'mfma', 'flop'),
-    3: ('k_panel', 'mfma', 'flop'),
+    5: ('k_gemm_mfma (with k_gj_rows and k_gj_update)', 'mfma', 'flop'),
+    3: ('k_gj_block', 'mfma', 'flop'),
     9: ('line-factor apply (k_stage_in, k_bwd_x, k_fwd_sparse, k_fwd, k_small, k_bwd_fused, k_bwd_t_sparse, k_stage_out_tab)',
         'hbm', 'byte'),
     10: ('two-column line-factor apply (k_stage_in, k_bwd_x, k_fwd_sparse, k_fwd, k_small, k_bwd_fused, k_bwd_t_sparse, k_stage_out_tab; NC=2)',

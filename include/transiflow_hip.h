@@ -315,8 +315,9 @@ int tf_adam(long n, float* w, const float* g, float* m, float* v, float lr, floa
 int tf_to_bf16(long n, const float* x, float scale, void* y, void* stream);
 
 /* ---- tile autotuner of the batched MFMA GEMM (no reference counterpart) ----
- * mode 1 (default): the first GEMM of each (type, M, N, K, batch) times the tile
- * candidates and keeps the fastest; mode 0: fixed rule.  tf_gemm_table copies rows
+ * mode 1 (default): the first GEMM of each (type, M, N, K, batch) between 256 tiles of
+ * 64 x 64 and 2048 of 128 x 128 times the tile candidates and keeps the fastest (fewer
+ * and more tiles: by rule); mode 0: fixed rule.  tf_gemm_table copies rows
  * (single, M, N, K, batch, tile) and returns the row count. */
 int tf_gemm_tuning(int mode);
 int tf_gemm_table(int* out_host, int max_rows);
