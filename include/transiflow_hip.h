@@ -178,7 +178,9 @@ int tf_krylov_create(tf_krylov** out, int n, int restart, int single);
 int tf_krylov_destroy(tf_krylov* k);
 /* on != 0 (the default): each Arnoldi step (SpMV through a device matrix descriptor, two
  * CGS passes, normalisation, the read-back of the Hessenberg column) is captured once per
- * basis index into a hipGraph and replayed; 0: the same launches are issued one by one. */
+ * basis index into a hipGraph and replayed, with a tf_bcr that replays its applies too
+ * (tf_bcr_set_graph) the whole iteration, apply and step, on the third use of a basis
+ * index; 0: the same launches are issued one by one. */
 int tf_krylov_set_graph(tf_krylov* k, int on);
 int tf_fgmres(tf_krylov* k, const int* row_ptr, const int* col, const void* val, int gauge, int prec_kind,
               void* prec, int ncell, int dof, const void* b, void* x, double tol, int maxit, int x_is_zero,
@@ -214,7 +216,9 @@ int tf_linelu_solve_f32(tf_linelu* h, const float* r, float* x, void* stream);
  * Odd-even reduction of the block-tridiagonal gauged Jacobian; every level is a batch of
  * dense inversions and GEMMs.  single != 0 factors and stores in FP32.  ylines != 0 (2D)
  * takes the grid columns as lines (m = ny*dof; nx and dof describe the grid) so that wide
- * domains factor short lines; vectors stay in the natural order. */
+ * domains factor short lines; vectors stay in the natural order.  In FP64 up to 64 lines of
+ * 3072 rows and more are eliminated one after the other instead, with sparse couplings
+ * throughout, unless tf_bcr_set_fused asks for the reduction's products. */
 typedef struct tf_bcr tf_bcr;
 int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines);
 int tf_bcr_destroy(tf_bcr* h);
@@ -257,7 +261,8 @@ int tf_bcr_set_gemm_split(tf_bcr* h, int split);
 /* on != 0 (before the first factorisation): the factorisation also forms Y L and Y U of the
  * lines eliminated at levels >= 1 in place of their L and U, and each backward level of the apply
  * is one kernel (x_e = Y r_e - (Y L) x_a - (Y U) x_b) instead of two (no reference counterpart:
- * worth it for factors applied many times, such as the lagged FP32 factor of the mixed solver). */
+ * worth it for factors applied many times, such as the lagged FP32 factor of the mixed solver).
+ * May allocate: a handle made for the other elimination order is made again. */
 int tf_bcr_set_fused(tf_bcr* h, int on);
 /* lines in 2..4 (fused factors): once the reduction is down to at most that many lines, each
  * factorisation also forms the dense inverse Z of their reduced system (about 20 m x m x m

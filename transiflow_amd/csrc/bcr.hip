@@ -20,7 +20,10 @@
 // per kept line -- so the sequential depth is (levels x panels), about 100 for
 // 256 lines, instead of (lines x panels) for the Thomas recursion.  At level
 // 0 the couplings are the sparse CSR entries (a few per row), so the level-0
-// products are sparse-dense and cost O(m^2).  The factor (Y, P1, P2, L, U) is
+// products are sparse-dense and cost O(m^2).
+// Long FP64 lines without the fused backward are taken in order instead (chain_plan):
+// each level eliminates one line, and every level's couplings are the sparse ones.
+// The factor (Y, P1, P2, L, U) is
 // kept in the storage type T (double, or float for the mixed-precision
 // variant, whose factorisation also runs in FP32).  For the FP32 apply of that
 // variant the blocks can also be copied to FP16 with one FP32 scale per row

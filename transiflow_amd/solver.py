@@ -37,7 +37,8 @@ Options (``parameters['HIP Solver']``, all optional):
                        (True);
 ``'Step Graphs'``      replay each native FGMRES Arnoldi step (SpMV, two CGS
                        passes, normalisation) as one captured hipGraph (True)
-                       or launch its kernels one by one;
+                       or launch its kernels one by one; with 'Apply Graph'
+                       the apply and the step of an iteration are one graph;
 ``'Pair Solves'``      (True) ``solve_pair`` -- the two solves of a Newton-
                        corrector iteration -- runs both in lockstep with one
                        pass over the line factor per application for both;
