@@ -216,11 +216,14 @@ int tf_linelu_solve_f32(tf_linelu* h, const float* r, float* x, void* stream);
  * Odd-even reduction of the block-tridiagonal gauged Jacobian; every level is a batch of
  * dense inversions and GEMMs.  single != 0 factors and stores in FP32.  ylines != 0 (2D)
  * takes the grid columns as lines (m = ny*dof; nx and dof describe the grid) so that wide
- * domains factor short lines; vectors stay in the natural order.  In FP64 up to 64 lines of
- * 3072 rows and more are eliminated one after the other instead, with sparse couplings
- * throughout, unless tf_bcr_set_fused asks for the reduction's products. */
+ * domains factor short lines; vectors stay in the natural order.
+ * create_inner: for an apply that is one step inside a preconditioner (the coarse solve of
+ * the two-grid method).  In FP64 up to 64 lines of 3072 rows and more are then eliminated
+ * one after the other, with sparse couplings throughout: cheaper, a fifth of the memory,
+ * and with larger rounding errors where convection dominates.  No tf_bcr_set_fused there. */
 typedef struct tf_bcr tf_bcr;
 int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines);
+int tf_bcr_create_inner(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines);
 int tf_bcr_destroy(tf_bcr* h);
 int tf_bcr_factor(tf_bcr* h, const int* row_ptr, const int* col, const double* val, int gauge, void* stream);
 int tf_bcr_status(tf_bcr* h, int* flags_host, void* stream);
@@ -261,8 +264,7 @@ int tf_bcr_set_gemm_split(tf_bcr* h, int split);
 /* on != 0 (before the first factorisation): the factorisation also forms Y L and Y U of the
  * lines eliminated at levels >= 1 in place of their L and U, and each backward level of the apply
  * is one kernel (x_e = Y r_e - (Y L) x_a - (Y U) x_b) instead of two (no reference counterpart:
- * worth it for factors applied many times, such as the lagged FP32 factor of the mixed solver).
- * May allocate: a handle made for the other elimination order is made again. */
+ * worth it for factors applied many times, such as the lagged FP32 factor of the mixed solver). */
 int tf_bcr_set_fused(tf_bcr* h, int on);
 /* lines in 2..4 (fused factors): once the reduction is down to at most that many lines, each
  * factorisation also forms the dense inverse Z of their reduced system (about 20 m x m x m

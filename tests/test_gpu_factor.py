@@ -125,3 +125,110 @@ def test_look_ahead_keeps_the_bits(hip, shape, single):
         out.append(z.cpu().numpy())
     assert numpy.isfinite(out[0]).all()
     assert numpy.array_equal(out[1], out[0]) and numpy.array_equal(out[2], out[0])
+
+
+def _flow(itf, seed):
+    """A flow-like state: a few smooth modes per unknown, velocities zero at the walls,
+    and noise a thousandth as large."""
+    rng = numpy.random.default_rng(seed)
+    at = [(numpy.arange(n) + 0.5) / n for n in (itf.nx, itf.ny, itf.nz)]
+    x = numpy.zeros((itf.nz, itf.ny, itf.nx, itf.dof))
+    for d in range(itf.dof):
+        field = 0.0
+        for _ in range(4):
+            term = [numpy.cos(numpy.pi * rng.integers(0, 4) * p) * (numpy.sin(numpy.pi * p) if d < 3 else 1.0)
+                    for p in at]
+            field = field + rng.standard_normal() * numpy.einsum('i,j,k->kji', *term)
+        x[..., d] = field / numpy.abs(field).max() * (0.4 if d < 3 else 0.2)
+    x += 1e-3 * rng.standard_normal(x.shape)
+    x[:, :, -1, 0] = x[:, -1, :, 1] = x[-1, :, :, 2] = 0.0
+    return x.reshape(-1)
+
+
+@pytest.mark.parametrize('shape,re', [((31, 31, 26), 340.0), ((29, 29, 18), 440.0), ((30, 30, 31), 460.0),
+                                      ((31, 30, 32), 480.0)])
+def test_direct_factor_of_long_lines_is_as_accurate_without_products(hip, shape, re):
+    """Planes of 3072 rows and more at Reynolds numbers where convection dominates: a
+    factor without Y L and Y U eliminates the planes in the order of the one with them, so
+    the nearly singular pivots that set the residual of an application are the same ones:
+    within a factor of 10 of each other."""
+    import torch
+    from transiflow_amd.solver import LineFactor
+    itf = hip.Interface({'Reynolds Number': re}, *shape)
+    g = itf.solver.gauge()
+    seed = int(re - 340) // 20
+    J = itf.jacobian(itf.vector_from_array(_flow(itf, seed)))
+    r = torch.from_numpy(seeded_state(itf.n, seed)).cuda()
+    r[g] = 0.0
+    res = {}
+    for fused in (True, False):
+        f = LineFactor(itf, J, g, single=False, factor=False)
+        f.set_fused(fused)
+        f.refactor(J, g)
+        z = f.apply(r, torch.empty_like(r))
+        res[fused] = float(torch.linalg.norm(r - J.matvec(z, gauge=g)) / torch.linalg.norm(r))
+        assert f.perturbed == 0
+    print('%s Re %g: residual %.1e with, %.1e without products' % (shape, re, res[True], res[False]), flush=True)
+    assert res[False] <= 10 * res[True]
+
+
+@pytest.mark.parametrize('shape', [(32, 24, 1), (32, 24, 2), (28, 28, 5), (56, 14, 32), (32, 24, 65), (30, 25, 4)])
+def test_inner_factor_matches_direct(hip, shape):
+    """The factor that a preconditioner may ask for: FP64 planes of 3072 rows and more are
+    eliminated one after the other from 2 to 64 planes, the same inverse at Re 100 to
+    rounding (1e-10, as for the two forms of the reduction) with the same bits for one
+    column and two, replayed and eager; one plane, 65 planes or 3000 rows give the direct
+    factor's bits.  In order no products are formed, and asking for them is refused."""
+    import torch
+    from transiflow_amd._lib import BackendError
+    from transiflow_amd.solver import LineFactor
+    itf = hip.Interface({'Reynolds Number': 100}, *shape)
+    g = itf.solver.gauge()
+    J = itf.jacobian(itf.vector_from_array(0.1 * seeded_state(itf.n, 11)))
+    r = [torch.from_numpy(seeded_state(itf.n, 12 + i)).cuda() for i in range(2)]
+    for v in r:
+        v[g] = 0.0
+    out = {}
+    for inner in (False, True):
+        f = LineFactor(itf, J, g, single=False, inner=inner)
+        got = []
+        for graph in (False, True, True):
+            f.set_graph(graph)
+            z = [torch.full_like(v, numpy.nan) for v in r]
+            p = [torch.full_like(v, numpy.nan) for v in r]
+            for a, b in zip(r, z):
+                f.apply(a, b)
+            f.apply_pair(r[0], r[1], p[0], p[1], single=False)
+            torch.cuda.synchronize()
+            got.append([v.cpu().numpy() for v in z + p])
+        for zs in got:
+            for i in range(2):
+                assert numpy.isfinite(zs[i]).all()
+                assert numpy.array_equal(zs[i], got[0][i]) and numpy.array_equal(zs[2 + i], got[0][i])
+        out[inner] = got[0][0]
+        del f
+    if shape[2] in (1, 65) or shape == (30, 25, 4):
+        assert numpy.array_equal(out[True], out[False])
+    else:
+        assert numpy.linalg.norm(out[True] - out[False]) <= 1e-10 * numpy.linalg.norm(out[False])
+        with pytest.raises(BackendError):
+            LineFactor(itf, J, g, single=False, factor=False, inner=True).set_fused(True)
+
+
+@pytest.mark.parametrize('shape,re', [((56, 56, 12), 150.0), ((56, 60, 16), 300.0)])
+def test_two_grid_coarse_order_leaves_the_solve_alone(hip, shape, re):
+    """The two-grid solve with its coarse planes (3136 and 3360 rows) one after the other,
+    and by the reduction ('Fused Apply'): the same number of iterations to the tolerance."""
+    import torch
+    count = []
+    for fused in (None, True):
+        itf = hip.Interface({'Reynolds Number': re, 'HIP Solver': {
+            'Preconditioner': 'multigrid', 'Restart': 100, 'Maximum Iterations': 600, 'Fused Apply': fused}}, *shape)
+        J = itf.jacobian(itf.vector_from_array(_flow(itf, 3)))
+        b = itf.vector_from_array(_flow(itf, 4))
+        x = itf.solve(J, b)
+        r = b.data - J.matvec(x.data)
+        r[itf.solver.gauge()] = 0.0
+        assert float(torch.linalg.norm(r) / torch.linalg.norm(b.data)) <= 1.1e-10
+        count.append(itf.solver.log[-1][0])
+    assert count[0] == count[1]

@@ -21,8 +21,9 @@
 // 256 lines, instead of (lines x panels) for the Thomas recursion.  At level
 // 0 the couplings are the sparse CSR entries (a few per row), so the level-0
 // products are sparse-dense and cost O(m^2).
-// Long FP64 lines without the fused backward are taken in order instead (chain_plan):
-// each level eliminates one line, and every level's couplings are the sparse ones.
+// Handles made for preconditioners (tf_bcr_create_inner) take long FP64 lines in order
+// instead (chain_plan): each level eliminates one line, and every level's couplings are
+// the sparse ones.
 // The factor (Y, P1, P2, L, U) is
 // kept in the storage type T (double, or float for the mixed-precision
 // variant, whose factorisation also runs in FP32).  For the FP32 apply of that
@@ -1128,16 +1129,20 @@ struct LevelPlan {
   std::vector<int> k, k1, k2, kfa, kfb, kslot;
 };
 
-// Lines of CHAIN_M rows and more are eliminated one after the other (the chain) unless
-// the factor keeps Y L and Y U: the couplings then stay sparse, and a line costs one
-// inversion and its neighbour a sparse update, where the reduction multiplies five to six
-// dense blocks per line (32 against 122 products of 2 m^3 at 32 lines).  One such matrix
-// fills the device; shorter lines need the reduction's batches.  Factorisation and apply
-// in FP64, chain against reduction: 24^3 (2304 rows) 47.6 / 44.9 ms and 747 / 602 us,
-// 28^3 (3136 rows) 93 / 119 ms and 1246 / 1229 us, 32^3 165 / 264 ms and 1908 / 2221 us.
-// Long chains can round more than the reduction (2D grids of 48 lines up to a hundred
-// times more in FP32; planes of 3D grids as much, but for states of noise at Re 1000 up to
-// ten times): FP64 only, where the solves refine that away, and up to CHAIN_N lines.
+// Lines of CHAIN_M rows and more of a tf_bcr_create_inner handle are eliminated one after
+// the other (the chain): the couplings then stay sparse, and a line costs one inversion
+// and its neighbour a sparse update, where the reduction multiplies four dense blocks per
+// line (32 against 122 products of 2 m^3 at 32 lines).  One such matrix fills the device;
+// shorter lines need the reduction's batches (24^3, 2304 rows: 47.6 against 44.9 ms and an
+// apply of 747 against 602 us).  Factorisation and apply in FP64, chain against reduction:
+// 28^3 (3136 rows) 77 / 115 ms and 1245 / 1228 us, 32^3 141 / 260 ms and 1904 / 2222 us.
+// Not for a direct solver: the chain's pivots are those of ever longer parts of the grid,
+// nearly singular ever more often as convection grows, so its apply rounds more.  Residual
+// of one apply on flow-like states of 28^2 .. 33^2 planes, chain over reduction in the
+// geometric mean (and at worst): Re <= 150 0.95 (1.2), 150-300 3 (8000), 250-500 16
+// (20000: 1.3e-8 for 6e-13).  As the coarse solve of the two-grid cycle, whose other errors
+// are of the order of one, it changes no iteration count and no digit of the result
+// (64^3 and six more grids, Re 50-600).  FP32 has no digits to spare and keeps the reduction.
 constexpr int CHAIN_M = 3072, CHAIN_N = 64;
 
 bool chain_pays(int m, int N, int single) { return !single && m >= CHAIN_M && N > 1 && N <= CHAIN_N; }
@@ -1838,7 +1843,6 @@ int solve_graph(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream
 
 template <typename V, int NC>
 int solve_any(tf_bcr* h, const V* const (&r)[NC], V* const (&x)[NC], hipStream_t st) {
-  if (h->lev.empty()) return tf::fail("tf_bcr_solve: the handle was lost to a failed allocation");
   if (h->use_graph)
     return h->single ? solve_graph<float, V, NC>(h, r, x, st) : solve_graph<double, V, NC>(h, r, x, st);
   return h->single ? solve_impl<float, V, NC>(h, r, x, st) : solve_impl<double, V, NC>(h, r, x, st);
@@ -1851,7 +1855,7 @@ namespace tf {
 // applies are to be replayed, and the number under which that stays the same apply.
 bool bcr_replays(const tf_bcr* h, unsigned long long* gen) {
   *gen = h->gen;
-  return h->use_graph != 0 && !h->lev.empty();
+  return h->use_graph != 0;
 }
 // the launches of one apply of nc (1 or 2) columns (single: FP32 vectors)
 int bcr_apply(tf_bcr* h, int single, int nc, const void* r0, const void* r1, void* x0, void* x1, hipStream_t st) {
@@ -1902,10 +1906,8 @@ extern "C" {
 // lines) instead of the rows j; n = nx ny dof.
 int tf_bcr_destroy(tf_bcr* h);
 static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines, bool chain);
-int tf_bcr_set_dense_top(tf_bcr* h, int lines);
-int tf_bcr_set_half(tf_bcr* h, int on, void* stream);
 
-int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines) {
+static int bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines, bool inner) {
   if (!out) return tf::fail("null handle");
   *out = nullptr;
   if (m < 1 || n % m != 0) return tf::fail("line block size must divide n");
@@ -1913,7 +1915,7 @@ int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int y
     return tf::fail("y-line order needs n = nx * m with m = ny * dof");
   tf_bcr* h = new tf_bcr();
   h->gen = new_gen();
-  const int rc = bcr_create_impl(h, n, m, single, nx, dof, ylines, chain_pays(m, n / m, single));
+  const int rc = bcr_create_impl(h, n, m, single, nx, dof, ylines, inner && chain_pays(m, n / m, single));
   if (rc) {
     // frees whatever was allocated before the failure (unset members are null)
     tf_bcr_destroy(h);
@@ -1923,37 +1925,12 @@ int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int y
   return 0;
 }
 
-// everything the handle owns
-static void bcr_release(tf_bcr* h) {
-  for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
-    if (g->exec) (void)hipGraphExecDestroy(g->exec);
-    if (g->graph) (void)hipGraphDestroy(g->graph);
-  }
-  if (h->cap) (void)hipStreamDestroy(h->cap);
-  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
-                  (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
-                  (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
-                  (void*)h->topsync, h->Z, h->zpool, h->xtab, h->Nx})
-    (void)hipFree(p);
-  (void)hipHostFree(h->host_flags);
-  h->side.release();
+int tf_bcr_create(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines) {
+  return bcr_create(out, n, m, single, nx, dof, ylines, false);
 }
 
-// An unfactored handle made again with the other elimination order, its settings kept.
-static int bcr_rebuild(tf_bcr* h, bool chain) {
-  const tf_bcr old = *h;
-  bcr_release(h);
-  *h = tf_bcr{};
-  h->gen = new_gen();
-  const Order& o = old.order;
-  if (int e = bcr_create_impl(h, old.n, old.m, old.single, o.nx, o.dof, o.ylines, chain)) return e;
-  h->use_graph = old.use_graph;
-  h->use_small = old.use_small;
-  h->split = old.split;
-  h->fused = old.fused;
-  if (old.zmax)
-    if (int e = tf_bcr_set_dense_top(h, old.zmax)) return e;
-  return old.half ? tf_bcr_set_half(h, 1, nullptr) : 0;
+int tf_bcr_create_inner(tf_bcr** out, int n, int m, int single, int nx, int dof, int ylines) {
+  return bcr_create(out, n, m, single, nx, dof, ylines, true);
 }
 
 static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof, int ylines, bool chain) {
@@ -2240,7 +2217,18 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
 
 int tf_bcr_destroy(tf_bcr* h) {
   if (!h) return 0;
-  bcr_release(h);
+  for (BcrGraph* g : {&h->g64[0], &h->g64[1], &h->g32[0], &h->g32[1]}) {
+    if (g->exec) (void)hipGraphExecDestroy(g->exec);
+    if (g->graph) (void)hipGraphDestroy(g->graph);
+  }
+  if (h->cap) (void)hipStreamDestroy(h->cap);
+  for (void* p : {h->D, h->Lm, h->Um, h->P1, h->P2, h->Pinv, h->Kc, h->Tb, (void*)h->Lr, (void*)h->Ur,
+                  (void*)h->Ut, (void*)h->Lt, (void*)h->nLr, (void*)h->nUr, (void*)h->nUt, (void*)h->nLt,
+                  (void*)h->flags, h->rw, h->tb, h->yb, h->xw, h->pool, h->H, h->S, h->hpool, h->W,
+                  (void*)h->topsync, h->Z, h->zpool, h->xtab, h->Nx})
+    (void)hipFree(p);
+  (void)hipHostFree(h->host_flags);
+  h->side.release();
   delete h;
   return 0;
 }
@@ -2248,7 +2236,6 @@ int tf_bcr_destroy(tf_bcr* h) {
 // Factor the gauged matrix (CSR, gauge row or -1).  Asynchronous on ``stream``.
 int tf_bcr_factor(tf_bcr* h, const int* rp, const int* ci, const double* v, int gauge, void* stream) {
   if (!h) return tf::fail("null handle");
-  if (h->lev.empty()) return tf::fail("tf_bcr_factor: the handle was lost to a failed allocation");
   hipStream_t st = (hipStream_t)stream;
   return h->single ? factor_impl<float>(h, rp, ci, v, gauge, st) : factor_impl<double>(h, rp, ci, v, gauge, st);
 }
@@ -2328,7 +2315,7 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
   if (on && !h->H) {
     // all three allocations succeed before any is kept (a failed call leaves no copies)
     void *H_ = nullptr, *S_ = nullptr;
-    const size_t copies = h->chain ? N : 3 * N + 2 * slots;  // (a chain reads D only)
+    const size_t copies = 3 * N + 2 * slots;
     hipError_t e = hipMalloc(&H_, sizeof(f16) * mm * copies);
     if (e == hipSuccess) e = hipMalloc(&S_, sizeof(float) * (size_t)m * copies);
     if (e != hipSuccess) {
@@ -2372,8 +2359,8 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
         uh.push_back(hb(2, e));
         us.push_back(sb(2, e));
         conv(0, e);
-        if (l > 0 && !h->chain && L.ea[b] >= 0) conv(1, e);
-        if (l > 0 && !h->chain && L.eb[b] >= 0) conv(2, e);
+        if (l > 0 && L.ea[b] >= 0) conv(1, e);
+        if (l > 0 && L.eb[b] >= 0) conv(2, e);
       }
       for (size_t b = 0; b < L.k.size(); ++b) {
         const int sl = L.kslot[b];
@@ -2382,8 +2369,8 @@ int tf_bcr_set_half(tf_bcr* h, int on, void* stream) {
         p2h.push_back(hb(4, sl));
         p2s.push_back(sb(4, sl));
         // (level 0 applies its multipliers through Y and the sparse couplings)
-        if (l > 0 && !h->chain && L.k1[b] >= 0) conv(3, sl);
-        if (l > 0 && !h->chain && L.k2[b] >= 0) conv(4, sl);
+        if (l > 0 && L.k1[b] >= 0) conv(3, sl);
+        if (l > 0 && L.k2[b] >= 0) conv(4, sl);
       }
       HOff o;
       o.Yh = pb.add_ptrs(yh);
@@ -2461,13 +2448,8 @@ int tf_bcr_set_fused(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
   if (h->factored && (on != 0) != (h->fused != 0))
     return tf::fail("tf_bcr_set_fused: the handle already holds a factor of the other form");
-  if ((on != 0) != (h->fused != 0)) {
-    drop_graphs(h);
-    h->fused = on ? 1 : 0;
-    const bool chain = !on && chain_pays(h->m, h->N, h->single);
-    if (chain != (h->chain != 0))
-      if (int e = bcr_rebuild(h, chain)) return e;
-  }
+  if (on && h->chain) return tf::fail("tf_bcr_set_fused: the handle eliminates its lines in order and forms no products");
+  if ((on != 0) != (h->fused != 0)) drop_graphs(h);
   h->fused = on ? 1 : 0;
   return 0;
 }

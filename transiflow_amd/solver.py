@@ -159,8 +159,9 @@ _SPLITS = {'fp32': 0, 'bf16x3': 3, 'bf16': 1}
 # two more products per line grow with the cube of the rows and save one launch per level
 # and apply: FP32 factor and two-column FP16 apply with and without, 24^3 (2304 rows) 29.8
 # / 25.7 ms and 252 / 270 us (even after 230 applies), 28^3 (3136) 77.7 / 65.0 ms and 465 /
-# 479 us (900), 32^3 (4096) 173.9 / 145.3 ms and 714 / 731 us (1700).  In FP64 the lines
-# are then eliminated one after the other: 32^3 315.5 / 141.6 ms and 2345 / 2194 us.
+# 479 us (900), 32^3 (4096) 173.9 / 145.3 ms and 714 / 731 us (1700); in FP64 28^3 140 / 115
+# ms and 1406 / 1418 us (2100), 32^3 315 / 260 ms and 2345 / 2365 us (2800).  A caller whose
+# factors serve more applies than that asks for 'Fused Apply'.
 FUSED_ROWS = 3072
 
 
@@ -232,9 +233,11 @@ class LineFactor:
     Thomas recursion (``'thomas'``, csrc/linelu.hip)."""
     _ABI = {'line': 'tf_bcr', 'thomas': 'tf_linelu'}
 
-    def __init__(self, itf, jac, gauge, single=False, kind='line', factor=True, layout=None):
+    def __init__(self, itf, jac, gauge, single=False, kind='line', factor=True, layout=None, inner=False):
         """``layout`` (n, m, nx, dof, ylines) overrides the problem's own (the
-        interleaved real form of a complex matrix has twice the rows per line)."""
+        interleaved real form of a complex matrix has twice the rows per line).
+        ``inner``: for one step inside a preconditioner, which may round more (long
+        FP64 lines one after the other; not with ``set_fused``)."""
         self.name = kind
         self._p = self._ABI[kind]
         h = ctypes.c_void_p()
@@ -243,7 +246,8 @@ class LineFactor:
             n, nx, dof = itf.n, itf.nx, itf.dof
             if layout is not None:
                 n, m, nx, dof, ylines = layout
-            _lib.call('tf_bcr_create', ctypes.byref(h), n, m, 1 if single else 0, nx, dof, ylines)
+            _lib.call('tf_bcr_create_inner' if inner else 'tf_bcr_create', ctypes.byref(h), n, m, 1 if single else 0,
+                      nx, dof, ylines)
         else:
             m = line_block_size(itf)
             _lib.call(self._p + '_create', ctypes.byref(h), itf.n, m, 1 if single else 0)
@@ -463,8 +467,9 @@ class Multigrid:
         Jc = c.jacobian(DeviceVector(self.xc))
         gc = c.pressure_row if (c.dof > c.dim and c.pressure_row is not None) else -1
         if self.cf is None:
-            self.cf = LineFactor(c, Jc, gc, single=self.single, kind='line', factor=False)
             opts = _opts(itf.parameters)
+            self.cf = LineFactor(c, Jc, gc, single=self.single, kind='line', factor=False,
+                                 inner=not _fused_apply(opts, self.single, line_block_size(c)))
             _configure_line(self.cf, opts, self.single)
             self.cf.set_graph(opts['Apply Graph'])
             if self.single:
