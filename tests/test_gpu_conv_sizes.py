@@ -64,3 +64,28 @@ def test_conv_layer_at_tile_edges(hip, dim, shape, cin, cout):
     close(dW[:K, :cout], P.T @ G, numpy.abs(P).T @ numpy.abs(G), n)
     close(db, G.sum(axis=0), numpy.abs(G).sum(axis=0), n)
     assert not dW.cpu().numpy()[K:].any() and not dW.cpu().numpy()[:, cout:].any()
+
+
+@pytest.mark.parametrize('dim,shape,cin,cout', [(2, (7, 5, 1), 3, 32), (3, (9, 7, 5), 4, 32), (3, (9, 7, 5), 32, 4)])
+def test_weight_gradient_without_the_bias_gradient(hip, dim, shape, cin, cout):
+    """db may be null, and g32 with it: the same dW bit for bit at each load width."""
+    import torch
+    from transiflow_amd import _lib
+    from transiflow_amd.vector import ptr, stream
+    nx, ny, nz = shape
+    n = nx * ny * nz
+    rng = numpy.random.default_rng(n + cin)
+    kpad, npad = _pad16(oc.taps(dim) * cin), _pad16(cout)
+    x, g = (oc.bf16(rng.standard_normal((n, c)).astype(numpy.float32)) for c in (cin, cout))
+    d = {k: torch.from_numpy(v).cuda() for k, v in dict(x=_bits(x), g16=_bits(g), g=g).items()}
+    out = []
+    for with_bias in (True, False):
+        work = torch.full((_lib.load().tf_conv_wgrad_work_size(n, kpad, npad),), float('nan'), dtype=torch.float32,
+                          device='cuda')
+        dW = torch.full((kpad, npad), float('nan'), dtype=torch.float32, device='cuda')
+        db = torch.full((cout,), float('nan'), dtype=torch.float32, device='cuda')
+        _lib.call('tf_conv_wgrad', nx, ny, nz, dim, cin, cout, kpad, npad, ptr(d['x']), ptr(d['g16']),
+                  ptr(d['g']) if with_bias else None, ptr(work), ptr(dW), ptr(db) if with_bias else None, stream())
+        out.append(dW.cpu().numpy())
+        assert torch.isfinite(db).all().item() == with_bias
+    assert numpy.isfinite(out[0]).all() and numpy.array_equal(out[0], out[1])

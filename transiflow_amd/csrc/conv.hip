@@ -280,7 +280,8 @@ inline int conv_tiles(long ncell) { return ncell <= 512L * 128 ? 1 : 4; }
 
 // Partial weight and bias gradients, one block per chunk of cells:
 //   partial[block][k][co] = sum over the block's cells of patch[cell][k] g[cell][co],
-//   then 32 entries       sum over the block's cells of g32[cell][co] (the FP32 gradient)
+//   then 32 entries       sum over the block's cells of g32[cell][co] (the FP32 gradient;
+//                         left unwritten when g32 is null)
 // as MFMAs with M = k, N = co and the cells as the reduction dimension.  The
 // block walks its cells WG_SUB at a time: the patch (all K values of WG_SUB
 // cells, zero outside the grid) and the gradient are staged transposed in LDS
@@ -416,6 +417,7 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_conv_wgrad(Grid3 g, long ncel
           for (int v = 0; v < 4; ++v) P[(long)(kt * 16 + 4 * q + v) * npad + n * 16 + r] = acc[t][n][v];
     }
   }
+  if (!g32) return;
   // bias: thread t sums channel t % cout of every (NT / cout)-th cell, then a tree per channel
   float* red = (float*)lds;
   const int rows = NT / cout, co = threadIdx.x % cout, first = threadIdx.x / cout;
@@ -432,15 +434,15 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_conv_wgrad(Grid3 g, long ncel
   }
 }
 
-// dW[e] (e < len), db[e - len] = sum_b partial[b][e]  (fixed order: deterministic).  64
-// entries per block, a quarter of the blocks' partials per wave.
+// dW[e] (e < len), db[e - len] (or null) = sum_b partial[b][e]  (fixed order:
+// deterministic).  64 entries per block, a quarter of the blocks' partials per wave.
 __global__ __launch_bounds__(256) void k_sum_partials(int nb, long len, int cout, const float* __restrict__ partial,
                                                       float* __restrict__ dW, float* __restrict__ db) {
   __shared__ float sh[256];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const long e = blockIdx.x * 64L + lane, pitch = len + 32;
   float s = 0.f;
-  if (e < pitch) {
+  if (e < (db ? pitch : len)) {
     const float* p = partial + e;
 #pragma unroll 8
     for (int b = wave; b < nb; b += 4) s += p[b * pitch];
@@ -585,7 +587,8 @@ int tf_conv_wgrad_work_size(long ncell, int kpad, int npad) {
   return n > 2147483647L ? -1 : (int)n;
 }
 
-// dW [kpad][npad] FP32 = sum over cells of patch(in)^T gout; db[cout] = sum of g32.
+// dW [kpad][npad] FP32 = sum over cells of patch(in)^T gout; db[cout] = sum of g32 (db
+// may be null: g32 is then not read).
 // in: BF16 [ncell][cin]; gout16 / g32: BF16 / FP32 [ncell][cout]; work: FP32 of
 // tf_conv_wgrad_work_size() elements.
 int tf_conv_wgrad(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, int npad, const void* in,
@@ -606,7 +609,7 @@ int tf_conv_wgrad(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, 
     constexpr int VEC = decltype(vec)::value;
     TF_HIP(hipFuncSetAttribute((const void*)k_conv_wgrad<VEC>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k_conv_wgrad<VEC>, wg_grid, wg_block, lds, st, g, ncell, chunk, cin, cout, kpad, npad, in16,
-                       g16, g32, work);
+                       g16, db ? g32 : nullptr, work);
     return 0;
   };
   int rc;
