@@ -251,3 +251,13 @@ def test_auto_preconditioner_choice():
     for g in (_grid(63, 63, 63), _grid(64, 64, 64, periodic=True), _grid(4096, 4096, 1)):
         with pytest.raises(SolverError, match='no preconditioner for this grid.*GB'):
             auto_preconditioner(g, False)
+
+
+def test_weight_gradient_of_an_empty_grid_is_refused():
+    """No cells: no work space, and an error instead of a launch or a division by zero."""
+    from transiflow_amd import _lib
+    lib = _lib.load()
+    assert [lib.tf_conv_wgrad_work_size(n, 16, 16) for n in (0, -1, 1, 32, 33)] == [0, 0, 288, 288, 576]
+    for grid in ((0, 4, 1), (4, 0, 1), (-3, 4, 1)):
+        with pytest.raises(_lib.BackendError):
+            _lib.call('tf_conv_wgrad', *grid, 2, 1, 1, 16, 16, None, None, None, None, None, None, None)

@@ -300,10 +300,11 @@ constexpr int WG_WAVES = 8;
 constexpr int WG_MAXT = 7;    // k-tiles per wave: 56 / 8
 constexpr int WG_KMAX = 896;  // staged K rows
 
-// cells per block (a multiple of WG_SUB) for about 256 blocks, at most 1024
+// cells per block (a multiple of WG_SUB) for about 256 blocks, at most 1024 (an empty
+// grid, too, gets a block size to divide by)
 inline long wgrad_chunk(long ncell) {
   const long c = ((ncell + 255) / 256 + WG_SUB - 1) / WG_SUB * WG_SUB;
-  return c < 1024 ? c : 1024;
+  return c < WG_SUB ? WG_SUB : (c < 1024 ? c : 1024);
 }
 inline long wgrad_blocks(long ncell) { return (ncell + wgrad_chunk(ncell) - 1) / wgrad_chunk(ncell); }
 inline size_t wgrad_lds(int kpad, int npad) { return sizeof(uint16_t) * (size_t)(kpad + npad) * WG_PITCH; }
@@ -596,6 +597,7 @@ int tf_conv_wgrad(int nx, int ny, int nz, int dim, int cin, int cout, int kpad, 
   if (int e = check_layer(dim, cin, cout, kpad, npad)) return e;
   const long ncell = (long)nx * ny * nz;
   if (kpad > WG_KMAX || ncell >= (1L << 31)) return tf::fail("conv wgrad: K or the grid too large");
+  if (nx < 1 || ny < 1 || nz < 1) return tf::fail("conv wgrad: empty grid");
   const long blocks = wgrad_blocks(ncell);
   const int chunk = (int)wgrad_chunk(ncell);
   hipStream_t st = (hipStream_t)stream;
