@@ -232,3 +232,47 @@ def test_two_grid_coarse_order_leaves_the_solve_alone(hip, shape, re):
         assert float(torch.linalg.norm(r) / torch.linalg.norm(b.data)) <= 1.1e-10
         count.append(itf.solver.log[-1][0])
     assert count[0] == count[1]
+
+
+@pytest.mark.parametrize('m', [20, 100, 300])
+@pytest.mark.parametrize('single,scale', [(False, 1.0), (False, 2.0 ** 150), (True, 1.0), (True, 2.0 ** 124),
+                                          (False, numpy.inf), (True, numpy.inf)])
+def test_zero_pivot_at_large_scales(hip, m, single, scale):
+    """A line with an empty row and column, its other entries near the end of the exponent
+    range: the one zero pivot is found, counted and replaced (by 1e-3 of the largest entry)
+    as at scale one, and the rest is inverted.  Rows sum to less than half their diagonal:
+    the inverse's error is below 10 m units of rounding.  An infinite entry makes every
+    finite pivot of its block a small one, which is counted too."""
+    import types
+
+    import torch
+    from scipy import sparse
+    from transiflow_amd.solver import LineILU
+    from transiflow_amd.vector import DeviceCsrMatrix
+    rng = numpy.random.default_rng(m)
+    A = numpy.diag(numpy.ones(m))
+    for off in (1, 2, 3):
+        A += 0.07 * numpy.diag(rng.uniform(-1, 1, m - off), off) + 0.07 * numpy.diag(rng.uniform(-1, 1, m - off), -off)
+    p = m // 2 + 3
+    A[p, :] = A[:, p] = 0.0
+    S = sparse.csr_matrix(A)
+    if numpy.isinf(scale):
+        S.data[3] = numpy.inf
+    else:
+        S.data *= scale
+    t = lambda v, dt: torch.from_numpy(numpy.ascontiguousarray(v)).to(dt).cuda()
+    M = DeviceCsrMatrix(t(S.indptr, torch.int32), t(S.indices, torch.int32), t(S.data, torch.float64), m)
+    P = LineILU(types.SimpleNamespace(nx=m, ny=1, nz=1, dof=1), single)
+    P.refactor(M, -1)
+    if numpy.isinf(scale):
+        assert P.perturbed > 1
+        return
+    r = rng.uniform(-1, 1, m)
+    dt = torch.float32 if single else torch.float64
+    out = torch.empty(m, dtype=dt, device='cuda')
+    (P.apply32 if single else P.apply)(t(r * scale, dt), out)
+    got, keep = out.double().cpu().numpy(), numpy.arange(m) != p
+    ref = numpy.linalg.solve(A[numpy.ix_(keep, keep)], r[keep])
+    assert P.perturbed == 1
+    assert numpy.max(numpy.abs(got[keep] - ref)) <= 10 * m * numpy.finfo(numpy.float32 if single else float).eps
+    assert abs(got[p] / r[p]) >= 500

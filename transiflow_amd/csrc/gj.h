@@ -114,10 +114,11 @@ __device__ __forceinline__ void invert64(T (&cur)[NS], T (&nxt)[NS], int& mystep
   for (int w = 0; w < 8; ++w) amax = fmax(amax, sh.wmax[w]);
   if (amax == (T)0) amax = 1;
   const T tol = (sizeof(T) == 8 ? (T)1e-13 : (T)1e-6) * amax;
-  // pivots of a smaller exponent go the careful way (below tol, or too small or large
-  // for the quick reciprocal)
+  // pivots of a smaller or larger exponent go the careful way (below tol, or too small or
+  // large for the quick reciprocal; with tol itself that large only those just above it go
+  // the quick one, and none do beside an infinite entry)
   const int elo = __builtin_amdgcn_readfirstlane(exponent_of(fmax(tol, (T)1e-30)) + 1);
-  const int ehi = exponent_of((T)1e30);
+  const int ehi = max(exponent_of((T)1e30), elo);
   mystep = 64;
   // pivot key: magnitude bits, then the lane (ties go to the lower one); used rows 0
   unsigned alive = 0x7fffffc0u, tag = 63u - (unsigned)lane;
