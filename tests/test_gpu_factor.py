@@ -276,3 +276,40 @@ def test_zero_pivot_at_large_scales(hip, m, single, scale):
     assert P.perturbed == 1
     assert numpy.max(numpy.abs(got[keep] - ref)) <= 10 * m * numpy.finfo(numpy.float32 if single else float).eps
     assert abs(got[p] / r[p]) >= 500
+
+
+@pytest.mark.parametrize('single', [False, True])
+@pytest.mark.parametrize('shape', [(21, 23), (22, 24), (43, 45), (64, 66), (86, 88), (20, 20, 4), (40, 33, 3), (48, 44, 2)])
+def test_line_factor_backward_error(hip, shape, single):
+    """The residual of an application against the size of what it is made of,
+    |b - A z| / (|A| |z| + |b|) in the maximum norm, which no condition number enters: the
+    rounding of sums over a block's rows grows like a random walk, so at most 10 units of
+    it times the square root of the rows.  The sizes take every way of forming the
+    level-0 products (eight, four or two rows of a block in LDS, or the multipliers in
+    memory: 1600, 5280 and 8448 rows, FP64 and FP32), with and without Y L and Y U and,
+    FP64, in order."""
+    import torch
+    from scipy import sparse
+    from transiflow_amd.solver import LineFactor
+    itf = hip.Interface({'Reynolds Number': 100}, *shape)
+    g = itf.solver.gauge()
+    J = itf.jacobian(itf.vector_from_array(0.1 * seeded_state(itf.n, 21)))
+    A = sparse.csr_matrix(tuple(v.cpu().numpy() for v in (J.val, J.col, J.row_ptr)), shape=(itf.n, itf.n))
+    norm = abs(A).sum(axis=1).max()
+    r = torch.from_numpy(seeded_state(itf.n, 22)).cuda()
+    r[g] = 0.0
+    for kind in ('fused', 'plain') + (() if single else ('inner',)):
+        f = LineFactor(itf, J, g, single=single, factor=False, inner=kind == 'inner')
+        f.set_fused(kind == 'fused')
+        f.refactor(J, g)
+        if single:
+            z = f.apply32(r.float(), torch.empty_like(r, dtype=torch.float32)).double()
+            b = r.float().double()
+        else:
+            z, b = f.apply(r, torch.empty_like(r)), r
+        res = float((b - J.matvec(z, gauge=g)).abs().max())
+        err = res / (norm * float(z.abs().max()) + float(b.abs().max()))
+        bound = 10 * numpy.sqrt(f.m) * numpy.finfo(numpy.float32 if single else numpy.float64).eps
+        print('%s m %d single %s %s: %.1e, bound %.1e' % (shape, f.m, single, kind, err, bound), flush=True)
+        assert f.perturbed == 0 and err <= bound
+        del f

@@ -142,3 +142,30 @@ def test_replayed_iterations_match_eager(hip, shape, restart):
     assert max(got[True][1]) > 3
     for a, b in zip(got[True][0], got[False][0]):
         assert numpy.isfinite(a).all() and numpy.array_equal(a, b)
+
+
+@pytest.mark.parametrize('precision,amplitude', [('fp64', 1.0), ('mixed', 0.5)])
+def test_replayed_iterations_with_copied_columns_match_eager(hip, precision, amplitude):
+    """The same in cycles of 150 steps: from step 96 on the block sums of a small grid no
+    longer fit the reductions that write the Hessenberg column to the host, and the columns
+    come by a copy and an event inside the replayed iterations instead."""
+    got = {}
+    for graphs in (False, True):
+        itf = hip.Interface({'Reynolds Number': 300,
+                             'HIP Solver': {'Preconditioner': 'line', 'Precision': precision, 'Reuse Factor': True,
+                                            'Reuse Limit': 100000, 'Restart': 150, 'Inner Iterations': 1000,
+                                            'Inner Tolerance': 1e-6, 'Maximum Iterations': 3000,
+                                            'Apply Graph': graphs, 'Step Graphs': graphs}}, 14, 9)
+        rng = numpy.random.default_rng(5)
+        vec = lambda s: itf.vector_from_array(rng.uniform(-1, 1, itf.n) * s)
+        itf.solve(itf.jacobian(vec(0.0)), vec(1.0))
+        out = []
+        for i in range(5):
+            J = itf.jacobian(vec(amplitude))
+            out += [itf.array_from_vector(v) for v in itf.solve_pair(J, vec(1.0), vec(1e-3))]
+            out.append(itf.array_from_vector(itf.solve(J, vec(1.0))))
+        got[graphs] = (out, [e[0] for e in itf.solver.log])
+    assert got[True][1] == got[False][1]
+    assert sum(its > 96 for its in got[True][1]) >= 10   # the pairs, at least
+    for a, b in zip(got[True][0], got[False][0]):
+        assert numpy.isfinite(a).all() and numpy.array_equal(a, b)
