@@ -1993,7 +1993,8 @@ static int bcr_create_impl(tf_bcr* h, int n, int m, int single, int nx, int dof,
   auto blk = [&](char* base, int j) -> void* { return base ? (void*)(base + bm * (size_t)j) : nullptr; };
   PoolBuilder pb;
   struct Off {
-    size_t e, ea, eb, Ye, Le, Ue, k, k1, k2, P1, P2, pA, pB, pC, dA1, dB1, dA2, dB2, dC, d1A, d2A, fA, fB, fC, zY1, zY2, zL, zU, zfa, zfb, hase1, hase2, faline, fbline, ylA, ylB, ylC, yuA, yuB, yuC;
+    size_t e, ea, eb, Ye, Le, Ue, k, k1, k2, P1, P2, pA, pB, pC, dA1, dB1, dA2, dB2, dC, d1A, d2A, fA, fB, fC;
+    size_t zY1, zY2, zL, zU, zfa, zfb, hase1, hase2, faline, fbline, ylA, ylB, ylC, yuA, yuB, yuC;
     int ne, nk, np1, np2, nfa, nfb, nyl, nyu;
   };
   std::vector<Off> offs;
@@ -2448,7 +2449,8 @@ int tf_bcr_set_fused(tf_bcr* h, int on) {
   if (!h) return tf::fail("null handle");
   if (h->factored && (on != 0) != (h->fused != 0))
     return tf::fail("tf_bcr_set_fused: the handle already holds a factor of the other form");
-  if (on && h->chain) return tf::fail("tf_bcr_set_fused: the handle eliminates its lines in order and forms no products");
+  if (on && h->chain)
+    return tf::fail("tf_bcr_set_fused: the handle eliminates its lines in order and forms no products");
   if ((on != 0) != (h->fused != 0)) drop_graphs(h);
   h->fused = on ? 1 : 0;
   return 0;

@@ -269,7 +269,8 @@ struct BlockLds {
 
 template <typename T>
 __global__ __launch_bounds__(512) void k_gj_block(int m, int k0, int pb, T* const* __restrict__ Xp,
-                                                  const T* __restrict__ Nb, T* __restrict__ Pb, int* __restrict__ nperturb, double repl) {
+                                                  const T* __restrict__ Nb, T* __restrict__ Pb,
+                                                  int* __restrict__ nperturb, double repl) {
   extern __shared__ __align__(16) char lds[];
   BlockLds<T>& sh = *(BlockLds<T>*)lds;
   constexpr int LD = BlockLds<T>::LD;

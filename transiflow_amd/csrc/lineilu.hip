@@ -34,8 +34,6 @@ constexpr int KL = 16;  // off-line couplings kept per row and per column
 constexpr int NDIR = 6;
 __constant__ int c_dj[NDIR] = {-1, 1, 0, 0, -1, 1};
 __constant__ int c_dk[NDIR] = {0, 0, -1, 1, 1, -1};
-const int h_dj[NDIR] = {-1, 1, 0, 0, -1, 1};
-const int h_dk[NDIR] = {0, 0, -1, 1, 1, -1};
 
 struct Cp {
   int line;  // line of the other end
